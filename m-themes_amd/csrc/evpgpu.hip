@@ -116,8 +116,9 @@ template <typename T> int dalloc(T **p, size_t n)
     return EVPGPU_OK;
 }
 
-// smallest eigenvalue of a symmetric 6x6 matrix (cyclic Jacobi rotations)
-double sym6_min_eig(double a[6][6])
+// smallest (and, with max, largest) eigenvalue of a symmetric 6x6 matrix
+// (cyclic Jacobi rotations)
+double sym6_min_eig(double a[6][6], double *max = nullptr)
 {
     for (int sweep = 0; sweep < 50; sweep++) {
         double off = 0.0, diag = 0.0;
@@ -144,9 +145,24 @@ double sym6_min_eig(double a[6][6])
                 }
             }
     }
-    double m = a[0][0];
-    for (int i = 1; i < 6; i++) m = a[i][i] < m ? a[i][i] : m;
+    double m = a[0][0], M = a[0][0];
+    for (int i = 1; i < 6; i++) {
+        m = a[i][i] < m ? a[i][i] : m;
+        M = a[i][i] > M ? a[i][i] : M;
+    }
+    if (max) *max = M;
     return m;
+}
+
+// the squares of C0's extreme eigenvalues, with a margin for their rounding
+void update_c0_bounds(evpgpu_ctx *c)
+{
+    double a[6][6], hi;
+    for (int i = 0; i < 6; i++)
+        for (int j = i; j < 6; j++) a[i][j] = a[j][i] = c->ld.c066[i * 6 + j];
+    const double lo = sym6_min_eig(a, &hi);
+    c->c0_lo2 = lo > 0.0 ? 0.9999 * lo * lo : 0.0;
+    c->c0_hi2 = lo > 0.0 ? 1.0001 * hi * hi : 0.0;
 }
 
 // min over orientations of lambda_min(S0 + S), both from their upper
@@ -199,7 +215,20 @@ NewtonParams newton_params(const evpgpu_ctx *c)
         P.int_n[p] = integral ? (int)ph.nrs[0] : 0;
         memcpy(P.bn[p], ph.bn, sizeof(P.bn[p]));
         memcpy(P.bb[p], ph.bb, sizeof(P.bb[p]));
+        // the Schmid tensors sym(n x b) in crystal axes (update_schmid,
+        // src/kinematics.c:430-463, rotates them by the voxel's orientation)
+        for (int s = 0; s < ph.nsys; s++) {
+            const double *n = ph.bn[s], *b = ph.bb[s];
+            const double t0 = n[0] * b[0], t1 = n[1] * b[1], t2 = n[2] * b[2];
+            P.mx[p][s][0] = (t1 - t0) * RSQ2;
+            P.mx[p][s][1] = (2. * t2 - t0 - t1) * RSQ6;
+            P.mx[p][s][2] = (n[1] * b[2] + n[2] * b[1]) * RSQ2;
+            P.mx[p][s][3] = (n[0] * b[2] + n[2] * b[0]) * RSQ2;
+            P.mx[p][s][4] = (n[0] * b[1] + n[1] * b[0]) * RSQ2;
+        }
     }
+    P.c0_lo2 = c->c0_lo2;
+    P.c0_hi2 = c->c0_hi2;
     P.crss_sym = c->crss_sym;
     P.nr_tol = c->nr_tol;
     P.tolx = c->tolx;
@@ -288,8 +317,8 @@ int green_iteration_queue(evpgpu_ctx *c, int prec, int refresh, const CtlConst &
     hipEvent_t e0, e1;
     tkernel(c, 0, &e0, &e1);
     st = newton_launch(c, P, c->sig, c->sig_alt, c->E, c->epsp, c->edot, c->tran, c->dd_on ? c->dd_k : c->crss,
-                       c->gamdot, c->phase, c->orient, c->sgr, c->N, c->partials, &nblk, c->d_status, nullptr,
-                       nullptr, c->newton_shortcut, e0, e1);
+                       c->gamdot, c->phase, c->orient, c->sgr, c->N, c->partials, &nblk, c->d_status,
+                       c->newton_shortcut, e0, e1);
     if (st) return st;
     {
         double *t = c->sig;
@@ -466,7 +495,7 @@ int evpgpu_create(evpgpu_ctx **out, int nx, int ny, int nz, int precision)
     c->tolx = 1.E-7;
     c->newton_shortcut = 1;
     c->fused = 1;
-    if (!st) st = dalloc(&c->partials, nblk * NRED);
+    if (!st) st = dalloc(&c->partials, 2 * nblk * NRED);
     if (!st) st = dalloc(&c->red, NRED + 1);
     if (!st) st = dalloc(&c->red2, (long long)REDUCE_G * NRED);
     if (!st) st = dalloc(&c->d_status, 1);
@@ -637,6 +666,7 @@ int evpgpu_set_loading(evpgpu_ctx *c, const evpgpu_loading *ld)
     c->creep_flag /= 6;
     c->have_loading = 1;
     update_lam_min(c);
+    update_c0_bounds(c);
     return EVPGPU_OK;
 }
 
@@ -887,7 +917,7 @@ int increment_core(evpgpu_ctx *c, int forced, int rep_mix, int rep64, evpgpu_sta
         tkernel(c, 0, &e0, &e1);
         st = newton_launch(c, P, c->sig_alt, c->sig, c->E, c->epsp, c->edot, c->tran,
                            c->dd_on ? c->dd_k : c->crss, c->gamdot, c->phase, c->orient, c->sgr, c->N,
-                           c->partials, &nblk, c->d_status, nullptr, nullptr, 0, e0, e1);
+                           c->partials, &nblk, c->d_status, 0, e0, e1);
         if (st) return st;
         EVP_CHECK(hipMemcpyAsync(c->h_status, c->d_status, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         EVP_CHECK(hipStreamSynchronize(c->stream));
@@ -1078,7 +1108,7 @@ int evpgpu_newton_host(evpgpu_ctx *c, int n, const int *phase, const int *orient
         if (orient[v] < 0 || orient[v] >= n_orient || phase[v] < 1 || phase[v] > c->nphases) return EVPGPU_ERR_ARG;
     int *dph = nullptr, *dor = nullptr, *dni = nullptr, *dst = nullptr;
     double *dsg = nullptr, *dsig = nullptr, *dstr = nullptr, *deps = nullptr, *dsc = nullptr,
-           *dcr = nullptr, *ded = nullptr, *dgd = nullptr, *der = nullptr, *dpart = nullptr;
+           *dcr = nullptr, *ded = nullptr, *dgd = nullptr, *der = nullptr;
     int st = EVPGPU_OK;
     if (!st) st = dalloc(&dph, n);
     if (!st) st = dalloc(&dor, n);
@@ -1093,7 +1123,6 @@ int evpgpu_newton_host(evpgpu_ctx *c, int n, const int *phase, const int *orient
     if (!st) st = dalloc(&ded, 6LL * n);
     if (!st) st = dalloc(&dgd, 12LL * n);
     if (!st) st = dalloc(&der, 2LL * n);
-    if (!st) st = dalloc(&dpart, (long long)((n + 63) / 64) * NRED);
 #define UP(d, s, cnt, T) \
     if (!st && hipMemcpy(d, s, sizeof(T) * (cnt), hipMemcpyHostToDevice) != hipSuccess) st = EVPGPU_ERR_HIP
     UP(dph, phase, n, int);
@@ -1109,11 +1138,8 @@ int evpgpu_newton_host(evpgpu_ctx *c, int n, const int *phase, const int *orient
     if (!st && hipMemset(dst, 0, sizeof(int)) != hipSuccess) st = EVPGPU_ERR_HIP;
     if (!st) {
         NewtonParams P = newton_params(c);
-        P.crss_sym = 0;
         P.dd = 0; // the power-law update on the caller's CRSS
-        int nb = 0;
-        st = newton_launch(c, P, dsig, dsig, dstr, deps, ded, dsc, dcr, dgd, dph, dor, dsg, n, dpart, &nb, dst,
-                           der, dni, 0);
+        st = newton_batch_launch(c, P, dsig, dsig, dstr, deps, ded, dsc, dcr, dgd, dph, dor, dsg, n, dst, der, dni);
         if (!st && hipStreamSynchronize(c->stream) != hipSuccess) st = EVPGPU_ERR_HIP;
     }
     int kst = 0;
@@ -1126,7 +1152,7 @@ int evpgpu_newton_host(evpgpu_ctx *c, int n, const int *phase, const int *orient
     DN(err2, der, 2LL * n, double);
     DN(niter, dni, n, int);
 #undef DN
-    void *ptrs[] = {dph, dor, dni, dst, dsg, dsig, dstr, deps, dsc, dcr, ded, dgd, der, dpart};
+    void *ptrs[] = {dph, dor, dni, dst, dsg, dsig, dstr, deps, dsc, dcr, ded, dgd, der};
     for (size_t i = 0; i < sizeof(ptrs) / sizeof(ptrs[0]); i++)
         if (ptrs[i]) (void)hipFree(ptrs[i]);
     if (!st && kst) st = kst;

@@ -35,9 +35,11 @@ struct NewtonParams {
     int int_n[2];    // integer rate exponent of the phase, 0 if not integral
     int crss_sym;    // 1: forward and backward CRSS are equal in every voxel
     double bn[2][EVPGPU_NSYSMX][3], bb[2][EVPGPU_NSYSMX][3]; // crystal-axis normals, directions
+    double mx[2][EVPGPU_NSYSMX][5]; // Schmid tensors, crystal axes (deviatoric 5-vectors)
     double s0p[21];  // S0 = C0^-1 (B-basis), packed upper triangle: the Newton step is
                      // solved in S0-scaled form
     double kmin_tolx2; // (0.99 TOLX min over orientations of lambda_min(S0 + S))^2
+    double c0_lo2, c0_hi2; // squares of C0's extreme eigenvalues (0: unknown)
     double nr_tol;   // Newton tolerance on the relative step (reference 1e-10)
     double tolx;     // line-search TOLX (reference 1e-7)
     int dd;          // dislocation-density law: the crss argument holds the
@@ -123,6 +125,7 @@ struct evpgpu_ctx {
     double *sgr;      // n_orient x 36: LU_inv_66(C_gr)
     double *h_sgr;    // host copy
     double lam_min;   // min over orientations of lambda_min(S0 + S), < 0 when stale
+    double c0_lo2, c0_hi2; // squares of C0's extreme eigenvalues, with a margin (0: not known)
     int n_orient;
 
     // spectral buffers
@@ -143,7 +146,7 @@ struct evpgpu_ctx {
     float2 *tw32[3];
 
     // reductions
-    double *partials; // max(nblk) * NRED
+    double *partials; // 2 * max(nblk) * NRED (a set per crystal phase)
     double *red;      // NRED (device)
     double *red2;     // REDUCE_G * NRED, first stage of the reduction
     double *h_red;    // NRED pinned host
@@ -248,12 +251,23 @@ int fused_anchor(evpgpu_ctx *c, const float *sigA, float *cA, double scale);
 int green_delta(evpgpu_ctx *c);
 int green_project(evpgpu_ctx *c);
 // newton.hip
+// The loop's per-voxel update: sigma, the block partials (nblk_out rows of
+// NRED, up to one set per crystal phase) and, with fast off, edot and gamdot
+// (with fast on both buffers keep what they held).
 int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, double *sig, const double *E,
                   const double *epsp, double *edot, const double *tran, const double *crss,
                   double *gamdot, const int *phase, const int *orient, const double *sgr,
-                  long long n, double *partials, int *nblk_out, int *status,
-                  double *err_vox, int *niter_vox, int fast, hipEvent_t ev_start = nullptr,
-                  hipEvent_t ev_stop = nullptr);
+                  long long n, double *partials, int *nblk_out, int *status, int fast,
+                  hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
+// rate-law evaluation: 0 non-integral exponent, 1 integral, 2 integral n <= 32
+// with 12 systems of one n and one gam0 in every crystal phase
+int newton_rate_mode(const NewtonParams &P);
+// newton_batch.hip: the power-law update of a caller's batch, with each
+// voxel's error norms and Newton count
+int newton_batch_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, double *sig, const double *E,
+                        const double *epsp, double *edot, const double *tran, const double *crss, double *gamdot,
+                        const int *phase, const int *orient, const double *sgr, long long n, int *status,
+                        double *err_vox, int *niter_vox);
 // the Newton kernel's parameters of a context (evpgpu.hip)
 NewtonParams context_newton_params(const evpgpu_ctx *c);
 // column sums of partials[nblk][nval] into out[0..nval); with status, also

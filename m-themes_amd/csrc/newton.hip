@@ -3,30 +3,37 @@
 // lane, plus the block partial sums of the convergence norms and the stress
 // averages that get_smacro needs (src/evolution.c:1415-1437, 473-497).
 //
-// The arithmetic follows the reference's: the same residual and rate law in
-// the same basis, the NR_MODIFIED backtracking line search with its
-// constants, branches and the TOLX rejection of small steps.  Rewritten, with
-// the same mathematics:
+// The arithmetic follows the reference's: the same equations in the same
+// basis, the NR_MODIFIED backtracking line search with its constants, branches
+// and the TOLX rejection of small steps.  Rewritten, with the same
+// mathematics:
 //   * the Newton step: J step = -R with J = I + C0 (S + dt D) is solved as
 //     K step = -S0 R with the symmetric positive definite K = S0 + S + dt D
-//     (S0 = C0^-1) by Cholesky, and the merit gradient J^T R as K (C0 R) --
-//     the reference forms LU_inv_66(J) with pivoting and multiplies;
+//     (S0 = C0^-1) by an L D L^T factorisation -- the reference forms
+//     LU_inv_66(J) with pivoting and multiplies; the slope of the merit
+//     function along that step is -|R|^2;
 //   * S = LU_inv_66(C_gr) is a per-orientation constant (read from a table,
 //     upper triangle), and d(edot)/d(sigma) is symmetric, so only upper
-//     triangles are formed; NR_quality never uses d(edot)/d(sigma);
+//     triangles are formed;
+//   * rates in the crystal axes, where the Schmid tensors are constants of the
+//     phase (scalar registers), between two 5x5 rotations of the voxel;
 //   * |x|^n by repeated squaring for integral n, 1/CRSS multiplied instead of
-//     divided, Schmid tensors as sym((Rn) x (Rb)), fused multiply-adds.
+//     divided, fused multiply-adds.
 // A non-positive-definite K returns status 35, the reference's singular-LU
 // exit.
 //
-// Data placement: the 12x5 Schmid tensors of a voxel are derived at kernel
-// start from its rotation (72 B read instead of 480 B) and kept in a
-// wave-private LDS slab laid out [component][lane] (conflict-free), which
-// keeps them out of the register file; C0 and S0 (packed triangles) are a
-// 42-entry LDS table read by broadcast; all other per-voxel arrays live in
-// registers with compile-time indices only.  One wave per SIMD: the solve
-// holds about 420 registers, so the code is shaped for latency (next Schmid
-// vector read ahead, constants hoisted, no scalar loops on the hot path).
+// What bounds it: FP64 vector issue, two waves per SIMD (256 registers each).
+// One voxel per lane; K0 = S0 + S, the rotation, the stress and the residual
+// stay in registers (116 of them), what is read once per evaluation (1/CRSS,
+// d, the tangent's weights) in LDS columns of the lane (15 KB per wave), the
+// constants arrive by scalar loads.  The 12 Schmid tensors in sample axes, as
+// an LDS slab of 30 KB per wave, held the kernel at one wave per SIMD, with
+// 5 LDS reads per system and evaluation, and every iteration evaluated the
+// accepted trial a second time.  Per launch, before and after: 583 -> 266 us at
+// 128^3 with 2 % pores (iterations 1-200 of an increment, n = 10), 81 -> 40 us
+// at 64^3, 118 -> 74 us at 64^3 under the dislocation-density law, 110 -> 37 us at
+// 24^3 with a non-integral exponent (pow() of each system once per evaluation
+// instead of twice, and one evaluation in three less).
 #include <hip/hip_ext.h>
 
 #include "evpgpu_impl.h"
@@ -108,8 +115,8 @@ __device__ __forceinline__ void v6_to_sym(const double v[6], double t[6])
     t[5] = v[4] * r2;
 }
 
-// 1/d for a positive normal d: the hardware estimate refined by two Newton
-// steps y += y (1 - d y) (the relative error e becomes e^2 per step)
+// 1/d for a normal d: the hardware estimate refined by two Newton steps
+// y += y (1 - d y) (the relative error e becomes e^2 per step)
 __device__ __forceinline__ double rcp_refined(double d)
 {
     double y = __builtin_amdgcn_rcp(d);
@@ -121,609 +128,598 @@ __device__ __forceinline__ double rcp_refined(double d)
     return y;
 }
 
-constexpr int NB_THREADS = 64; // one wave per block: the LDS slab is wave-private
+constexpr int NB_THREADS = 64; // one wave per block: the LDS columns are wave-private
 
-struct RateIn {
-    const double *sc;                              // LDS slab, sc[(s*5+j)*64]
-    const double *k0;                              // LDS: C0 then S0, packed triangles
-    double itf[EVPGPU_NSYSMX], itb[EVPGPU_NSYSMX]; // 1/CRSS forward, backward;
-                                                   // RM_DISL: itf the passing stress
-    const double *tpn;                             // RM_DISL: this voxel's constants, system
-    long long tps;                                 // stride tps: passing stress, 1/(tau_0 +
-                                                   // tau_cut), gam_o, first passing stress
-};
-#define SC(i, j) in.sc[((i)*5 + (j)) * NB_THREADS]
+// The kernel's NewtonParams (its first argument) in the kernel-argument
+// segment: wave-uniform reads from it become scalar loads.  fresh() hides the
+// address from the optimiser and ties it to a value the arithmetic before it
+// produces, so that a block of constants is loaded about where it is used:
+// hoisted they would not fit the scalar registers, and each use of a spilled
+// one costs two lane reads.
+typedef const __attribute__((address_space(4))) double *cdouble;
 
-// StrainRate_eval (src/constitutive.c:5-67) as one pass over the slip
-// systems: each system's Schmid vector is read from LDS once and feeds the
-// resolved shear, the rate, edot and d(edot)/d(sigma).  The sums run over the
-// systems in ascending order, as the reference's separate loops do.
-// DD: dt d(edot)/d(sigma) is added into the packed Newton matrix kk (which
-// holds S0 + S on entry).  GD: the slip rates are kept (gamdot).
-template <bool DD, int RM, bool GD, int NE>
-__device__ __forceinline__ void srate(const NewtonParams &P, int p, const RateIn &in,
-                                      const double s[6], double ed[5], double kk[21],
-                                      double gd[EVPGPU_NSYSMX])
+__device__ __forceinline__ cdouble params_at(size_t byte)
 {
-    // (the per-system test stays a branch on the phase's count even where it
-    // is always 12: without it the compiler interleaves the systems'
-    // arithmetic and the fast variant spills)
-    const int ns = P.nsys[p];
+    return (cdouble)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + byte);
+}
+
+__device__ __forceinline__ cdouble fresh(cdouble p, const double &after)
+{
+    __asm__ volatile("" : "+s"(p) : "v"(after) : "memory");
+    return p;
+}
+
+// the same after every one of n accumulators has been brought up to date (a
+// sum left for later would keep its constants in scalar registers)
+template <int N> __device__ __forceinline__ cdouble fresh_after(cdouble p, const double (&a)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N; i++) __asm__ volatile("" ::"v"(a[i]));
+    return fresh(p, a[0]);
+}
+
+// n Schmid constants (5 per system) from m
+template <int N> struct Consts {
+    double c[N];
+};
+template <int N> __device__ __forceinline__ Consts<N> load_consts(cdouble m)
+{
+    Consts<N> o;
+#pragma unroll
+    for (int i = 0; i < N; i++) o.c[i] = m[i];
+    return o;
+}
+
+// x^m of a wave-uniform or compile-time exponent, as the rate law needs it
+template <int RM, int NE> __device__ __forceinline__ double rate_power(double a, int intn, double nrs)
+{
+    if (RM == RM_FAST) return NE > 0 ? ipowc<(NE > 0 ? NE - 1 : 0)>(a) : ipow5(a, intn - 1);
+    if (RM == RM_LOOP) return ipow(a, intn - 1);
+    return pow(a, nrs - 1.);
+}
+
+// The slip systems are handled SYS_GROUP at a time: their Schmid constants
+// come in by scalar loads (5 doubles each) ahead of the group's arithmetic.
+constexpr int SYS_GROUP = 2;
+
+// StrainRate_eval (src/constitutive.c:5-67) at the stress s: edot (sample
+// axes).  Resolved shears and rates are formed in the crystal axes, where the
+// Schmid tensors are constants of the phase: Q (5x5, rotation of deviators
+// crystal -> sample, row-major) takes the stress in and the rate out.  The
+// derivative of each system's rate in its resolved shear, times dt, goes to
+// the lane's LDS column w (tangent() reads it if a Newton step follows).
+// it: LDS columns of 1/CRSS, forward then backward (RM_DISL: the passing
+// stress, then 1/(tau_0 + tau_cut)).  GD: the slip rates are written.
+template <int RM, bool CSYM, bool GD, int NE>
+__device__ __forceinline__ void rates(const NewtonParams &P, int p, const double *it, double *w,
+                                      const double *g0c, long long N, const double Q[25],
+                                      const double s[6], double ed[5], double *gd, bool keep)
+{
+    const int ns = RM == RM_FAST || RM == RM_DISL ? EVPGPU_NSYSMX : P.nsys[p];
     const int intn = P.int_n[p];
-    // RM_FAST: the phase's rate constants, as the general path multiplies
-    // them ((gam0 n) p1) itau
-    const double g0 = P.gam0[p][0], g0n = P.gam0[p][0] * P.nrs[p][0];
-    // RM_DISL: 1/(tau_0 + tau_cut) and gam_o of every system, loaded
-    // together before the loop (read at their use, under the per-lane test
-    // of the passing stress, each active system waited on its own loads)
-    double itcs[EVPGPU_NSYSMX], g0ks[EVPGPU_NSYSMX];
-    if (RM == RM_DISL) {
+    const double g0 = P.gam0[p][0], ndt = P.nrs[p][0] * P.dt;
+    double sc[5], e[5];
 #pragma unroll
-        for (int k = 0; k < EVPGPU_NSYSMX; k++) {
-            itcs[k] = in.tpn[(EVPGPU_NSYSMX + k) * in.tps];
-            g0ks[k] = in.tpn[(2 * EVPGPU_NSYSMX + k) * in.tps];
-        }
+    for (int j = 0; j < 5; j++) {
+        double a = Q[j] * s[0];
+#pragma unroll
+        for (int i = 1; i < 5; i++) a = fma(Q[5 * i + j], s[i], a);
+        sc[j] = a;
+        e[j] = 0.0;
     }
+    cdouble mx = params_at(offsetof(NewtonParams, mx)) + p * (EVPGPU_NSYSMX * 5);
+    Consts<5 * SYS_GROUP> next = load_consts<5 * SYS_GROUP>(fresh(mx, s[0]));
 #pragma unroll
-    for (int i = 0; i < 5; i++) ed[i] = 0.;
-    double scn[5];
+    for (int k0 = 0; k0 < EVPGPU_NSYSMX; k0 += SYS_GROUP) {
+        const Consts<5 * SYS_GROUP> m = next;
+        if (k0 + SYS_GROUP < EVPGPU_NSYSMX)
+            next = load_consts<5 * SYS_GROUP>(fresh_after(mx, e) + 5 * (k0 + SYS_GROUP));
 #pragma unroll
-    for (int j = 0; j < 5; j++) scn[j] = SC(0, j);
-#pragma unroll
-    for (int k = 0; k < EVPGPU_NSYSMX; k++) {
-        // the next system's Schmid vector is read before this one's
-        // arithmetic, so the LDS latency is hidden behind it
-        double sc[5];
-#pragma unroll
-        for (int j = 0; j < 5; j++) sc[j] = scn[j];
-        if (k + 1 < EVPGPU_NSYSMX)
-#pragma unroll
-            for (int j = 0; j < 5; j++) scn[j] = SC(k + 1, j);
-        if (k < ns) {
-            double r = sc[0] * s[0] + sc[1] * s[1] + sc[2] * s[2] + sc[3] * s[3] + sc[4] * s[4];
-            double r1 = 0.0, r2 = 0.0; // the rate and its derivative in the resolved shear
+        for (int k = k0; k < k0 + SYS_GROUP; k++) {
+            if (k >= ns) break;
+            const double *mk = m.c + 5 * (k - k0);
+            const double m0 = mk[0], m1 = mk[1], m2 = mk[2], m3 = mk[3], m4 = mk[4];
+            double r = m0 * sc[0];
+            r = fma(m1, sc[1], r);
+            r = fma(m2, sc[2], r);
+            r = fma(m3, sc[3], r);
+            r = fma(m4, sc[4], r);
+            double g, d; // the rate and dt times its derivative in the resolved shear
             if (RM == RM_DISL) {
                 // gam = gam_o sinh((|rss| - tau_pass)/(tau_0 + tau_cut)) sign(rss)
                 // above the passing stress, 0 below (FORWARD_PLUS_BACKWARD)
-                const double a = fabs(r);
-                if (a > in.itf[k]) {
-                    const double itc = itcs[k];
-                    const double g0k = g0ks[k];
-                    const double x = (a - in.itf[k]) * itc;
+                const double a = fabs(r), tp = it[k * NB_THREADS];
+                const double itc = it[(EVPGPU_NSYSMX + k) * NB_THREADS], g0k = g0c[k * N];
+                g = d = 0.0;
+                if (a > tp) {
+                    const double x = (a - tp) * itc;
                     // sinh and cosh from one expm1: with m = e^x - 1 and
                     // q = e^-x, sinh x = m (1 + q) / 2 (no cancellation at
                     // small x) and cosh x = (1 + m + q) / 2
-                    const double m = expm1(x), q = rcp_refined(1.0 + m);
-                    r2 = g0k * (0.5 * m * (1.0 + q)) * (double)(2 * (r > 0) - 1);
-                    if (DD) r1 = g0k * (0.5 * ((1.0 + m) + q)) * itc;
+                    const double em = expm1(x), q = rcp_refined(1.0 + em);
+                    g = copysign(g0k * (0.5 * em * (1.0 + q)), r);
+                    d = g0k * (0.5 * ((1.0 + em) + q)) * itc * P.dt;
                 }
             } else {
-            double itau = (r < 0) ? in.itb[k] : in.itf[k];
-            r = r * itau;
-            double a = fabs(r), p1, p2;
-            if (RM == RM_FAST) {
-                p1 = NE > 0 ? ipowc<(NE > 0 ? NE - 1 : 0)>(a) : ipow5(a, intn - 1);
-                p2 = p1 * a;
-            } else if (RM == RM_LOOP) {
-                p1 = ipow(a, intn - 1);
-                p2 = p1 * a;
-            } else {
-                p1 = pow(a, P.nrs[p][k] - 1.);
-                p2 = pow(a, P.nrs[p][k]);
+                const double itau = CSYM ? it[k * NB_THREADS]
+                                         : it[((r < 0 ? EVPGPU_NSYSMX : 0) + k) * NB_THREADS];
+                const double x = r * itau, a = fabs(x);
+                const double p1 = (RM == RM_FAST ? g0 : P.gam0[p][k]) * rate_power<RM, NE>(a, intn, P.nrs[p][k]);
+                g = p1 * x;
+                // n < 1: |x|^(n-1) has no value at x = 0, |x|^n has
+                if (RM == RM_POW && P.nrs[p][k] < 1.0)
+                    g = copysign(P.gam0[p][k] * pow(a, P.nrs[p][k]), x);
+                d = (p1 * itau) * (RM == RM_FAST ? ndt : P.nrs[p][k] * P.dt);
             }
-            r2 = (RM == RM_FAST ? g0 : P.gam0[p][k]) * p2 * (double)(2 * (r > 0) - 1);
-            if (DD) r1 = (RM == RM_FAST ? g0n : P.gam0[p][k] * P.nrs[p][k]) * p1 * itau;
-            }
-            if (GD) gd[k] = r2;
+            if (GD && keep) gd[k * N] = g;
+            w[k * NB_THREADS] = d;
+            e[0] = fma(m0, g, e[0]);
+            e[1] = fma(m1, g, e[1]);
+            e[2] = fma(m2, g, e[2]);
+            e[3] = fma(m3, g, e[3]);
+            e[4] = fma(m4, g, e[4]);
+        }
+    }
 #pragma unroll
-            for (int i = 0; i < 5; i++) ed[i] += sc[i] * r2;
-            if (DD) {
-                r1 *= P.dt;
+    for (int i = 0; i < 5; i++) {
+        double a = Q[5 * i] * e[0];
 #pragma unroll
-                for (int i = 0; i < 5; i++) {
-                    const double w = sc[i] * r1;
+        for (int j = 1; j < 5; j++) a = fma(Q[5 * i + j], e[j], a);
+        ed[i] = a;
+    }
+}
+
+// K = K0 + dt d(edot)/d(sigma) (packed upper triangle) from the weights the
+// last rates() left: D' = sum_k w_k m_k m_k^T in crystal axes, then Q D' Q^T.
+__device__ __forceinline__ void tangent(int ns, int p, const double *w, const double Q[25],
+                                        const double K0[21], double K[21])
+{
+    double D[15]; // upper triangle, row by row
 #pragma unroll
-                    for (int j = i; j < 5; j++) kk[PK(i, j)] += w * sc[j];
-                }
+    for (int i = 0; i < 15; i++) D[i] = 0.0;
+    cdouble mx = params_at(offsetof(NewtonParams, mx)) + p * (EVPGPU_NSYSMX * 5);
+    Consts<5 * SYS_GROUP> next = load_consts<5 * SYS_GROUP>(fresh(mx, K0[0]));
+#pragma unroll
+    for (int k0 = 0; k0 < EVPGPU_NSYSMX; k0 += SYS_GROUP) {
+        const Consts<5 * SYS_GROUP> mc = next;
+        if (k0 + SYS_GROUP < EVPGPU_NSYSMX)
+            next = load_consts<5 * SYS_GROUP>(fresh_after(mx, D) + 5 * (k0 + SYS_GROUP));
+#pragma unroll
+        for (int k = k0; k < k0 + SYS_GROUP; k++) {
+            if (k >= ns) break;
+            const double *m = mc.c - 5 * k0;
+            const double wk = w[k * NB_THREADS];
+            int c = 0;
+#pragma unroll
+            for (int i = 0; i < 5; i++) {
+                const double a = wk * m[5 * k + i];
+#pragma unroll
+                for (int j = i; j < 5; j++, c++) D[c] = fma(a, m[5 * k + j], D[c]);
             }
         }
     }
-}
-
-// 1/sqrt(d) for a positive normal d: the hardware estimate refined by two
-// Newton steps y += y (1 - d y^2) / 2 (the estimate's relative error e
-// becomes about 1.5 e^2 per step), to within about an ulp
-__device__ __forceinline__ double rsqrt_refined(double d)
-{
-    double y = __builtin_amdgcn_rsq(d);
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const double e = fma(-(d * y), y, 1.0);
-        y = fma(0.5 * y, e, y);
+    for (int i = 0; i < 5; i++) {
+        double t[5]; // row i of Q D'
+#pragma unroll
+        for (int j = 0; j < 5; j++) {
+            double a = 0.0;
+#pragma unroll
+            for (int q = 0; q < 5; q++) {
+                const int lo = q < j ? q : j, hi = q < j ? j : q;
+                const double d = D[lo * 5 - lo * (lo - 1) / 2 + (hi - lo)];
+                a = q == 0 ? Q[5 * i] * d : fma(Q[5 * i + q], d, a);
+            }
+            t[j] = a;
+        }
+#pragma unroll
+        for (int j = i; j < 5; j++) {
+            double a = K0[PK(i, j)];
+#pragma unroll
+            for (int q = 0; q < 5; q++) a = fma(t[q], Q[5 * j + q], a);
+            K[PK(i, j)] = a;
+        }
+        K[PK(i, 5)] = K0[PK(i, 5)];
     }
-    return y;
+    K[PK(5, 5)] = K0[PK(5, 5)];
 }
 
-// Cholesky factorisation of the packed symmetric 6x6 k (in place: the lower
-// factor L, stored transposed in the same packing) and the solve
-// L L^T x = b (b overwritten).  Returns false if k is not positive definite.
-__device__ __forceinline__ bool chol6_solve(double k[21], double b[6])
+// L D L^T of the packed symmetric 6x6 k (in place) and the solve k x = b (b
+// overwritten).  Returns false if k is not positive definite.
+__device__ __forceinline__ bool ldl6_solve(double k[21], double b[6])
 {
     double inv[6];
+    bool pd = true;
 #pragma unroll
     for (int j = 0; j < 6; j++) {
-        double d = k[PK(j, j)];
-#pragma unroll
-        for (int q = 0; q < j; q++) d -= k[PK(q, j)] * k[PK(q, j)];
-        if (!(d > 0.0)) return false;
-        inv[j] = rsqrt_refined(d);
+        // column j of L scaled by its pivot stays in k; the update of the
+        // columns after it takes L_ij from k_ij inv_j
+        const double d = k[PK(j, j)];
+        pd = pd && d > 0.0;
+        inv[j] = rcp_refined(d);
 #pragma unroll
         for (int i = j + 1; i < 6; i++) {
-            double s = k[PK(j, i)];
+            const double l = k[PK(j, i)] * inv[j];
 #pragma unroll
-            for (int q = 0; q < j; q++) s -= k[PK(q, i)] * k[PK(q, j)];
-            k[PK(j, i)] = s * inv[j];
+            for (int q = i; q < 6; q++) k[PK(i, q)] = fma(-l, k[PK(j, q)], k[PK(i, q)]);
+            b[i] = fma(-l, b[j], b[i]);
         }
-    }
-#pragma unroll
-    for (int i = 0; i < 6; i++) {
-        double s = b[i];
-#pragma unroll
-        for (int q = 0; q < i; q++) s -= k[PK(q, i)] * b[q];
-        b[i] = s * inv[i];
     }
 #pragma unroll
     for (int i = 5; i >= 0; i--) {
         double s = b[i];
 #pragma unroll
-        for (int q = i + 1; q < 6; q++) s -= k[PK(i, q)] * b[q];
+        for (int q = i + 1; q < 6; q++) s = fma(-k[PK(i, q)], b[q], s);
         b[i] = s * inv[i];
     }
-    return true;
+    return pd;
 }
 
-// An empty asm statement that takes x in a register: the value must be
-// ready at this point (its load is not moved below it)
-__device__ __forceinline__ void keep_reg(const double &x)
+// y = A x for a packed symmetric 6x6 A of NewtonParams, added to y
+__device__ __forceinline__ void sym6_mul_add(cdouble A, const double x[6], double y[6])
 {
-    __asm__ volatile("" ::"v"(x));
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+#pragma unroll
+        for (int j = 0; j < 6; j++) y[i] = fma(A[PK(i, j)], x[j], y[i]);
 }
 
-// Per-voxel constants of the Newton solve: the compliance S = LU_inv_66(C_gr)
-// (symmetric; its upper triangle), lambda and eps_p - E in the B-basis.
-struct Vox {
-    double S[21];
-    double xl[6], bp[6];
-    double signorm; // Frobenius norm of lambda (src/evolution.c:92-96)
-};
-
-// R(s) = s - lambda + C0 t,  t = eps_p + dt edot(s) + S s - E
-// (src/evolution.c:126-140; t is the strain mismatch of the error norm)
-__device__ __forceinline__ void residual(const NewtonParams &P, const RateIn &in, const Vox &V,
-                                         const double sig[6],
-                                         const double ed[5], double t[6], double res[6])
+// r = K0 s + dt edot + d (d: LDS columns)
+__device__ __forceinline__ void scaled_residual(double dt, const double K0[21], const double *d,
+                                                const double s[6], const double ed[5], double r[6])
 {
 #pragma unroll
     for (int i = 0; i < 6; i++) {
-        double a = V.bp[i] + (i < 5 ? ed[i] * P.dt : 0.0);
+        double a = i < 5 ? fma(ed[i], dt, d[i * NB_THREADS]) : d[i * NB_THREADS];
 #pragma unroll
-        for (int j = 0; j < 6; j++) a += V.S[PK(i, j)] * sig[j];
-        t[i] = a;
-    }
-#pragma unroll
-    for (int i = 0; i < 6; i++) {
-        double r = sig[i] - V.xl[i];
-#pragma unroll
-        for (int j = 0; j < 6; j++) r += in.k0[PK(i, j)] * t[j];
-        res[i] = r;
+        for (int j = 0; j < 6; j++) a = fma(K0[PK(i, j)], s[j], a);
+        r[i] = a;
     }
 }
 
-template <int RM, bool GD, int NE>
-__device__ __forceinline__ double nr_quality(const NewtonParams &P, int p, const RateIn &in,
-                                             const Vox &V, const double sig[6],
-                                             double gd[EVPGPU_NSYSMX])
+__device__ __forceinline__ double norm2(const double v[6])
 {
-    double ed[5], t[6], res[6];
-    srate<false, RM, GD, NE>(P, p, in, sig, ed, nullptr, gd);
-    residual(P, in, V, sig, ed, t, res);
-    double f = 0.0;
+    double a = v[0] * v[0];
 #pragma unroll
-    for (int i = 0; i < 6; i++) f += res[i] * res[i];
-    return f / 2.0;
+    for (int i = 1; i < 6; i++) a = fma(v[i], v[i], a);
+    return a;
 }
 
-// returns 0, EVPGPU_ERR_SINGULAR or EVPGPU_ERR_LINESEARCH
-// FAST: an iteration whose step the reference's line search is certain to
-// reject (TOLX) ends right after the residual.  Since D >= 0, K = S0 + S +
-// dt D >= S0 + S, so |step|_inf <= |S0 R|_2 / lambda_min(S0 + S); when that
-// bound is below TOLX (P.kmin_tolx2 holds (0.99 TOLX lambda_min)^2, the
-// minimum over all orientations) the reference's test
-// max|step_i|/max(|s_i|,1) < TOLX holds and its first trial is rejected,
-// leaving s, edot, the error norms and the
-// counts exactly as computed here.  Only gamdot (from the rejected trial
-// point) differs; the loop recomputes the last Newton launch of an increment
-// with FAST off before gamdot is used, so FAST launches do not form gamdot.
-template <int RM, bool FAST, int NE>
-__device__ int update_voxel(const NewtonParams &P, int p, RateIn &in, const Vox &V,
-                            double sig6[6], double edotp[6], double gd[EVPGPU_NSYSMX],
-                            double &conv_s, double &conv_e, int &iterl, int &trials)
+// The rotation of deviators, crystal -> sample, for the orientation T (3x3,
+// row-major): column j of Q (5x5, row-major) is the 5-vector of T B_j T^T, from
+// the products of T's columns.
+__device__ __forceinline__ void rotation5(const double T[9], double Q[25])
 {
-    constexpr bool GD = !FAST;
-    trials = 0;
-    double ed[5], res[6], old[6], k[21];
-    double ce = 0.0;
-    iterl = 0;
-    double erral = 10 * P.nr_tol;
+    double dg[3][5]; // sqrt 2 times the 5-vectors of c_a c_a^T
 #pragma unroll
-    for (int i = 0; i < 6; i++) sig6[i] = V.xl[i];
-    while ((iterl < 500) && (fabs(erral) > fabs(P.nr_tol))) {
-        // read C0, S0 and the Schmid vectors from LDS where they are used:
-        // hoisted out of the loop they would occupy 204 more registers
-        __asm__ volatile("" ::: "memory");
-        iterl++;
-#pragma unroll
-        for (int i = 0; i < 6; i++) old[i] = sig6[i];
-        // the Newton matrix K = S0 + S + dt D (below), D added by srate
-#pragma unroll
-        for (int i = 0; i < 6; i++)
-#pragma unroll
-            for (int j = i; j < 6; j++) k[PK(i, j)] = in.k0[21 + PK(i, j)] + V.S[PK(i, j)];
-        srate<true, RM, GD, NE>(P, p, in, sig6, ed, k, gd);
-        if (RM == RM_DISL && P.dd_first && iterl == 1) {
-            // the first call used the previous call's mobile density; every
-            // later one sees the density that call formed
-#pragma unroll
-            for (int s = 0; s < EVPGPU_NSYSMX; s++)
-                if (s < P.nsys[p]) in.itf[s] = in.tpn[s * in.tps];
-        }
-#pragma unroll
-        for (int i = 0; i < 6; i++) edotp[i] = i < 5 ? ed[i] : 0.0;
-        double gradf[6], step[6];
-        {
-            double t[6];
-            residual(P, in, V, sig6, ed, t, res);
-            ce = 0.0;
-#pragma unroll
-            for (int i = 0; i < 6; i++) ce += t[i] * t[i];
-        }
-        // S0 R: the right-hand side of the step, and its norm bounds the step
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            double b = 0.0;
-#pragma unroll
-            for (int j = 0; j < 6; j++) b += in.k0[21 + PK(i, j)] * res[j];
-            step[i] = b;
-        }
-        bool skip = false;
-        if (FAST) {
-            double y2 = 0.0;
-#pragma unroll
-            for (int i = 0; i < 6; i++) y2 += step[i] * step[i];
-            skip = (y2 > 0.0) && (y2 < P.kmin_tolx2);
-        }
-        if (skip) {
-            trials++; // the reference's one rejected trial
-        } else {
-        {
-            // The Newton matrix J = I + C0 (S + dt D) times S0 = C0^-1 is the
-            // symmetric positive definite K = S0 + S + dt D: the step solves
-            // K step = -S0 R (Cholesky), and the merit-function gradient
-            // J^T R = R + (S + dt D) C0 R equals K (C0 R).
-            double u[6];
-#pragma unroll
-            for (int i = 0; i < 6; i++) {
-                double a = 0.0;
-#pragma unroll
-                for (int j = 0; j < 6; j++) a += in.k0[PK(i, j)] * res[j];
-                u[i] = a;
-            }
-#pragma unroll
-            for (int i = 0; i < 6; i++) {
-                double g = 0.0;
-#pragma unroll
-                for (int j = 0; j < 6; j++) g += k[PK(i, j)] * u[j];
-                gradf[i] = g;
-            }
-            if (!chol6_solve(k, step)) return EVPGPU_ERR_SINGULAR;
-#pragma unroll
-            for (int i = 0; i < 6; i++) step[i] = -step[i];
-        }
-        double f_old = 0.0;
-#pragma unroll
-        for (int i = 0; i < 6; i++) f_old += res[i] * res[i];
-        f_old *= 0.5;
-        const double stpmax = 10.0, ALF = 1.E-4, TOLX = P.tolx;
-        double sum = 0.0, slope = 0.0, test = 0.0;
-#pragma unroll
-        for (int i = 0; i < 6; i++) sum += step[i] * step[i];
-        sum = sqrt(sum);
-        if (sum > stpmax) {
-#pragma unroll
-            for (int i = 0; i < 6; i++) step[i] *= stpmax / sum;
-        }
-#pragma unroll
-        for (int i = 0; i < 6; i++) slope += gradf[i] * step[i];
-        if (slope >= 0) return EVPGPU_ERR_LINESEARCH;
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            double d = fabs(old[i]);
-            double t = fabs(step[i]) / (d > 1.0 ? d : 1.0);
-            if (t > test) test = t;
-        }
-        double alamin = TOLX / test, alam = 1.0, alam2 = 0.0, f2 = 0.0;
-        // The first trial (alam = 1) is rejected when 1 < alamin, whatever
-        // its merit value: the step is left undone and only gamdot (from the
-        // trial point) is affected, which FAST launches do not form -- so
-        // they skip the evaluation.  This is how nearly every voxel's solve
-        // ends: an accepted step has relative size >= TOLX, which keeps the
-        // relative-step test (1e-10) open, so the last step is a TOLX reject.
-        if (FAST && alam < alamin) {
-            trials++;
-        } else {
-        while (true) {
-            __asm__ volatile("" ::: "memory");
-#pragma unroll
-            for (int i = 0; i < 6; i++) sig6[i] = old[i] + alam * step[i];
-            double f_new = nr_quality<RM, GD, NE>(P, p, in, V, sig6, gd);
-            trials++;
-            if (alam < alamin) {
-#pragma unroll
-                for (int i = 0; i < 6; i++) sig6[i] = old[i];
-                break;
-            } else if (f_new <= f_old + ALF * alam * slope) {
-                break;
-            }
-            const double next = ls_backtrack(alam, alam2, f_new, f2, f_old, slope);
-            alam2 = alam;
-            f2 = f_new; // the backtrack value the cubic step needs (Q18)
-            alam = next;
-        }
-        } // line search
-        } // !skip
-        double conv_nr = 0.0;
-#pragma unroll
-        for (int i = 0; i < 6; i++) conv_nr += (sig6[i] - old[i]) * (sig6[i] - old[i]);
-        erral = sqrt(conv_nr) / V.signorm;
+    for (int a = 0; a < 3; a++) {
+        const double x = T[a], y = T[3 + a], z = T[6 + a];
+        const double xx = x * x, yy = y * y, zz = z * z;
+        dg[a][0] = yy - xx;
+        dg[a][1] = (2.0 * zz - xx - yy) * RSQ3;
+        dg[a][2] = 2.0 * (y * z);
+        dg[a][3] = 2.0 * (x * z);
+        dg[a][4] = 2.0 * (x * y);
     }
-    // the norms of the last iteration (the reference overwrites them in
-    // every iteration)
-    double cs = 0.0;
+    // B_0 = (e1e1 - e0e0)/sqrt 2, B_1 = (2 e2e2 - e0e0 - e1e1)/sqrt 6
 #pragma unroll
-    for (int i = 0; i < 6; i++) cs += (sig6[i] - V.xl[i]) * (sig6[i] - V.xl[i]);
-    conv_s = sqrt(cs);
-    conv_e = sqrt(ce);
-    return 0;
+    for (int i = 0; i < 5; i++) {
+        Q[5 * i] = 0.5 * (dg[1][i] - dg[0][i]);
+        Q[5 * i + 1] = (0.5 * RSQ3) * (2.0 * dg[2][i] - dg[0][i] - dg[1][i]);
+    }
+    // B_2, B_3, B_4: sym(e1e2), sym(e0e2), sym(e0e1) times sqrt 2
+    const int ca[3] = {1, 0, 0}, cb[3] = {2, 2, 1};
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const double x0 = T[ca[q]], y0 = T[3 + ca[q]], z0 = T[6 + ca[q]];
+        const double x1 = T[cb[q]], y1 = T[3 + cb[q]], z1 = T[6 + cb[q]];
+        const double xx = x0 * x1, yy = y0 * y1, zz = z0 * z1;
+        Q[2 + q] = yy - xx;
+        Q[7 + q] = (2.0 * zz - xx - yy) * RSQ3;
+        Q[12 + q] = fma(y0, z1, z0 * y1);
+        Q[17 + q] = fma(x0, z1, z0 * x1);
+        Q[22 + q] = fma(x0, y1, y0 * x1);
+    }
+}
+
+// merit function of NR_MODIFIED: |R|^2 / 2 with R = C0 r
+__device__ __forceinline__ double merit(const double r[6])
+{
+    double R[6] = {0., 0., 0., 0., 0., 0.};
+    sym6_mul_add(fresh(params_at(offsetof(NewtonParams, c0p)), r[0]), r, R);
+    return 0.5 * norm2(R);
 }
 
 // One lane per voxel.  Reads lambda from sig_in and writes the new stress to
-// sig (separate buffers), edot and -- with FAST off -- gamdot; block partials
-// (NRED doubles per block) of err_s, err_e, Newton iterations, sum sig, sum
-// sig over phase 1 and line-search trials.
+// sig (the same buffer or another) and, with FAST off, edot and gamdot; block
+// partials (NRED doubles per block) of err_s, err_e, Newton iterations, sum
+// sig, sum sig over phase 1 and line-search trials.
+//
+// The update works on r = S0 R, R the reference's residual
+// s - lambda + C0 (eps_p + dt edot(s) + S s - E): with K0 = S0 + S and
+// d = eps_p - E - S0 lambda it is r = K0 s + dt edot(s) + d, the Newton step
+// solves (K0 + dt D) step = -r, and R itself is needed only where the line
+// search has to compare |R|^2.  An accepted trial's rates and residual are
+// the next iteration's start, and its tangent is formed only if that
+// iteration takes a step.
+//
+// FAST: an iteration whose step the reference's line search is certain to
+// reject (TOLX) ends right after the residual.  Since D >= 0, K = S0 + S +
+// dt D >= S0 + S, so |step|_inf <= |r|_2 / lambda_min(S0 + S); when that
+// bound is below TOLX (P.kmin_tolx2 holds (0.99 TOLX lambda_min)^2, the
+// minimum over all orientations) the reference's test
+// max|step_i|/max(|s_i|,1) < TOLX holds and its first trial is rejected,
+// leaving s, edot, the error norms and the counts exactly as computed here.
+// Only gamdot (from the rejected trial point) differs; the loop repeats the
+// last Newton launch of an increment with FAST off before edot or gamdot is
+// used, so FAST launches write neither.
 template <int RM, bool CSYM, bool FAST, int NE>
-__global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_newton(
-    NewtonParams P, long long N, const int *__restrict__ phase, const int *__restrict__ orient,
-    const double *__restrict__ sgr, const double *sig_in, double *sig, const double *__restrict__ E,
-    const double *__restrict__ epsp, double *__restrict__ edot, const double *__restrict__ tran,
-    const double *__restrict__ crss, double *__restrict__ gamdot, double *__restrict__ partials,
-    int *__restrict__ status, double *__restrict__ err_vox, int *__restrict__ niter_vox)
+__global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_newton(
+    NewtonParams P, long long N, int p, int lead, const int *__restrict__ phase,
+    const int *__restrict__ orient, const double *__restrict__ sgr, const double *sig_in, double *sig,
+    const double *__restrict__ E, const double *__restrict__ epsp, double *__restrict__ edot,
+    const double *__restrict__ tran, const double *__restrict__ crss, double *__restrict__ gamdot,
+    double *__restrict__ partials, int *__restrict__ status)
 {
     if (P.skip && *P.skip) return;
-    __shared__ double slab[EVPGPU_NSYSMX * 5 * NB_THREADS];
-    // C0 and S0 (packed upper triangles) as broadcast LDS reads: kept in
-    // scalar registers they do not fit, and each use of a spilled one costs
-    // two lane reads
-    __shared__ double k0[42];
-    long long v = (long long)blockIdx.x * NB_THREADS + threadIdx.x;
-    // the voxel's phase and orientation index go out with the C0/S0 loads,
-    // unconditionally (a lane past the end reads the last voxel's and drops
-    // them), so that one wait covers all four: with one wave per SIMD every
-    // wait on memory stalls the SIMD
-    const long long vc = v < N ? v : N - 1;
-    const int ph_raw = phase[vc], ori = orient[vc];
-    const double c0v = P.c0p[threadIdx.x % 21], s0v = P.s0p[threadIdx.x % 21];
-    const int ph = v < N ? ph_raw : 1;
-    if (threadIdx.x < 21) {
-        k0[threadIdx.x] = c0v;
-        k0[21 + threadIdx.x] = s0v;
-    }
-    __syncthreads();
-    // this lane's err_s, err_e, Newton iterations and line-search trials
-    double r_cs = 0.0, r_ce = 0.0, r_it = 0.0, r_tr = 0.0;
-    int pl = 0;
-    if (v < N) {
-        pl = ph - 1;
-        pl = pl < 0 ? 0 : (pl > 1 ? 1 : pl);
-    }
-    // the two phases' gas flags as a select of kernel arguments, not an
-    // indexed (memory) read
+    constexpr bool GD = !FAST;
+    // LDS columns: 1/CRSS, the tangent's weights, d and (FAST off) edot
+    constexpr int NIT = CSYM ? EVPGPU_NSYSMX : 2 * EVPGPU_NSYSMX, ND = NIT + EVPGPU_NSYSMX;
+    __shared__ double slab[(ND + 6 + (FAST ? 0 : 5)) * NB_THREADS];
+    const int lane = threadIdx.x;
+    const long long v0 = (long long)blockIdx.x * NB_THREADS + lane;
+    // a lane past the end takes the last voxel's inputs and drops the result
+    const unsigned v = (unsigned)(v0 < N ? v0 : N - 1);
+    const int ph = phase[v], ori = orient[v];
+    const int pl = ph - 1 < 0 ? 0 : (ph - 1 > 1 ? 1 : ph - 1);
     const bool gas_l = pl == 0 ? P.is_gas[0] != 0 : P.is_gas[1] != 0;
-    // Crystal voxels, one phase of the wave at a time: inside the loop the
-    // phase index p is wave-uniform, so the rate-law constants, slip-system
-    // counts and crystal axes are scalar operands and the slip-system loops
-    // branch on scalars (a wave holds one crystal phase almost always).
-    bool pending = v < N && !gas_l;
-    // every pass clears at least the lead lane, so it ends after one pass
-    // per distinct phase (two at most)
-    for (unsigned long long todo = __ballot(pending); todo; todo = __ballot(pending)) {
-        const int p = __builtin_amdgcn_readlane(pl, __ffsll(todo) - 1);
-        // lanes of phase p, tested through the ballot mask: a branch on
-        // pl == p itself would let the compiler substitute the per-lane pl
-        // for the uniform p inside the branch
-        const unsigned long long sel = __ballot(pending && pl == p);
-        if ((sel >> (threadIdx.x & 63)) & 1ull) {
-            pending = false;
-            Vox V;
-            RateIn in;
-            // every load of the voxel's inputs first -- stress, plastic and
-            // total strain, the orientation's S, the rotation and the
-            // per-system CRSS (all 12: the arrays hold them whatever the
-            // phase's count) -- then the arithmetic: one wait on memory
-            // instead of one per group
-            double t[6], tp[6], te[6], T9[9], c1[EVPGPU_NSYSMX], c2[EVPGPU_NSYSMX];
+    const bool mine = v0 < N && !gas_l && pl == p;
+    double *red = slab + lane; // the lane's NRED sums, in its own columns at the end
+    if (__any(mine)) {
+        double *it = slab + lane, *w = slab + NIT * NB_THREADS + lane;
+        double *dl = slab + ND * NB_THREADS + lane, *edl = slab + (ND + 6) * NB_THREADS + lane;
+        double K0[21], Q[25], s[6], r[6];
+        double sn2; // |lambda|_F^2 (src/evolution.c:92-96)
+        {
+            // every load of the voxel's inputs first, then the arithmetic
+            double d[6], t[6], tp[6], te[6], T9[9], c1[EVPGPU_NSYSMX], c2[EVPGPU_NSYSMX];
 #pragma unroll
             for (int c = 0; c < 6; c++) t[c] = sig_in[c * N + v];
 #pragma unroll
             for (int c = 0; c < 6; c++) tp[c] = epsp[c * N + v];
 #pragma unroll
             for (int c = 0; c < 6; c++) te[c] = E[c * N + v];
-            const double *sv = sgr + 36LL * ori;
-#pragma unroll
-            for (int i = 0; i < 6; i++)
-#pragma unroll
-                for (int j = i; j < 6; j++) V.S[PK(i, j)] = sv[i * 6 + j];
 #pragma unroll
             for (int q = 0; q < 9; q++) T9[q] = tran[q * N + v];
             const long long S12 = (long long)EVPGPU_NSYSMX * N;
 #pragma unroll
-            for (int s = 0; s < EVPGPU_NSYSMX; s++) {
+            for (int k = 0; k < EVPGPU_NSYSMX; k++) {
                 if (RM == RM_DISL) {
-                    c1[s] = crss[(P.dd_first ? 3 * S12 : 0) + s * N + v];
+                    // crss holds the increment's constants: passing stress,
+                    // 1/(tau_0 + tau_cut), gam_o, the first call's passing stress
+                    c1[k] = crss[(P.dd_first ? 3 * S12 : 0) + k * N + v];
+                    c2[k] = crss[S12 + k * N + v];
                 } else {
-                    c1[s] = crss[(s * 2) * N + v];
-                    c2[s] = CSYM ? c1[s] : crss[(s * 2 + 1) * N + v];
+                    c1[k] = crss[(k * 2) * N + v];
+                    if (!CSYM) c2[k] = crss[(k * 2 + 1) * N + v];
                 }
             }
-            // |lambda|_F over the full 3x3, row-major order
-            V.signorm = sqrt(t[0] * t[0] + t[5] * t[5] + t[4] * t[4] + t[5] * t[5] + t[1] * t[1] +
-                             t[3] * t[3] + t[4] * t[4] + t[3] * t[3] + t[2] * t[2]);
-            sym_to_v6(t, V.xl);
-            {
-                double e6[6], s6[6];
-                sym_to_v6(tp, e6);
-                sym_to_v6(te, s6);
+            const double *sv = sgr + 36LL * ori;
 #pragma unroll
-                for (int i = 0; i < 6; i++) V.bp[i] = e6[i] - s6[i];
-            }
-            // the fast variants have every crystal phase on 12 systems: a
-            // compile-time count keeps the per-system loops free of branches
-            const int ns = RM == RM_FAST || RM == RM_DISL ? EVPGPU_NSYSMX : P.nsys[p];
-            // Schmid tensors in sample axes: sym((T n) x (T b)) in the 5-D basis
-            // (update_schmid, src/kinematics.c:430-463), into this lane's LDS column
-            double T[3][3];
+            for (int i = 0; i < 6; i++)
 #pragma unroll
-            for (int q = 0; q < 9; q++) T[q / 3][q % 3] = T9[q];
-            in.sc = slab + threadIdx.x;
-            in.k0 = k0;
-            // unrolled (straight-line where the count is the constant 12), so
-            // that the loads above stay ahead of this arithmetic
+                for (int j = i; j < 6; j++) K0[PK(i, j)] = sv[i * 6 + j];
+            sn2 = t[0] * t[0] + t[1] * t[1] + t[2] * t[2] + 2.0 * (t[3] * t[3] + t[4] * t[4] + t[5] * t[5]);
+            sym_to_v6(t, s);
 #pragma unroll
-            for (int s = 0; s < EVPGPU_NSYSMX; s++) {
-                if (s >= ns) break;
-                double tn[3], tb[3];
+            for (int i = 0; i < 6; i++) te[i] = tp[i] - te[i];
+            sym_to_v6(te, d);
+            // d = eps_p - E - S0 lambda, K0 = S0 + S
+            cdouble S0 = fresh(params_at(offsetof(NewtonParams, s0p)), s[0]);
 #pragma unroll
-                for (int a = 0; a < 3; a++) {
-                    tn[a] = T[a][0] * P.bn[p][s][0] + T[a][1] * P.bn[p][s][1] + T[a][2] * P.bn[p][s][2];
-                    tb[a] = T[a][0] * P.bb[p][s][0] + T[a][1] * P.bb[p][s][1] + T[a][2] * P.bb[p][s][2];
-                }
-                double P00 = tn[0] * tb[0], P11 = tn[1] * tb[1], P22 = tn[2] * tb[2];
-                double P12 = (tn[1] * tb[2] + tn[2] * tb[1]) / 2.0;
-                double P02 = (tn[0] * tb[2] + tn[2] * tb[0]) / 2.0;
-                double P01 = (tn[0] * tb[1] + tn[1] * tb[0]) / 2.0;
-                double *col = slab + threadIdx.x + s * 5 * NB_THREADS;
-                col[0 * NB_THREADS] = P00 * (-1. * RSQ2) + P11 * RSQ2;
-                col[1 * NB_THREADS] = P00 * (-1. * RSQ6) + P11 * (-1. * RSQ6) + P22 * (2. * RSQ6);
-                col[2 * NB_THREADS] = P12 * RSQ2 + P12 * RSQ2;
-                col[3 * NB_THREADS] = P02 * RSQ2 + P02 * RSQ2;
-                col[4 * NB_THREADS] = P01 * RSQ2 + P01 * RSQ2;
-            }
-            // the voxel's other inputs are taken here, after the Schmid
-            // arithmetic: left alone, the compiler sinks their loads past the
-            // Newton loop's entry test and the wave waits on memory twice
+            for (int i = 0; i < 6; i++)
 #pragma unroll
-            for (int i = 0; i < 6; i++) keep_reg(V.bp[i]);
+                for (int j = 0; j < 6; j++) d[i] = fma(-S0[PK(i, j)], s[j], d[i]);
 #pragma unroll
-            for (int i = 0; i < 21; i++) keep_reg(V.S[i]);
+            for (int i = 0; i < 21; i++) K0[i] += S0[i];
+#pragma unroll
+            for (int i = 0; i < 6; i++) dl[i * NB_THREADS] = d[i];
+            rotation5(T9, Q);
 #pragma unroll
             for (int k = 0; k < EVPGPU_NSYSMX; k++) {
-                keep_reg(c1[k]);
-                if (!CSYM && RM != RM_DISL) keep_reg(c2[k]);
-            }
-            if (RM == RM_DISL) {
-                // crss holds the increment's constants: passing stress,
-                // 1/(tau_0 + tau_cut), gam_o, the first call's passing stress
-                in.tpn = crss + v;
-                in.tps = N;
-#pragma unroll
-                for (int s = 0; s < EVPGPU_NSYSMX; s++) in.itf[s] = s < ns ? c1[s] : 0.0;
-            } else {
-#pragma unroll
-            for (int s = 0; s < EVPGPU_NSYSMX; s++) {
-                if (s < ns) {
-                    in.itf[s] = 1.0 / c1[s];
-                    in.itb[s] = CSYM ? in.itf[s] : 1.0 / c2[s];
+                if (RM == RM_DISL) {
+                    it[k * NB_THREADS] = c1[k];
+                    it[(EVPGPU_NSYSMX + k) * NB_THREADS] = c2[k];
                 } else {
-                    in.itf[s] = in.itb[s] = 1.0;
+                    it[k * NB_THREADS] = rcp_refined(c1[k]);
+                    if (!CSYM) it[(EVPGPU_NSYSMX + k) * NB_THREADS] = rcp_refined(c2[k]);
                 }
             }
-            }
-            double s6[6], e6[6], gd[EVPGPU_NSYSMX], cs, ce;
-            int it, ntr;
-            int st = update_voxel<RM, FAST, NE>(P, p, in, V, s6, e6, gd, cs, ce, it, ntr);
-            if (st) {
-                atomicCAS(status, 0, st);
-            } else {
-                v6_to_sym(s6, t);
+        }
+        const double *g0c = crss + 2LL * EVPGPU_NSYSMX * N + v; // RM_DISL: gam_o
+        double *gd = gamdot + v;
+        const int ns = RM == RM_FAST || RM == RM_DISL ? EVPGPU_NSYSMX : P.nsys[p];
+        // The loops below are wave-uniform: a lane that has finished runs
+        // along with its state frozen (open false), which keeps the control
+        // flow scalar and the registers of the two loops disjoint.
+        bool open = mine, singular = false, uphill = false;
+        int iterl = 0, trials = 0;
+        {
+            double ed[5];
+            rates<RM, CSYM, GD, NE>(P, p, it, w, g0c, N, Q, s, ed, gd, open);
+            scaled_residual(P.dt, K0, dl, s, ed, r);
+            if (!FAST)
 #pragma unroll
-                for (int c = 0; c < 6; c++) sig[c * N + v] = t[c];
+                for (int i = 0; i < 5; i++) edl[i * NB_THREADS] = ed[i];
+        }
+        if (RM == RM_DISL && P.dd_first) {
+            // the first call used the previous call's mobile density; every
+            // later one sees the density that call formed
+#pragma unroll
+            for (int k = 0; k < EVPGPU_NSYSMX; k++) it[k * NB_THREADS] = crss[k * N + v];
+        }
+        double y2 = norm2(r);
+        bool moved = false; // the last step, accepted, ended the solve
+        for (;;) {
+            iterl += open;
+            if (FAST) {
+                const bool sk = open && y2 > 0.0 && y2 < P.kmin_tolx2;
+                trials += sk; // the reference's one rejected trial
+                open = open && !sk;
+                if (!__any(open)) break;
+            }
+            double step[6];
+            {
+                double K[21];
+                tangent(ns, p, w, Q, K0, K);
+#pragma unroll
+                for (int i = 0; i < 6; i++) step[i] = -r[i];
+                const bool pd = ldl6_solve(K, step);
+                singular = singular || (open && !pd);
+                // the slope of the merit function along the step is
+                // -scale |R|^2: zero only where the residual is
+                uphill = uphill || (open && pd && y2 == 0.0);
+                open = open && pd && y2 != 0.0;
+            }
+            // stpmax = 10 (src/evolution.c:166-170)
+            const double sum = norm2(step);
+            double scale = 1.0;
+            if (sum > 100.0) {
+                scale = 10.0 / sqrt(sum);
+#pragma unroll
+                for (int i = 0; i < 6; i++) step[i] *= scale;
+            }
+            // a trial is rejected (TOLX) when alam max|step_i|/max(|s_i|,1) < TOLX
+            auto rejected = [&](double alam) {
+                bool far = false;
+#pragma unroll
+                for (int i = 0; i < 6; i++)
+                    far = far || alam * fabs(step[i]) >= P.tolx * fmax(fabs(s[i]), 1.0);
+                return !far;
+            };
+            double alam = 1.0;
+            bool rej = rejected(alam);
+            // A rejected first trial leaves the step undone whatever its
+            // merit value; only gamdot (from the trial point) is affected,
+            // which FAST launches do not form, so they skip the evaluation.
+            if (FAST) {
+                trials += open && rej;
+                open = open && !rej;
+                if (!__any(open)) break;
+            }
+            double alam2 = 0.0, f2 = 0.0, sn[6], en[5], rn[6], y2n;
+            bool search = open;
+            for (;;) {
+#pragma unroll
+                for (int i = 0; i < 6; i++) sn[i] = fma(alam, step[i], s[i]);
+                // (a lane whose search is over repeats its last trial)
+                rates<RM, CSYM, GD, NE>(P, p, it, w, g0c, N, Q, sn, en, gd, search);
+                scaled_residual(P.dt, K0, dl, sn, en, rn);
+                trials += search;
+                y2n = norm2(rn);
+                // |C0 r|^2 lies between c0_lo2 |r|^2 and c0_hi2 |r|^2 (C0's
+                // extreme eigenvalues squared): where that decides the descent
+                // test, the merit functions are not formed
+                search = search && !rej && !(P.c0_hi2 * y2n <= 0.9997 * P.c0_lo2 * y2);
+                if (!__any(search)) break;
+                if (search) {
+                    const double fo = merit(r), fn = merit(rn), slope = -2.0 * scale * fo;
+                    search = !(fn <= fo + 1.E-4 * alam * slope);
+                    if (search) {
+                        const double next = ls_backtrack(alam, alam2, fn, f2, fo, slope);
+                        alam2 = alam;
+                        f2 = fn; // the backtrack value the cubic step needs (Q18)
+                        alam = next;
+                        rej = rejected(alam);
+                    }
+                }
+                if (!__any(search)) break;
+            }
+            open = open && !rej;
+            double cn = 0.0;
+#pragma unroll
+            for (int i = 0; i < 6; i++) cn = fma(sn[i] - s[i], sn[i] - s[i], cn);
+            // the relative step against the tolerance (|sn - s| / |lambda|)
+            if (open && (iterl >= 500 || !(cn > P.nr_tol * P.nr_tol * sn2))) {
+                // done: edot and err_e stay those of the iteration's start
+#pragma unroll
+                for (int i = 0; i < 6; i++) it[i * NB_THREADS] = sn[i];
+                moved = true;
+                open = false;
+            }
+            if (!__any(open)) break;
+            if (open) {
+#pragma unroll
+                for (int i = 0; i < 6; i++) {
+                    s[i] = sn[i];
+                    r[i] = rn[i];
+                    if (!FAST && i < 5) edl[i * NB_THREADS] = en[i];
+                }
+                y2 = y2n;
+            }
+        }
+        if (singular || uphill) atomicCAS(status, 0, singular ? EVPGPU_ERR_SINGULAR : EVPGPU_ERR_LINESEARCH);
+        if (mine && !singular && !uphill) {
+            double lam[6], t[6], so[6];
+#pragma unroll
+            for (int c = 0; c < 6; c++) t[c] = sig_in[c * N + v];
+            sym_to_v6(t, lam);
+            // the strain mismatch eps_p + dt edot + S s - E = r - S0 (s - lambda)
+            double ds[6], cs = 0.0;
+#pragma unroll
+            for (int i = 0; i < 6; i++) {
+                ds[i] = lam[i] - s[i];
+                so[i] = moved ? it[i * NB_THREADS] : s[i];
+            }
+            sym6_mul_add(fresh(params_at(offsetof(NewtonParams, s0p)), ds[0]), ds, r);
+#pragma unroll
+            for (int i = 0; i < 6; i++) cs = fma(so[i] - lam[i], so[i] - lam[i], cs);
+            v6_to_sym(so, t);
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                sig[c * N + v] = t[c];
+                red[(3 + c) * NB_THREADS] = t[c];
+                red[(9 + c) * NB_THREADS] = pl == 0 ? t[c] : 0.0;
+            }
+            red[0] = sqrt(cs);
+            red[NB_THREADS] = sqrt(norm2(r));
+            red[2 * NB_THREADS] = (double)iterl;
+            red[15 * NB_THREADS] = (double)trials;
+            if (!FAST) {
+                double e6[6];
+#pragma unroll
+                for (int i = 0; i < 6; i++) e6[i] = i < 5 ? edl[i * NB_THREADS] : 0.0;
                 v6_to_sym(e6, t);
 #pragma unroll
                 for (int c = 0; c < 6; c++) edot[c * N + v] = t[c];
-                if (!FAST)
-#pragma unroll
-                    for (int s = 0; s < EVPGPU_NSYSMX; s++)
-                        if (s < ns) gamdot[s * N + v] = gd[s];
-                r_cs = cs;
-                r_ce = ce;
-                r_it = (double)it;
-                r_tr = (double)ntr;
-                if (err_vox) {
-                    err_vox[2 * v] = cs;
-                    err_vox[2 * v + 1] = ce;
-                }
-                if (niter_vox) niter_vox[v] = it;
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NRED; i++) red[i * NB_THREADS] = 0.0;
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NRED; i++) red[i * NB_THREADS] = 0.0;
     }
-    double red[NRED];
-#pragma unroll
-    for (int i = 0; i < NRED; i++) red[i] = 0.0;
-    red[0] = r_cs;
-    red[1] = r_ce;
-    red[2] = r_it;
-    red[15] = r_tr;
-    if (v < N) {
-        if (gas_l) {
-#pragma unroll
-            for (int c = 0; c < 6; c++) {
-                sig[c * N + v] = 0.0;
-                edot[c * N + v] = 0.0;
-            }
-            if (err_vox) err_vox[2 * v] = err_vox[2 * v + 1] = 0.0;
-            if (niter_vox) niter_vox[v] = 0;
-        }
+    if (lead && gas_l && v0 < N) {
 #pragma unroll
         for (int c = 0; c < 6; c++) {
-            double sc = sig[c * N + v];
-            red[3 + c] = sc;
-            red[9 + c] = (phase[v] == 1) ? sc : 0.0;
+            sig[c * N + v] = 0.0;
+            if (!FAST) edot[c * N + v] = 0.0;
         }
     }
-    // Block partial sums, transposed through the slab (no longer needed):
-    // value i is summed by lanes 4i..4i+3 over 16 entries each, then across
-    // the four (a + b == b + a, so all four hold the same sum): a fixed order
-    // at a quarter of the instructions of 16 butterfly reductions.
-    static_assert(NB_THREADS == 64 && NRED * 4 == NB_THREADS && NRED * 65 <= EVPGPU_NSYSMX * 5 * NB_THREADS,
+    // Block partial sums: value i is summed by lanes 4i..4i+3 over 16 entries
+    // each (every value from its own start, so that the 64 lanes spread over
+    // the banks), then across the four (a + b == b + a, so all four hold the
+    // same sum): a fixed order at a quarter of the instructions of 16
+    // butterfly reductions.
+    static_assert(NB_THREADS == 64 && NRED * 4 == NB_THREADS && NRED <= 2 * EVPGPU_NSYSMX,
                   "one wave per block, 16 partial sums");
-    const int lane = threadIdx.x;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NRED; i++) slab[i * 65 + lane] = red[i];
     __syncthreads();
     const int vi = lane >> 2, q = lane & 3;
     double sum = 0.0;
 #pragma unroll
-    for (int j = 0; j < 16; j++) sum += slab[vi * 65 + q * 16 + j];
+    for (int j = 0; j < 16; j++) sum += slab[vi * NB_THREADS + q * 16 + ((j + vi) & 15)];
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);
     if (q == 0) partials[(long long)blockIdx.x * NRED + vi] = sum;
@@ -767,13 +763,8 @@ __global__ __launch_bounds__(256) void k_reduce_rows(const double *__restrict__ 
 
 } // namespace
 
-int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, double *sig, const double *E,
-                  const double *epsp, double *edot, const double *tran, const double *crss,
-                  double *gamdot, const int *phase, const int *orient, const double *sgr,
-                  long long n, double *partials, int *nblk_out, int *status, double *err_vox,
-                  int *niter_vox, int fast, hipEvent_t ev_start, hipEvent_t ev_stop)
+int newton_rate_mode(const NewtonParams &P)
 {
-    int nblk = (int)((n + NB_THREADS - 1) / NB_THREADS);
     // the integral-exponent variants need every crystal phase to have one;
     // the fast one also n <= 32, a full set of systems and one gam0
     bool intn = true, fastrm = true;
@@ -785,28 +776,38 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
             if (P.gam0[q][k] != P.gam0[q][0] || P.nrs[q][k] != P.nrs[q][0]) one = false;
         if (!one) fastrm = false;
     }
-    const int rm = !intn ? RM_POW : (fastrm ? RM_FAST : RM_LOOP);
+    return !intn ? RM_POW : (fastrm ? RM_FAST : RM_LOOP);
+}
+
+int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, double *sig, const double *E,
+                  const double *epsp, double *edot, const double *tran, const double *crss,
+                  double *gamdot, const int *phase, const int *orient, const double *sgr,
+                  long long n, double *partials, int *nblk_out, int *status, int fast, hipEvent_t ev_start,
+                  hipEvent_t ev_stop)
+{
+    const int nblk = (int)((n + NB_THREADS - 1) / NB_THREADS);
+    const int rm = newton_rate_mode(P);
     // the dislocation-density variant assumes 12 systems in every crystal phase
     if (P.dd)
         for (int q = 0; q < 2; q++)
             if (!P.is_gas[q] && P.nsys[q] != EVPGPU_NSYSMX) return EVPGPU_ERR_ARG;
-    // compile-time exponents for the common n = 10 and n = 20 (every crystal
-    // phase the same n, forward = backward CRSS)
-    int ne = 0;
-    if (rm == RM_FAST && P.crss_sym) {
-        int n0 = 0;
-        bool same = true;
-        for (int q = 0; q < 2; q++) {
-            if (P.is_gas[q]) continue;
-            if (n0 && P.int_n[q] != n0) same = false;
-            n0 = P.int_n[q];
-        }
-        if (same && (n0 == 10 || n0 == 20)) ne = n0;
-    }
-    // the events (when given) take the kernel's own start and end times: no
-    // marker packets between the launches
-#define NEWTON_ARGS dim3(nblk), dim3(NB_THREADS), 0, c->stream, ev_start, ev_stop, 0, P, n, phase, orient, sgr, \
-                    sig_in, sig, E, epsp, edot, tran, crss, gamdot, partials, status, err_vox, niter_vox
+    // One launch per crystal phase (two at most; nblk rows of partials each):
+    // the phase is then an argument, its constants scalar loads.  The first
+    // also clears the gas voxels; a grid of gas only takes one launch.
+    int crystal[2], nc = 0;
+    for (int q = 0; q < 2; q++)
+        if (!P.is_gas[q]) crystal[nc++] = q;
+    if (nc == 0) crystal[nc++] = 0;
+    for (int q = 0; q < nc; q++) {
+        const int p = crystal[q], lead = q == 0;
+        double *part = partials + (long long)q * nblk * NRED;
+        // compile-time exponents for the common n = 10 and n = 20
+        const int ne = rm == RM_FAST && P.crss_sym && (P.int_n[p] == 10 || P.int_n[p] == 20) ? P.int_n[p] : 0;
+        // the events (when given) take the kernel's own start and end times: no
+        // marker packets between the launches
+#define NEWTON_ARGS dim3(nblk), dim3(NB_THREADS), 0, c->stream, lead ? ev_start : nullptr,                  \
+                    q == nc - 1 ? ev_stop : nullptr, 0, P, n, p, lead, phase, orient, sgr, sig_in, sig, E, epsp, \
+                    edot, tran, crss, gamdot, part, status
 #define LAUNCH(A, B, F) hipExtLaunchKernelGGL((k_newton<A, B, F, 0>), NEWTON_ARGS)
 #define LAUNCH_NE(E, F) hipExtLaunchKernelGGL((k_newton<RM_FAST, true, F, E>), NEWTON_ARGS)
 #define LAUNCH_RM(B, F)                                                                  \
@@ -817,21 +818,22 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
         else if (rm == RM_LOOP) LAUNCH(RM_LOOP, B, F);                                   \
         else LAUNCH(RM_POW, B, F);                                                       \
     } while (0)
-    if (P.dd) {
-        if (fast) LAUNCH(RM_DISL, false, true);
-        else LAUNCH(RM_DISL, false, false);
-    } else if (fast) {
-        if (P.crss_sym) LAUNCH_RM(true, true);
-        else LAUNCH_RM(false, true);
-    } else {
-        if (P.crss_sym) LAUNCH_RM(true, false);
-        else LAUNCH_RM(false, false);
-    }
+        if (P.dd) {
+            if (fast) LAUNCH(RM_DISL, false, true);
+            else LAUNCH(RM_DISL, false, false);
+        } else if (fast) {
+            if (P.crss_sym) LAUNCH_RM(true, true);
+            else LAUNCH_RM(false, true);
+        } else {
+            if (P.crss_sym) LAUNCH_RM(true, false);
+            else LAUNCH_RM(false, false);
+        }
 #undef LAUNCH_RM
 #undef LAUNCH_NE
 #undef LAUNCH
 #undef NEWTON_ARGS
-    if (nblk_out) *nblk_out = nblk;
+    }
+    if (nblk_out) *nblk_out = nc * nblk;
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 

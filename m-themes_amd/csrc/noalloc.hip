@@ -1,7 +1,7 @@
 // noalloc.hip -- the per-voxel stress update on caller-owned device buffers
 // with no device allocation: evpgpu_newton_device_noalloc.
 //
-// It runs the kernel evpgpu_newton_host runs (k_newton, the full update of
+// It runs the kernel evpgpu_newton_host runs (k_newton_batch, the full update of
 // src/evolution.c:44-310 for a batch of voxels) on device pointers the
 // caller passes, for callers that cannot allocate (code under HIP graph
 // capture, tight serving loops).  The kernel's scratch -- NRED block partial
@@ -15,12 +15,10 @@
 
 namespace {
 
-// largest batch: 2^21 voxels (a 128^3 grid), 32768 blocks of 16 partials
+// largest batch: 2^21 voxels (a 128^3 grid)
 constexpr long long NOALLOC_MAX_N = EVPGPU_NOALLOC_MAX_VOXELS;
-constexpr long long NOALLOC_NBLK = NOALLOC_MAX_N / 64;
-// partial sums, then the status word (and its validation flag) in the last
-// 256-byte line
-constexpr long long SCRATCH_DOUBLES = NOALLOC_NBLK * NRED + 32;
+// the status word, in a 256-byte line of its own
+constexpr long long SCRATCH_DOUBLES = 32;
 
 static __device__ __align__(256) double scratch[SCRATCH_DOUBLES];
 
@@ -67,8 +65,7 @@ extern "C" int evpgpu_newton_device_noalloc(evpgpu_ctx *c, int n, const int *pha
     double *sp = nullptr;
     int st = scratch_ptr(&sp);
     if (st) return st;
-    double *partials = sp;
-    int *status = (int *)(sp + NOALLOC_NBLK * NRED);
+    int *status = (int *)sp;
     // the status word starts at zero on every call (a fill kernel, not a
     // memset node)
     st = fill_zero_int(c, status, 1);
@@ -82,11 +79,9 @@ extern "C" int evpgpu_newton_device_noalloc(evpgpu_ctx *c, int n, const int *pha
         return EVPGPU_ERR_HIP;
     if (*c->h_status) return *c->h_status;
     NewtonParams P = context_newton_params(c);
-    P.crss_sym = 0;
     P.dd = 0; // the power-law update on the caller's CRSS, as evpgpu_newton_host
-    int nb = 0;
-    st = newton_launch(c, P, sig6, sig6, strain6, eps6, edot6, tranmat9, crss24, gamdot12, phase, orient, sgr, n,
-                       partials, &nb, status, err2, niter, 0);
+    st = newton_batch_launch(c, P, sig6, sig6, strain6, eps6, edot6, tranmat9, crss24, gamdot12, phase, orient, sgr,
+                             n, status, err2, niter);
     if (st) return st;
     if (hipMemcpyAsync(c->h_status, status, sizeof(int), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
