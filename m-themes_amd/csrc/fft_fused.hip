@@ -333,6 +333,16 @@ template <typename R, int NX> constexpr int tbx()
                                                : 2;
 }
 
+// Where tiles of tbx() columns give fewer than TILE_FILL workgroups (two per
+// CU), the x-line kernel takes tiles of 4: the chip is then short of
+// workgroups and a pass is one tile's latency, which grows with its columns.
+// Measured, tbx() -> 4 columns, FP64 / FP32: 16^3 10.4 -> 9.4 / 9.8 -> 8.4 us,
+// 24^3 16.4 -> 10.1 / 14.3 -> 9.4, 32^3 17.8 -> 10.6 / 14.6 -> 9.7, 48^3
+// 19.3 -> 15.5 / 22.3 -> 13.4, 64^3 26.2 -> 20.6 / 23.9 -> 16.4 (2 and 1 columns no faster);
+// at 96^3 (588 tiles of 8) both take 37.0 in FP32, at 128^3 (1040 tiles of 8) 4
+// columns take 69.8 against 61.1.
+constexpr int TILE_FILL = 512;
+
 // plane (ny = nz) and line (nx) lengths of the fused kernels: powers of two
 // and the common mixed-radix lengths
 #define PLANE_DISPATCH(CALL)                                   \
@@ -405,15 +415,19 @@ int xg(evpgpu_ctx *c)
 {
     typedef typename CT<R>::T C;
     const GreenParams G = green_params(c);
-#define CALLL(NX_)                                                                                        \
-    {                                                                                                    \
-        constexpr int T = tbx<R, NX_>();                                                                 \
-        hipLaunchKernelGGL((k_x_green<R, NX_, T, GMODE>), dim3((c->ny * c->nzh + T - 1) / T), dim3(NTX), 0,  \
-                           c->stream, (C *)c->spec, c->acc, c->skA, G, c->ny, c->nz, c->nzh, c->NK,      \
-                           twp<R>(c, 0), c->skip);                                                       \
+    const int ncol = c->ny * c->nzh;
+#define XG(NX_, T_)                                                                                        \
+    hipLaunchKernelGGL((k_x_green<R, NX_, T_, GMODE>), dim3((ncol + T_ - 1) / T_), dim3(NTX), 0, c->stream, \
+                       (C *)c->spec, c->acc, c->skA, G, c->ny, c->nz, c->nzh, c->NK, twp<R>(c, 0), c->skip)
+#define CALLL(NX_)                                             \
+    {                                                          \
+        constexpr int T = tbx<R, NX_>(), S = T < 4 ? T : 4;    \
+        if (S < T && ncol < TILE_FILL * T) XG(NX_, S);         \
+        else XG(NX_, T);                                       \
     }
     LINE_DISPATCH(CALLL);
 #undef CALLL
+#undef XG
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 

@@ -49,7 +49,8 @@ static_assert(sizeof(LoopCtl) % sizeof(double) == 0 && sizeof(CtlConst) % sizeof
               "control blocks are whole doubles");
 static_assert(NL + NK <= 256, "one double per thread");
 
-// Stage 2 of the Newton partial sums (k_reduce_rows' order: thread t sums
+// Stage 2 of the Newton partial sums, or their only stage where the blocks
+// are few (k_reduce_rows' order: thread t sums
 // value t % 16 over the stage-1 rows t / 16, t / 16 + 16, ..., then the 16
 // row lanes of each value are summed in order), then the control step.  The
 // control block and the constants come in through LDS (one double per
@@ -142,11 +143,18 @@ int ctl_phase_launch(evpgpu_ctx *c, int limit, int conv, int first)
 
 int ctl_iter_launch(evpgpu_ctx *c, int nblk)
 {
-    int g = 0;
-    int st = reduce_stage1(c, c->partials, nblk, NRED, c->skip, &g);
-    if (st) return st;
+    // up to REDUCE_G rows of partials (32^3 voxels) are k_loop_ctl's own input:
+    // the first stage would only copy them (4.2 us of a 38 us iteration at
+    // 16^3); more rows than that one workgroup reads too slowly
+    int g = nblk;
+    const double *rows = c->partials;
+    if (nblk > REDUCE_G) {
+        int st = reduce_stage1(c, c->partials, nblk, NRED, c->skip, &g);
+        if (st) return st;
+        rows = c->red2;
+    }
     if (g < 1 || g > REDUCE_G) return EVPGPU_ERR_ARG; // k_loop_ctl loads at most REDUCE_G rows
-    hipLaunchKernelGGL(k_loop_ctl, dim3(1), dim3(256), 0, c->stream, (const double *)c->red2, g,
-                       (const int *)c->d_status, c->ctl, (const CtlConst *)c->ctl_k);
+    hipLaunchKernelGGL(k_loop_ctl, dim3(1), dim3(256), 0, c->stream, rows, g, (const int *)c->d_status, c->ctl,
+                       (const CtlConst *)c->ctl_k);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
