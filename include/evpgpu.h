@@ -151,12 +151,13 @@ int evpgpu_set_newton_tolerances(evpgpu_ctx *ctx, double tol, double tolx);
 int evpgpu_set_newton_shortcut(evpgpu_ctx *ctx, int on);
 /* Where ny = nz <= 128, a Green iteration's transforms run as three fused
  * passes (z+y plane R2C, x lines with the Green step, y+z plane C2R) instead
- * of seven; the results agree with the seven-pass path to rounding.  Off
- * forces the seven passes.  Default on. */
+ * of seven, and on other grids as five where nx has an x-line kernel; the
+ * results agree with the seven-pass path to rounding.  Off forces the seven
+ * passes.  Default on. */
 int evpgpu_set_fused_transforms(evpgpu_ctx *ctx, int on);
 /* The Green loop's control (get_smacro, the error norms and the loop test,
  * src/evolution.c:473-547,1354,1415-1458) runs on the device after every
- * iteration.  With the fused transforms the host queues the iterations in
+ * iteration.  The host queues the iterations in
  * batches of `batch` (1..4), two batches in flight, and reads the loop's
  * flags once per batch; the iterations queued past the loop's end do
  * nothing.  0 waits for every iteration.  Results are identical either way.

@@ -258,9 +258,8 @@ int green_iteration_queue(evpgpu_ctx *c, int prec, int refresh, const CtlConst &
 // One Green iteration, queued: prec FP64 runs the FFT/Green/C2R path in FP64
 // on sigma; MIXED runs it in FP32 on delta = sigma - sigma_A (anchor
 // refreshed first when refresh != 0).  The strain update adds the dD of the
-// last control step: read from the control block by the fused kernels, from
-// the host copy of it otherwise (the loop then waits for every iteration).
-// Ends with the loop control's step.
+// last control step, read from the control block.  Ends with the loop
+// control's step.
 int green_iteration(evpgpu_ctx *c, int prec, int refresh, const CtlConst &K)
 {
     // the timers record one Green iteration in timing_every
@@ -274,41 +273,24 @@ int green_iteration_queue(evpgpu_ctx *c, int prec, int refresh, const CtlConst &
 {
     const double scale = K.scale;
     int st = EVPGPU_OK;
-    const bool fused = c->fused && fused_ok(c);
+    // three passes where a (y, z) plane fits one workgroup; else the y and z
+    // passes around the x-line kernel where it has nx; else seven
+    const bool fused = c->fused && fused_ok(c), lines = c->fused && lines_ok(c);
     if (prec == EVPGPU_MIXED && refresh) {
         tmark(c, 5, 0);
         st = to_f32_launch(c, c->sig, c->sigA, 6 * c->N);
-        if (fused) {
-            if (!st) st = fused_anchor(c, c->sigA, c->cA, scale);
-        } else {
-            if (!st) st = fft_forward_anchor(c, c->sigA);
-            if (!st) st = green_anchor(c);
-            if (!st) st = fft_inverse_anchor(c, c->cA, scale);
-        }
+        if (!st) st = fused ? fused_anchor(c, c->sigA, c->cA, scale) : pass_anchor(c, c->sigA, c->cA, scale, lines);
         if (st) return st;
         tmark(c, 5, 1);
     }
-    if (fused) {
-        const double *addd = (const double *)((const char *)c->ctl + offsetof(LoopCtl, add));
-        st = prec == EVPGPU_MIXED ? fused_iteration_delta(c, c->sig, c->sigA, c->E, addd, c->cA, scale)
-                                  : fused_iteration_fp64(c, c->sig, c->E, addd, scale);
-        if (st) return st;
-    } else {
-    const double *add = c->h_ctl[0].add;
-    tmark(c, 1, 0);
-    st = prec == EVPGPU_MIXED ? fft_forward_delta(c, c->sig, c->sigA) : fft_forward(c, c->sig, 6, prec);
+    const double *addd = (const double *)((const char *)c->ctl + offsetof(LoopCtl, add));
+    if (prec == EVPGPU_MIXED)
+        st = fused ? fused_iteration_delta(c, c->sig, c->sigA, c->E, addd, c->cA, scale)
+                   : pass_iteration_delta(c, c->sig, c->sigA, c->E, addd, c->cA, scale, lines);
+    else
+        st = fused ? fused_iteration_fp64(c, c->sig, c->E, addd, scale)
+                   : pass_iteration_fp64(c, c->sig, c->E, addd, scale, lines);
     if (st) return st;
-    tmark(c, 1, 1);
-    tmark(c, 2, 0);
-    st = prec == EVPGPU_MIXED ? green_delta(c) : green_apply(c, prec, 1);
-    if (st) return st;
-    tmark(c, 2, 1);
-    tmark(c, 3, 0);
-    st = prec == EVPGPU_MIXED ? fft_inverse_delta(c, c->E, add, c->cA, scale)
-                              : fft_inverse_update(c, 6, prec, c->E, add, scale);
-    if (st) return st;
-    tmark(c, 3, 1);
-    }
     NewtonParams P = newton_params(c);
     P.dd_first = c->dd_first;
     P.skip = c->skip;
@@ -336,8 +318,7 @@ bool phase_ends(const LoopCtl &L, int limit, int conv)
 
 // One phase of the Green loop: iterations of one precision while
 // iter < limit (and, with conv, while the error norms exceed Err); first
-// runs at least one.  With the fused kernels and loop_batch > 0 the
-// iterations are queued in batches of loop_batch, two batches in flight: the
+// runs at least one.  With loop_batch > 0 the iterations are queued in batches of loop_batch, two batches in flight: the
 // host reads the older batch's flags while the device runs the newer one,
 // and the iterations queued past the end of the phase return at once.
 // Otherwise the host waits for every iteration.  On return the host copy of
@@ -347,7 +328,7 @@ int run_phase(evpgpu_ctx *c, int prec, int limit, int conv, int first, const Ctl
     int st = ctl_phase_launch(c, limit, conv, first);
     if (st) return st;
     if (!first && phase_ends(c->h_ctl[0], limit, conv)) return EVPGPU_OK;
-    const bool ahead = c->fused && fused_ok(c) && c->loop_batch > 0;
+    const bool ahead = c->loop_batch > 0;
     const int B = ahead ? c->loop_batch : 1, depth = ahead ? 2 : 1;
     const int ae = c->anchor_every > 0 ? c->anchor_every : 1;
     const int iter0 = c->h_ctl[0].f.iter;
@@ -1075,7 +1056,7 @@ int evpgpu_fft_c2r_host(evpgpu_ctx *c, const double *in, double *out)
         EVP_CHECK(hipMemcpy(c->spec, in, sizeof(double) * 2 * c->NK, hipMemcpyHostToDevice));
     }
     int st = fill_zero(c, c->rwork, c->N);
-    if (!st) st = fft_inverse_update(c, 1, c->precision, c->rwork, nullptr, 1.0);
+    if (!st) st = fft_inverse_update(c, 1, c->precision, c->rwork, 1.0);
     if (st) return st;
     EVP_CHECK(hipStreamSynchronize(c->stream));
     EVP_CHECK(hipMemcpy(out, c->rwork, sizeof(double) * c->N, hipMemcpyDeviceToHost));

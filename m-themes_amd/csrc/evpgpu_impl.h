@@ -216,15 +216,16 @@ void adjoint_free(evpgpu_ctx *c);
 // ---- launchers (defined in the .hip files) ----
 // fft.hip
 int fft_forward(evpgpu_ctx *c, const double *real_in, int ncomp, int precision);
-int fft_inverse_update(evpgpu_ctx *c, int ncomp, int precision, double *target,
-                       const double *add_const, double scale);
+int fft_inverse_update(evpgpu_ctx *c, int ncomp, int precision, double *target, double scale);
 int fft_inverse_real(evpgpu_ctx *c, const double2 *cin, int ncomp, double *out, double scale);
 int fft_twiddles(evpgpu_ctx *c);
 int fft_forward_to(evpgpu_ctx *c, const double *real_in, int ncomp, double2 *dst);
-int fft_forward_delta(evpgpu_ctx *c, const double *sig, const float *anchor);
-int fft_forward_anchor(evpgpu_ctx *c, const float *anchor);
-int fft_inverse_delta(evpgpu_ctx *c, double *E, const double *add, const float *cA, double scale);
-int fft_inverse_anchor(evpgpu_ctx *c, float *cA, double scale);
+// one iteration's transforms and Green step (add: 6 values in device memory);
+// lines: the x passes and the Green step in the x-line kernel (lines_ok)
+int pass_iteration_fp64(evpgpu_ctx *c, const double *sig, double *E, const double *add, double scale, bool lines);
+int pass_iteration_delta(evpgpu_ctx *c, const double *sig, const float *sigA, double *E, const double *add,
+                         const float *cA, double scale, bool lines);
+int pass_anchor(evpgpu_ctx *c, const float *sigA, float *cA, double scale, bool lines);
 int fft_inverse_set(evpgpu_ctx *c, double *target, const double *base, double scale);
 // green.hip
 int green_apply(evpgpu_ctx *c, int precision, int accumulate);
@@ -241,7 +242,11 @@ void tcollect_slot(evpgpu_ctx *c, int slot, int keep);
 // its own start and end (hipExtLaunchKernelGGL), or nulls when not timing
 void tkernel(evpgpu_ctx *c, int k, hipEvent_t *start, hipEvent_t *stop);
 
+bool lines_ok(const evpgpu_ctx *c);
 bool fused_ok(const evpgpu_ctx *c);
+int x_green_fp64(evpgpu_ctx *c);
+int x_green_delta(evpgpu_ctx *c);
+int x_green_anchor(evpgpu_ctx *c);
 // the Green operator's parameters from the context's loading
 GreenParams green_params(const evpgpu_ctx *c);
 int fused_iteration_fp64(evpgpu_ctx *c, const double *sig, double *E, const double *add, double scale);

@@ -99,10 +99,12 @@ __device__ __forceinline__ int xcd_tile(int b, int nb)
 template <typename R, int L, bool INV>
 __global__ __launch_bounds__(NT) void k_fft_strided(typename CT<R>::T *data, int ninner, int nbx,
                                                     long long es, int O2, long long S1,
-                                                    long long S2, const typename CT<R>::T *tw)
+                                                    long long S2, const typename CT<R>::T *tw,
+                                                    const int *skip)
 {
     typedef typename CT<R>::T C;
     constexpr int P = L + 1;
+    if (skip && *skip) return;
     __shared__ C lds[TB * P];
     // the twiddle table in LDS, loaded with the tile (from memory, every
     // stage waited on its twiddles)
@@ -139,10 +141,12 @@ __global__ __launch_bounds__(NT) void k_fft_strided(typename CT<R>::T *data, int
 template <typename R, int L, int IN>
 __global__ __launch_bounds__(NT) void k_fft_z_r2c(const double *in, const float *inA,
                                                   typename CT<R>::T *out, long long N,
-                                                  long long NK, const typename CT<R>::T *tw)
+                                                  long long NK, const typename CT<R>::T *tw,
+                                                  const int *skip)
 {
     typedef typename CT<R>::T C;
     constexpr int M = L / 2, P = M + 1;
+    if (skip && *skip) return;
     __shared__ C lds[TB * P];
     __shared__ C s_tw[L]; // the twiddle table, loaded with the lines
     for (int i = threadIdx.x; i < L; i += NT) s_tw[i] = tw[i];
@@ -189,15 +193,17 @@ __global__ __launch_bounds__(NT) void k_fft_z_r2c(const double *in, const float 
 // MODE 2: target[c] += add[c] + fa[c] + re*scale   (mixed loop: anchor + delta)
 // MODE 3: fo[c]      = (float)(re*scale)           (mixed loop: anchor update)
 // MODE 4: target[c]  = base[c] + re*scale          (projection of a strain change)
+// add[c]: six values in device memory (null: zeros)
 template <typename R, int L, int MODE>
 __global__ __launch_bounds__(NT) void k_fft_z_c2r(const typename CT<R>::T *in, double *target,
                                                   const float *fa, float *fo, const double *base,
-                                                  long long N, long long NK, double a0, double a1,
-                                                  double a2, double a3, double a4, double a5,
-                                                  double scale, const typename CT<R>::T *tw)
+                                                  long long N, long long NK, const double *addd,
+                                                  double scale, const typename CT<R>::T *tw,
+                                                  const int *skip)
 {
     typedef typename CT<R>::T C;
     constexpr int M = L / 2, P = M + 1;
+    if (skip && *skip) return;
     __shared__ C lds[TB * P];
     __shared__ C s_tw[L]; // the twiddle table, loaded with the lines
     for (int i = threadIdx.x; i < L; i += NT) s_tw[i] = tw[i];
@@ -211,7 +217,7 @@ __global__ __launch_bounds__(NT) void k_fft_z_c2r(const typename CT<R>::T *in, d
         split_inverse<R, M>(lds + (i / (M / 2 + 1)) * P, i % (M / 2 + 1), (const C *)s_tw);
     __syncthreads();
     gstages<true, M, 0, 1, TB, P, 1, 0, NT, 2>(lds, (const C *)s_tw);
-    const double add = comp == 0 ? a0 : comp == 1 ? a1 : comp == 2 ? a2 : comp == 3 ? a3 : comp == 4 ? a4 : a5;
+    const double add = addd ? addd[comp] : 0.0;
     const long long off = comp * N + line0 * L;
     for (int e = threadIdx.x; e < M * TB; e += NT) {
         const int t = e / M, n = e % M;
@@ -315,9 +321,10 @@ __device__ __forceinline__ void dft2_lines(const C *a, C *b, const C *tw, int L,
 template <typename R, bool INV>
 __global__ __launch_bounds__(NT) void k_dft_strided(typename CT<R>::T *data, int L, int ninner, int nbx,
                                                     long long es, int O2, long long S1, long long S2,
-                                                    const typename CT<R>::T *tw)
+                                                    const typename CT<R>::T *tw, const int *skip)
 {
     typedef typename CT<R>::T C;
+    if (skip && *skip) return;
     extern __shared__ unsigned char dft_smem[];
     const int TBL = dft_lines(L);
     C *a = reinterpret_cast<C *>(dft_smem), *b = a + TBL * L, *tws = b + TBL * L;
@@ -339,9 +346,10 @@ __global__ __launch_bounds__(NT) void k_dft_strided(typename CT<R>::T *data, int
 template <typename R, int IN>
 __global__ __launch_bounds__(NT) void k_dft_z_r2c(const double *in, const float *inA, typename CT<R>::T *out,
                                                   int L, long long nlines, long long N, long long NK,
-                                                  const typename CT<R>::T *tw)
+                                                  const typename CT<R>::T *tw, const int *skip)
 {
     typedef typename CT<R>::T C;
+    if (skip && *skip) return;
     extern __shared__ unsigned char dft_smem[];
     const int TBL = dft_lines(L), P = L / 2 + 1;
     C *a = reinterpret_cast<C *>(dft_smem), *b = a + TBL * L, *tws = b + TBL * L;
@@ -369,11 +377,11 @@ __global__ __launch_bounds__(NT) void k_dft_z_r2c(const double *in, const float 
 template <typename R, int MODE>
 __global__ __launch_bounds__(NT) void k_dft_z_c2r(const typename CT<R>::T *in, double *target, const float *fa,
                                                   float *fo, const double *base, int L, long long nlines,
-                                                  long long N, long long NK, double a0, double a1, double a2,
-                                                  double a3, double a4, double a5, double scale,
-                                                  const typename CT<R>::T *tw)
+                                                  long long N, long long NK, const double *addd, double scale,
+                                                  const typename CT<R>::T *tw, const int *skip)
 {
     typedef typename CT<R>::T C;
+    if (skip && *skip) return;
     extern __shared__ unsigned char dft_smem[];
     const int TBL = dft_lines(L), P = L / 2 + 1;
     C *a = reinterpret_cast<C *>(dft_smem), *b = a + TBL * L, *tws = b + TBL * L;
@@ -396,7 +404,7 @@ __global__ __launch_bounds__(NT) void k_dft_z_c2r(const typename CT<R>::T *in, d
         a[e] = v;
     }
     __syncthreads();
-    const double add = comp == 0 ? a0 : comp == 1 ? a1 : comp == 2 ? a2 : comp == 3 ? a3 : comp == 4 ? a4 : a5;
+    const double add = addd ? addd[comp] : 0.0;
     const long long off = comp * N + line0 * L;
     dft2_lines<true>(a, b, tws, L, TBL, nt, L, [&](int t, int n, C z) {
         const long long i = off + (long long)t * L + n;
@@ -460,13 +468,13 @@ int pass_y(evpgpu_ctx *c, typename CT<R>::T *d, int ncomp)
         const int L = c->ny, tbl = dft_lines(L), nbx = (c->nzh + tbl - 1) / tbl;
         hipLaunchKernelGGL((k_dft_strided<R, INV>), dim3(nbx * ncomp * c->nx), dim3(NT),
                            sizeof(typename CT<R>::T) * (2 * tbl + 1) * L, c->stream, d, L, c->nzh, nbx, (long long)c->nzh, 1,
-                           (long long)c->ny * c->nzh, 0LL, twp<R>(c, 1));
+                           (long long)c->ny * c->nzh, 0LL, twp<R>(c, 1), c->skip);
         return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
     }
     const int nbx = (c->nzh + TB - 1) / TB;
     dim3 g(nbx * ncomp * c->nx);
 #define CALLY(L) hipLaunchKernelGGL((k_fft_strided<R, L, INV>), g, dim3(NT), 0, c->stream, d, c->nzh, nbx, \
-                                    (long long)c->nzh, 1, (long long)c->ny * c->nzh, 0LL, twp<R>(c, 1))
+                                    (long long)c->nzh, 1, (long long)c->ny * c->nzh, 0LL, twp<R>(c, 1), c->skip)
     FFT_DISPATCH(c->ny, CALLY);
 #undef CALLY
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
@@ -479,21 +487,22 @@ int pass_x(evpgpu_ctx *c, typename CT<R>::T *d, int ncomp)
         const int L = c->nx, tbl = dft_lines(L), nbx = (c->nzh + tbl - 1) / tbl;
         hipLaunchKernelGGL((k_dft_strided<R, INV>), dim3(nbx * ncomp * c->ny), dim3(NT),
                            sizeof(typename CT<R>::T) * (2 * tbl + 1) * L, c->stream, d, L, c->nzh, nbx,
-                           (long long)c->ny * c->nzh, c->ny, (long long)c->NK, (long long)c->nzh, twp<R>(c, 0));
+                           (long long)c->ny * c->nzh, c->ny, (long long)c->NK, (long long)c->nzh, twp<R>(c, 0),
+                           c->skip);
         return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
     }
     const int nbx = (c->nzh + TB - 1) / TB;
     dim3 g(nbx * ncomp * c->ny);
 #define CALLX(L) hipLaunchKernelGGL((k_fft_strided<R, L, INV>), g, dim3(NT), 0, c->stream, d, c->nzh, nbx, \
                                     (long long)c->ny * c->nzh, c->ny, (long long)c->NK,                 \
-                                    (long long)c->nzh, twp<R>(c, 0))
+                                    (long long)c->nzh, twp<R>(c, 0), c->skip)
     FFT_DISPATCH(c->nx, CALLX);
 #undef CALLX
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
 template <typename R, int IN>
-int fwd(evpgpu_ctx *c, const double *real_in, const float *inA, int ncomp, typename CT<R>::T *spec)
+int fwd_zy(evpgpu_ctx *c, const double *real_in, const float *inA, int ncomp, typename CT<R>::T *spec)
 {
     // the Stockham z kernels take whole groups of TB lines
     if (!is_stockham_len(c->nz) || (c->nx * c->ny) % TB != 0) {
@@ -501,46 +510,53 @@ int fwd(evpgpu_ctx *c, const double *real_in, const float *inA, int ncomp, typen
         const long long nl = (long long)c->nx * c->ny;
         hipLaunchKernelGGL((k_dft_z_r2c<R, IN>), dim3((unsigned)((nl + tbl - 1) / tbl), ncomp), dim3(NT),
                            sizeof(typename CT<R>::T) * (2 * tbl + 1) * L, c->stream, real_in, inA, spec, L, nl, c->N,
-                           c->NK, twp<R>(c, 2));
+                           c->NK, twp<R>(c, 2), c->skip);
         if (hipGetLastError() != hipSuccess) return EVPGPU_ERR_HIP;
     } else {
     dim3 g((unsigned)(c->nx * c->ny / TB), ncomp);
 #define CALLZ(L) hipLaunchKernelGGL((k_fft_z_r2c<R, L, IN>), g, dim3(NT), 0, c->stream, real_in, inA, \
-                                    spec, c->N, c->NK, twp<R>(c, 2))
+                                    spec, c->N, c->NK, twp<R>(c, 2), c->skip)
     FFT_DISPATCH(c->nz, CALLZ);
 #undef CALLZ
     }
-    int st = pass_y<R, false>(c, spec, ncomp);
-    if (st) return st;
-    return pass_x<R, false>(c, spec, ncomp);
+    return pass_y<R, false>(c, spec, ncomp);
+}
+
+template <typename R, int IN>
+int fwd(evpgpu_ctx *c, const double *real_in, const float *inA, int ncomp, typename CT<R>::T *spec)
+{
+    int st = fwd_zy<R, IN>(c, real_in, inA, ncomp, spec);
+    return st ? st : pass_x<R, false>(c, spec, ncomp);
 }
 
 template <typename R, int MODE>
-int inv(evpgpu_ctx *c, typename CT<R>::T *spec, int ncomp, double *target, const double *addc,
-        double scale, const float *fa = nullptr, float *fo = nullptr, const double *base = nullptr)
+int inv_yz(evpgpu_ctx *c, typename CT<R>::T *spec, int ncomp, double *target, const double *addd,
+           double scale, const float *fa = nullptr, float *fo = nullptr, const double *base = nullptr)
 {
-    int st = pass_x<R, true>(c, spec, ncomp);
+    int st = pass_y<R, true>(c, spec, ncomp);
     if (st) return st;
-    st = pass_y<R, true>(c, spec, ncomp);
-    if (st) return st;
-    double a[6] = {0, 0, 0, 0, 0, 0};
-    if (addc)
-        for (int i = 0; i < ncomp && i < 6; i++) a[i] = addc[i];
     if (!is_stockham_len(c->nz) || (c->nx * c->ny) % TB != 0) {
         const int L = c->nz, tbl = dft_lines(L);
         const long long nl = (long long)c->nx * c->ny;
         hipLaunchKernelGGL((k_dft_z_c2r<R, MODE>), dim3((unsigned)((nl + tbl - 1) / tbl), ncomp), dim3(NT),
                            sizeof(typename CT<R>::T) * (2 * tbl + 1) * L, c->stream, spec, target, fa, fo, base,
-                           L, nl, c->N, c->NK, a[0], a[1], a[2], a[3], a[4], a[5], scale, twp<R>(c, 2));
+                           L, nl, c->N, c->NK, addd, scale, twp<R>(c, 2), c->skip);
         return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
     }
     dim3 g((unsigned)(c->nx * c->ny / TB), ncomp);
 #define CALLZI(L) hipLaunchKernelGGL((k_fft_z_c2r<R, L, MODE>), g, dim3(NT), 0, c->stream, spec, target, \
-                                     fa, fo, base, c->N, c->NK, a[0], a[1], a[2], a[3], a[4], a[5],   \
-                                     scale, twp<R>(c, 2))
+                                     fa, fo, base, c->N, c->NK, addd, scale, twp<R>(c, 2), c->skip)
     FFT_DISPATCH(c->nz, CALLZI);
 #undef CALLZI
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
+}
+
+template <typename R, int MODE>
+int inv(evpgpu_ctx *c, typename CT<R>::T *spec, int ncomp, double *target, const double *addd,
+        double scale, const float *fa = nullptr, float *fo = nullptr, const double *base = nullptr)
+{
+    int st = pass_x<R, true>(c, spec, ncomp);
+    return st ? st : inv_yz<R, MODE>(c, spec, ncomp, target, addd, scale, fa, fo, base);
 }
 
 } // namespace
@@ -579,34 +595,63 @@ int fft_forward(evpgpu_ctx *c, const double *real_in, int ncomp, int precision)
     return fwd<double, 0>(c, real_in, nullptr, ncomp, (double2 *)c->spec);
 }
 
-// mixed loop: FP32 transform of (sig - anchor), anchor stored in FP32
 // FP64 R2C of ncomp real fields into a caller-chosen spectrum buffer
 int fft_forward_to(evpgpu_ctx *c, const double *real_in, int ncomp, double2 *dst)
 {
     return fwd<double, 0>(c, real_in, nullptr, ncomp, dst);
 }
 
-int fft_forward_delta(evpgpu_ctx *c, const double *sig, const float *anchor)
+// One Green iteration's transforms for grids that do not take the fused
+// planes (fft_fused.hip).  Where the x-line kernel has nx (lines), it does the
+// forward and inverse x transforms and the Green step in one pass over the
+// spectrum: five passes instead of seven (144 x 160 x 160 FP64: the two x
+// passes and the Green pass, 243 us, become one of 170 us).
+int pass_iteration_fp64(evpgpu_ctx *c, const double *sig, double *E, const double *add, double scale, bool lines)
 {
-    return fwd<float, 1>(c, sig, anchor, 6, (float2 *)c->spec);
+    double2 *spec = (double2 *)c->spec;
+    tmark(c, 1, 0);
+    int st = lines ? fwd_zy<double, 0>(c, sig, nullptr, 6, spec) : fwd<double, 0>(c, sig, nullptr, 6, spec);
+    tmark(c, 1, 1);
+    tmark(c, 2, 0);
+    if (!st) st = lines ? x_green_fp64(c) : green_apply(c, EVPGPU_FP64, 1);
+    tmark(c, 2, 1);
+    tmark(c, 3, 0);
+    if (!st)
+        st = lines ? inv_yz<double, 0>(c, spec, 6, E, add, scale) : inv<double, 0>(c, spec, 6, E, add, scale);
+    tmark(c, 3, 1);
+    return st;
 }
 
-// mixed loop: FP64 transform of the FP32 anchor field
-int fft_forward_anchor(evpgpu_ctx *c, const float *anchor)
+// mixed loop: FP32 transform of (sig - anchor), anchor stored in FP32;
+// E += add + cA + re/N
+int pass_iteration_delta(evpgpu_ctx *c, const double *sig, const float *sigA, double *E, const double *add,
+                         const float *cA, double scale, bool lines)
 {
-    return fwd<double, 2>(c, nullptr, anchor, 6, (double2 *)c->spec);
+    float2 *spec = (float2 *)c->spec;
+    tmark(c, 1, 0);
+    int st = lines ? fwd_zy<float, 1>(c, sig, sigA, 6, spec) : fwd<float, 1>(c, sig, sigA, 6, spec);
+    tmark(c, 1, 1);
+    tmark(c, 2, 0);
+    if (!st) st = lines ? x_green_delta(c) : green_delta(c);
+    tmark(c, 2, 1);
+    tmark(c, 3, 0);
+    if (!st)
+        st = lines ? inv_yz<float, 2>(c, spec, 6, E, add, scale, cA) : inv<float, 2>(c, spec, 6, E, add, scale, cA);
+    tmark(c, 3, 1);
+    return st;
 }
 
-// mixed loop: E += add + cA + re/N from the FP32 delta spectrum
-int fft_inverse_delta(evpgpu_ctx *c, double *E, const double *add, const float *cA, double scale)
+// mixed loop, anchor (FP64 transform of the FP32 anchor field): skA =
+// antisym(Gamma sigma_A) ; cA = re/N
+int pass_anchor(evpgpu_ctx *c, const float *sigA, float *cA, double scale, bool lines)
 {
-    return inv<float, 2>(c, (float2 *)c->spec, 6, E, add, scale, cA, nullptr, nullptr);
-}
-
-// mixed loop: cA = re/N of the FP64 anchor spectrum
-int fft_inverse_anchor(evpgpu_ctx *c, float *cA, double scale)
-{
-    return inv<double, 3>(c, (double2 *)c->spec, 6, nullptr, nullptr, scale, nullptr, cA, nullptr);
+    double2 *spec = (double2 *)c->spec;
+    int st = lines ? fwd_zy<double, 2>(c, nullptr, sigA, 6, spec) : fwd<double, 2>(c, nullptr, sigA, 6, spec);
+    if (!st) st = lines ? x_green_anchor(c) : green_anchor(c);
+    if (!st)
+        st = lines ? inv_yz<double, 3>(c, spec, 6, nullptr, nullptr, scale, nullptr, cA)
+                   : inv<double, 3>(c, spec, 6, nullptr, nullptr, scale, nullptr, cA);
+    return st;
 }
 
 // target = base + re*scale of the FP64 spectrum (6 comps)
@@ -615,13 +660,12 @@ int fft_inverse_set(evpgpu_ctx *c, double *target, const double *base, double sc
     return inv<double, 4>(c, (double2 *)c->spec, 6, target, nullptr, scale, nullptr, nullptr, base);
 }
 
-// inverse of c->spec (ncomp comps) accumulated into target: t += add[c] + re*scale
-int fft_inverse_update(evpgpu_ctx *c, int ncomp, int precision, double *target,
-                       const double *add_const, double scale)
+// inverse of c->spec (ncomp comps) accumulated into target: t += re*scale
+int fft_inverse_update(evpgpu_ctx *c, int ncomp, int precision, double *target, double scale)
 {
     if (precision == EVPGPU_MIXED)
-        return inv<float, 0>(c, (float2 *)c->spec, ncomp, target, add_const, scale);
-    return inv<double, 0>(c, (double2 *)c->spec, ncomp, target, add_const, scale);
+        return inv<float, 0>(c, (float2 *)c->spec, ncomp, target, nullptr, scale);
+    return inv<double, 0>(c, (double2 *)c->spec, ncomp, target, nullptr, scale);
 }
 
 // inverse of an FP64 spectrum (destroyed) into out = re*scale

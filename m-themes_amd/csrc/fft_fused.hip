@@ -109,13 +109,12 @@ __global__ __launch_bounds__(NTH) void k_zy_r2c(const double *__restrict__ in, c
 
 // MODE 0: target += add + re*scale; 1: target = re*scale; 2: target += add +
 // fa + re*scale; 3: fo = (float)(re*scale); 4: target = base + re*scale.
-// add is addd[comp] when addd is given (device memory), else a0..a5.
+// add is addd[comp] (six values in device memory; null: zero).
 template <typename R, int NY, int NZ, int MODE>
 __global__ __launch_bounds__(NTH) void k_yz_c2r(const typename CT<R>::T *__restrict__ in, double *target,
                                                 const float *__restrict__ fa, float *__restrict__ fo,
                                                 const double *__restrict__ basef, long long N, long long NK,
-                                                double a0, double a1, double a2, double a3, double a4,
-                                                double a5, const double *__restrict__ addd, double scale,
+                                                const double *__restrict__ addd, double scale,
                                                 const typename CT<R>::T *__restrict__ twy,
                                                 const typename CT<R>::T *__restrict__ twz,
                                                 const int *__restrict__ skip)
@@ -159,8 +158,7 @@ __global__ __launch_bounds__(NTH) void k_yz_c2r(const typename CT<R>::T *__restr
     }
     __syncthreads();
     gstages<true, M, 0, 1, NY, P, 1, 0, NTH, 2>(lds, (const C *)s_twz);
-    const double add = addd ? addd[comp]
-                            : comp == 0 ? a0 : comp == 1 ? a1 : comp == 2 ? a2 : comp == 3 ? a3 : comp == 4 ? a4 : a5;
+    const double add = addd ? addd[comp] : 0.0;
     const long long base = comp * N + (long long)x * NY * NZ;
     // (loading the read-modify-write operands of all the thread's elements
     // before the first wait was measured slower here: 70 us against 63 us)
@@ -223,15 +221,15 @@ __global__ __launch_bounds__(NTX) void k_x_green(typename CT<R>::T *__restrict__
     // Line (c, j) = component c, column q0 + j; element x at spec[c*NK + x*ncol + q0 + j].
     const int ncol = ny * nzh;
     // Workgroups go to the 8 XCDs round robin (block b to XCD b mod 8), and
-    // each XCD has its own L2.  A tile row is 64 B when TBX complex values
-    // fill half a 128-byte line, so the two tiles that share the lines are
-    // given to blocks b and b + 8 (the same XCD, dispatched together):
-    // within each group of 16 blocks, block g*16 + r takes tile
-    // g*16 + 2 (r mod 8) + r / 8.
+    // each XCD has its own L2.  The SH tiles that share the 128-byte lines of
+    // a row (2 where TBX complex values fill half a line) are given to blocks
+    // b, b + 8, .. (the same XCD, dispatched together): within each group of
+    // 8 SH blocks, block r takes tile SH (r mod 8) + r / 8.
+    constexpr int SH = TBX * (int)sizeof(C) < 128 ? 128 / (TBX * (int)sizeof(C)) : 1;
     int tile = blockIdx.x;
-    if (blockIdx.x < gridDim.x / 16 * 16) {
-        const int g = blockIdx.x / 16, r = blockIdx.x % 16;
-        tile = g * 16 + (r % 8) * 2 + r / 8;
+    if (blockIdx.x < gridDim.x / (8 * SH) * (8 * SH)) {
+        const int g = blockIdx.x / (8 * SH), r = blockIdx.x % (8 * SH);
+        tile = g * 8 * SH + (r % 8) * SH + r / 8;
     }
     const int q0 = tile * TBX;
     const int nk = min(TBX, ncol - q0);
@@ -323,10 +321,12 @@ template <> const float2 *twp<float>(evpgpu_ctx *c, int axis) { return c->tw32[a
 // lines per x-green workgroup: 6 components x TBX lines x px() in LDS,
 // sized so that three workgroups share a CU's LDS (their load, transform and
 // Green phases then overlap)
+// (FP64 lines longer than 128: two, which is what its registers allow anyway;
+// a tile of 2 columns would use 32 of the 128 bytes of a line)
 template <typename R, int NX> constexpr int tbx()
 {
     constexpr int cs = (int)sizeof(typename CT<R>::T);
-    constexpr int cap = LDS_MAX / 3 - 1024 - NX * cs; // less the twiddle table
+    constexpr int cap = LDS_MAX / (sizeof(R) == 8 && NX > 128 ? 2 : 3) - 1024 - NX * cs; // less the twiddle table
     return 6 * 16 * px<R>(NX, 16) * cs <= cap  ? 16
            : 6 * 8 * px<R>(NX, 8) * cs <= cap  ? 8
            : 6 * 4 * px<R>(NX, 4) * cs <= cap  ? 4
@@ -360,18 +360,30 @@ constexpr int TILE_FILL = 512;
     default: return EVPGPU_ERR_SIZE;                           \
     }
 
+// x-line lengths: the Stockham lengths of fft.hip
 #define LINE_DISPATCH(CALL)             \
     switch (c->nx) {                    \
     case 8: CALL(8); break;             \
+    case 12: CALL(12); break;           \
     case 16: CALL(16); break;           \
+    case 20: CALL(20); break;           \
     case 24: CALL(24); break;           \
     case 32: CALL(32); break;           \
+    case 36: CALL(36); break;           \
+    case 40: CALL(40); break;           \
     case 48: CALL(48); break;           \
+    case 60: CALL(60); break;           \
     case 64: CALL(64); break;           \
+    case 72: CALL(72); break;           \
+    case 80: CALL(80); break;           \
     case 96: CALL(96); break;           \
+    case 100: CALL(100); break;         \
     case 120: CALL(120); break;         \
     case 128: CALL(128); break;         \
+    case 144: CALL(144); break;         \
+    case 160: CALL(160); break;         \
     case 192: CALL(192); break;         \
+    case 200: CALL(200); break;         \
     case 240: CALL(240); break;         \
     case 256: CALL(256); break;         \
     default: return EVPGPU_ERR_SIZE;    \
@@ -390,21 +402,16 @@ int zy(evpgpu_ctx *c, const double *in, const float *inA)
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
-// addc: host values of the constant added per component (or null: none);
-// addd: the same in device memory (read by the kernel, overrides addc)
+// addd: the constant added per component, in device memory (or null: none)
 template <typename R, int MODE>
-int yz(evpgpu_ctx *c, double *target, const double *addc, double scale, const float *fa, float *fo,
-       const double *basef, const double *addd = nullptr)
+int yz(evpgpu_ctx *c, double *target, double scale, const float *fa, float *fo, const double *addd = nullptr)
 {
     typedef typename CT<R>::T C;
     const C *spec = (const C *)c->spec;
-    double a[6] = {0, 0, 0, 0, 0, 0};
-    if (addc)
-        for (int i = 0; i < 6; i++) a[i] = addc[i];
 #define CALLP(NY_, NZ_)                                                                                    \
     hipLaunchKernelGGL((k_yz_c2r<R, NY_, NZ_, MODE>), dim3(c->nx, 6), dim3(NTH), 0, c->stream, spec, target, \
-                       fa, fo, basef, c->N, c->NK, a[0], a[1], a[2], a[3], a[4], a[5], addd, scale,          \
-                       twp<R>(c, 1), twp<R>(c, 2), c->skip)
+                       fa, fo, (const double *)nullptr, c->N, c->NK, addd, scale, twp<R>(c, 1), twp<R>(c, 2), \
+                       c->skip)
     PLANE_DISPATCH(CALLP);
 #undef CALLP
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
@@ -433,17 +440,31 @@ int xg(evpgpu_ctx *c)
 
 } // namespace
 
+// the lengths nx of LINE_DISPATCH
+bool lines_ok(const evpgpu_ctx *c)
+{
+    static const int lines[] = {8,  12, 16, 20, 24,  32,  36,  40,  48,  60,  64, 72,
+                                80, 96, 100, 120, 128, 144, 160, 192, 200, 240, 256};
+    for (int n : lines)
+        if (c->nx == n) return true;
+    return false;
+}
+
 // the fused path covers the plane lengths ny = nz of PLANE_DISPATCH (<= 128:
-// the plane fits in LDS in FP64) and the line lengths nx of LINE_DISPATCH
+// the plane fits in LDS in FP64) and the line lengths
 bool fused_ok(const evpgpu_ctx *c)
 {
     static const int planes[] = {8, 16, 24, 32, 48, 64, 96, 120, 128};
-    static const int lines[] = {8, 16, 24, 32, 48, 64, 96, 120, 128, 192, 240, 256};
-    bool p = false, l = false;
-    for (int n : planes) p = p || (c->ny == n && c->nz == n);
-    for (int n : lines) l = l || c->nx == n;
-    return p && l;
+    for (int n : planes)
+        if (c->ny == n && c->nz == n) return lines_ok(c);
+    return false;
 }
+
+// the x-line pass on its own: x transform, Green step and inverse x transform
+// of the (y, z)-transformed spectrum (the same modes as below)
+int x_green_fp64(evpgpu_ctx *c) { return xg<double, 0>(c); }
+int x_green_delta(evpgpu_ctx *c) { return xg<float, 2>(c); }
+int x_green_anchor(evpgpu_ctx *c) { return xg<double, 3>(c); }
 
 // FP64 iteration: spec = R2C(sigma) ; Green (acc += antisym) ; E += add + C2R/N
 // (add: 6 values in device memory)
@@ -456,7 +477,7 @@ int fused_iteration_fp64(evpgpu_ctx *c, const double *sig, double *E, const doub
     if (!st) st = xg<double, 0>(c);
     tmark(c, 2, 1);
     tmark(c, 3, 0);
-    if (!st) st = yz<double, 0>(c, E, nullptr, scale, nullptr, nullptr, nullptr, add);
+    if (!st) st = yz<double, 0>(c, E, scale, nullptr, nullptr, add);
     tmark(c, 3, 1);
     return st;
 }
@@ -473,7 +494,7 @@ int fused_iteration_delta(evpgpu_ctx *c, const double *sig, const float *sigA, d
     if (!st) st = xg<float, 2>(c);
     tmark(c, 2, 1);
     tmark(c, 3, 0);
-    if (!st) st = yz<float, 2>(c, E, nullptr, scale, cA, nullptr, nullptr, add);
+    if (!st) st = yz<float, 2>(c, E, scale, cA, nullptr, add);
     tmark(c, 3, 1);
     return st;
 }
@@ -483,6 +504,6 @@ int fused_anchor(evpgpu_ctx *c, const float *sigA, float *cA, double scale)
 {
     int st = zy<double, 2>(c, nullptr, sigA);
     if (!st) st = xg<double, 3>(c);
-    if (!st) st = yz<double, 3>(c, nullptr, nullptr, scale, nullptr, cA, nullptr);
+    if (!st) st = yz<double, 3>(c, nullptr, scale, nullptr, cA);
     return st;
 }

@@ -41,9 +41,10 @@ using gop::gamma_apply;
 template <typename R, int MODE>
 __global__ __launch_bounds__(256) void k_green(typename CT<R>::T *spec, double2 *acc,
                                                double2 *out9, float2 *skA, GreenParams P, int nx,
-                                               int ny, int nz, int nzh, long long NK)
+                                               int ny, int nz, int nzh, long long NK, const int *skip)
 {
     typedef typename CT<R>::T C;
+    if (skip && *skip) return;
     __shared__ R c0s[36];
     if (threadIdx.x < 36) c0s[threadIdx.x] = (R)P.ga[threadIdx.x];
     __syncthreads();
@@ -228,7 +229,7 @@ int green_anchor(evpgpu_ctx *c)
     const GreenParams P = green_params(c);
     unsigned nb = (unsigned)((c->NK + 255) / 256);
     hipLaunchKernelGGL((k_green<double, 3>), dim3(nb), dim3(256), 0, c->stream, (double2 *)c->spec, nullptr,
-                       nullptr, c->skA, P, c->nx, c->ny, c->nz, c->nzh, c->NK);
+                       nullptr, c->skA, P, c->nx, c->ny, c->nz, c->nzh, c->NK, c->skip);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
@@ -237,7 +238,7 @@ int green_delta(evpgpu_ctx *c)
     const GreenParams P = green_params(c);
     unsigned nb = (unsigned)((c->NK + 255) / 256);
     hipLaunchKernelGGL((k_green<float, 2>), dim3(nb), dim3(256), 0, c->stream, (float2 *)c->spec, c->acc,
-                       nullptr, c->skA, P, c->nx, c->ny, c->nz, c->nzh, c->NK);
+                       nullptr, c->skA, P, c->nx, c->ny, c->nz, c->nzh, c->NK, c->skip);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
@@ -248,11 +249,11 @@ int green_apply(evpgpu_ctx *c, int precision, int accumulate)
     if (precision == EVPGPU_MIXED)
         hipLaunchKernelGGL((k_green<float, 0>), dim3(nb), dim3(256), 0, c->stream, (float2 *)c->spec,
                            accumulate ? c->acc : nullptr, nullptr, nullptr, P, c->nx, c->ny, c->nz, c->nzh,
-                           c->NK);
+                           c->NK, c->skip);
     else
         hipLaunchKernelGGL((k_green<double, 0>), dim3(nb), dim3(256), 0, c->stream, (double2 *)c->spec,
                            accumulate ? c->acc : nullptr, nullptr, nullptr, P, c->nx, c->ny, c->nz, c->nzh,
-                           c->NK);
+                           c->NK, c->skip);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
@@ -261,6 +262,6 @@ int green_full9(evpgpu_ctx *c, const double2 *in6, double2 *out9)
     const GreenParams P = green_params(c);
     unsigned nb = (unsigned)((c->NK + 255) / 256);
     hipLaunchKernelGGL((k_green<double, 1>), dim3(nb), dim3(256), 0, c->stream, (double2 *)in6, nullptr,
-                       out9, nullptr, P, c->nx, c->ny, c->nz, c->nzh, c->NK);
+                       out9, nullptr, P, c->nx, c->ny, c->nz, c->nzh, c->NK, c->skip);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
