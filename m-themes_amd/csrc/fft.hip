@@ -140,7 +140,7 @@ __global__ __launch_bounds__(NT) void k_fft_strided(typename CT<R>::T *data, int
 // loop's delta); IN 2: an FP32 field.
 template <typename R, int L, int IN>
 __global__ __launch_bounds__(NT) void k_fft_z_r2c(const double *in, const float *inA,
-                                                  typename CT<R>::T *out, long long N,
+                                                  typename CT<R>::T *out, long long nlines, long long N,
                                                   long long NK, const typename CT<R>::T *tw,
                                                   const int *skip)
 {
@@ -152,9 +152,10 @@ __global__ __launch_bounds__(NT) void k_fft_z_r2c(const double *in, const float 
     for (int i = threadIdx.x; i < L; i += NT) s_tw[i] = tw[i];
     const int comp = blockIdx.y;
     const long long line0 = (long long)blockIdx.x * TB;
+    const int nt = (int)min((long long)TB, nlines - line0);
     const long long off = comp * N + line0 * L; // even: the pairs below are aligned
     staged_copy<NT, (M * TB + NT - 1) / NT, IN == 1 ? 8 : 16, C>(
-        M * TB,
+        M * nt,
         [&](int e) {
             R a, b;
             if (IN == 0) {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(NT) void k_fft_z_r2c(const double *in, const float 
         split_forward<R, M>(lds + (i / (M / 2 + 1)) * P, i % (M / 2 + 1), (const C *)s_tw);
     __syncthreads();
     C *dst = out + comp * NK + line0 * P;
-    for (int e = threadIdx.x; e < P * TB; e += NT) dst[e] = lds[e];
+    for (int e = threadIdx.x; e < P * nt; e += NT) dst[e] = lds[e];
 }
 
 // ---- z pass, half spectrum -> real, Re(IFFT) of the Hermitian extension
@@ -197,9 +198,9 @@ __global__ __launch_bounds__(NT) void k_fft_z_r2c(const double *in, const float 
 template <typename R, int L, int MODE>
 __global__ __launch_bounds__(NT) void k_fft_z_c2r(const typename CT<R>::T *in, double *target,
                                                   const float *fa, float *fo, const double *base,
-                                                  long long N, long long NK, const double *addd,
-                                                  double scale, const typename CT<R>::T *tw,
-                                                  const int *skip)
+                                                  long long nlines, long long N, long long NK,
+                                                  const double *addd, double scale,
+                                                  const typename CT<R>::T *tw, const int *skip)
 {
     typedef typename CT<R>::T C;
     constexpr int M = L / 2, P = M + 1;
@@ -209,9 +210,10 @@ __global__ __launch_bounds__(NT) void k_fft_z_c2r(const typename CT<R>::T *in, d
     for (int i = threadIdx.x; i < L; i += NT) s_tw[i] = tw[i];
     const int comp = blockIdx.y;
     const long long line0 = (long long)blockIdx.x * TB;
+    const int nt = (int)min((long long)TB, nlines - line0);
     const C *src = in + comp * NK + line0 * P;
     staged_copy<NT, (P * TB + NT - 1) / NT, sizeof(R) == 8 ? 8 : 16, C>(
-        P * TB, [&](int e) { return src[e]; }, [&](int e, C v) { lds[e] = v; });
+        P * nt, [&](int e) { return src[e]; }, [&](int e, C v) { lds[e] = v; });
     __syncthreads();
     for (int i = threadIdx.x; i < TB * (M / 2 + 1); i += NT)
         split_inverse<R, M>(lds + (i / (M / 2 + 1)) * P, i % (M / 2 + 1), (const C *)s_tw);
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(NT) void k_fft_z_c2r(const typename CT<R>::T *in, d
     gstages<true, M, 0, 1, TB, P, 1, 0, NT, 2>(lds, (const C *)s_tw);
     const double add = addd ? addd[comp] : 0.0;
     const long long off = comp * N + line0 * L;
-    for (int e = threadIdx.x; e < M * TB; e += NT) {
+    for (int e = threadIdx.x; e < M * nt; e += NT) {
         const int t = e / M, n = e % M;
         const C z = lds[t * P + n];
         const double r0 = (double)z.x * scale, r1 = (double)z.y * scale;
@@ -242,8 +244,8 @@ __global__ __launch_bounds__(NT) void k_fft_z_c2r(const typename CT<R>::T *in, d
     }
 }
 
-// ---- any length: two-level DFTs.  An axis whose length is not a power of
-// two (FFTW, which the reference calls, takes any length) is transformed with
+// ---- any length: two-level DFTs.  An axis whose length has no Stockham plan
+// (FFTW, which the reference calls, takes any length) is transformed with
 // L = L1 L2 (L1 the largest divisor <= sqrt L): length-L1 DFTs down the
 // columns of the L1 x L2 view of each line, the twiddles w^(n2 k1), then
 // length-L2 DFTs along the rows (Cooley-Tukey with direct inner DFTs), the
@@ -417,14 +419,21 @@ __global__ __launch_bounds__(NT) void k_dft_z_c2r(const typename CT<R>::T *in, d
     });
 }
 
-// lengths with a Stockham plan (2^m 3^a 5^b, divisible by 4, in [8, 256];
-// the list of FFT_DISPATCH); the others take the two-level DFT kernels
-bool is_stockham_len(int L)
+// Lengths with a Stockham plan: the 2^m 3^a 5^b of FFT_DISPATCH; the others
+// take the two-level DFT kernels.  Real lines (z) go through a transform of
+// half the length, so theirs are the even ones.  (45 x 50 x 27 in FP32: the y
+// passes 8.6 -> 4.3 us each, and x with the Green step 22 -> 9 us, against the
+// DFT kernels these lengths took before.)
+bool is_stockham_len(int L, bool real = false)
 {
-    static const int lens[] = {8, 12, 16, 20, 24, 32, 36, 40, 48, 60, 64, 72, 80, 96, 100, 120,
-                               128, 144, 160, 192, 200, 240, 256};
-    for (int l : lens)
+    static const int even[] = {
+        8, 10, 12, 16, 18, 20, 24, 30, 32, 36, 40, 48, 50, 54, 60, 64, 72, 80, 90, 96, 100, 108,
+        120, 128, 144, 150, 160, 180, 192, 200, 216, 240, 250, 256};
+    static const int odd[] = {15, 25, 27, 45, 75, 125, 225};
+    for (int l : even)
         if (l == L) return true;
+    for (int l : odd)
+        if (l == L) return !real;
     return false;
 }
 
@@ -433,33 +442,55 @@ template <> const double2 *twp<double>(evpgpu_ctx *c, int axis) { return c->tw64
 template <> const float2 *twp<float>(evpgpu_ctx *c, int axis) { return c->tw32[axis]; }
 
 // dispatch on a runtime length
-#define FFT_DISPATCH(L_, CALL) \
+#define FFT_DISPATCH_EVEN(L_, CALL, ODD_) \
     switch (L_) {              \
-    case 8: CALL(8); break;    \
-    case 12: CALL(12); break;  \
-    case 16: CALL(16); break;  \
-    case 20: CALL(20); break;  \
-    case 24: CALL(24); break;  \
-    case 32: CALL(32); break;  \
-    case 36: CALL(36); break;  \
-    case 40: CALL(40); break;  \
-    case 48: CALL(48); break;  \
-    case 60: CALL(60); break;  \
-    case 64: CALL(64); break;  \
-    case 72: CALL(72); break;  \
-    case 80: CALL(80); break;  \
-    case 96: CALL(96); break;  \
+    case 8: CALL(8); break; \
+    case 10: CALL(10); break; \
+    case 12: CALL(12); break; \
+    case 16: CALL(16); break; \
+    case 18: CALL(18); break; \
+    case 20: CALL(20); break; \
+    case 24: CALL(24); break; \
+    case 30: CALL(30); break; \
+    case 32: CALL(32); break; \
+    case 36: CALL(36); break; \
+    case 40: CALL(40); break; \
+    case 48: CALL(48); break; \
+    case 50: CALL(50); break; \
+    case 54: CALL(54); break; \
+    case 60: CALL(60); break; \
+    case 64: CALL(64); break; \
+    case 72: CALL(72); break; \
+    case 80: CALL(80); break; \
+    case 90: CALL(90); break; \
+    case 96: CALL(96); break; \
     case 100: CALL(100); break; \
+    case 108: CALL(108); break; \
     case 120: CALL(120); break; \
     case 128: CALL(128); break; \
     case 144: CALL(144); break; \
+    case 150: CALL(150); break; \
     case 160: CALL(160); break; \
+    case 180: CALL(180); break; \
     case 192: CALL(192); break; \
     case 200: CALL(200); break; \
+    case 216: CALL(216); break; \
     case 240: CALL(240); break; \
+    case 250: CALL(250); break; \
     case 256: CALL(256); break; \
+    ODD_                       \
     default: return EVPGPU_ERR_SIZE; \
     }
+#define FFT_ODD(CALL) \
+    case 15: CALL(15); break; \
+    case 25: CALL(25); break; \
+    case 27: CALL(27); break; \
+    case 45: CALL(45); break; \
+    case 75: CALL(75); break; \
+    case 125: CALL(125); break; \
+    case 225: CALL(225); break;
+#define FFT_DISPATCH(L_, CALL) FFT_DISPATCH_EVEN(L_, CALL, FFT_ODD(CALL))
+#define FFT_DISPATCH_REAL(L_, CALL) FFT_DISPATCH_EVEN(L_, CALL, )
 
 template <typename R, bool INV>
 int pass_y(evpgpu_ctx *c, typename CT<R>::T *d, int ncomp)
@@ -504,19 +535,18 @@ int pass_x(evpgpu_ctx *c, typename CT<R>::T *d, int ncomp)
 template <typename R, int IN>
 int fwd_zy(evpgpu_ctx *c, const double *real_in, const float *inA, int ncomp, typename CT<R>::T *spec)
 {
-    // the Stockham z kernels take whole groups of TB lines
-    if (!is_stockham_len(c->nz) || (c->nx * c->ny) % TB != 0) {
+    const long long nl = (long long)c->nx * c->ny;
+    if (!is_stockham_len(c->nz, true)) {
         const int L = c->nz, tbl = dft_lines(L);
-        const long long nl = (long long)c->nx * c->ny;
         hipLaunchKernelGGL((k_dft_z_r2c<R, IN>), dim3((unsigned)((nl + tbl - 1) / tbl), ncomp), dim3(NT),
                            sizeof(typename CT<R>::T) * (2 * tbl + 1) * L, c->stream, real_in, inA, spec, L, nl, c->N,
                            c->NK, twp<R>(c, 2), c->skip);
         if (hipGetLastError() != hipSuccess) return EVPGPU_ERR_HIP;
     } else {
-    dim3 g((unsigned)(c->nx * c->ny / TB), ncomp);
+    dim3 g((unsigned)((nl + TB - 1) / TB), ncomp);
 #define CALLZ(L) hipLaunchKernelGGL((k_fft_z_r2c<R, L, IN>), g, dim3(NT), 0, c->stream, real_in, inA, \
-                                    spec, c->N, c->NK, twp<R>(c, 2), c->skip)
-    FFT_DISPATCH(c->nz, CALLZ);
+                                    spec, nl, c->N, c->NK, twp<R>(c, 2), c->skip)
+    FFT_DISPATCH_REAL(c->nz, CALLZ);
 #undef CALLZ
     }
     return pass_y<R, false>(c, spec, ncomp);
@@ -535,18 +565,18 @@ int inv_yz(evpgpu_ctx *c, typename CT<R>::T *spec, int ncomp, double *target, co
 {
     int st = pass_y<R, true>(c, spec, ncomp);
     if (st) return st;
-    if (!is_stockham_len(c->nz) || (c->nx * c->ny) % TB != 0) {
+    const long long nl = (long long)c->nx * c->ny;
+    if (!is_stockham_len(c->nz, true)) {
         const int L = c->nz, tbl = dft_lines(L);
-        const long long nl = (long long)c->nx * c->ny;
         hipLaunchKernelGGL((k_dft_z_c2r<R, MODE>), dim3((unsigned)((nl + tbl - 1) / tbl), ncomp), dim3(NT),
                            sizeof(typename CT<R>::T) * (2 * tbl + 1) * L, c->stream, spec, target, fa, fo, base,
                            L, nl, c->N, c->NK, addd, scale, twp<R>(c, 2), c->skip);
         return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
     }
-    dim3 g((unsigned)(c->nx * c->ny / TB), ncomp);
+    dim3 g((unsigned)((nl + TB - 1) / TB), ncomp);
 #define CALLZI(L) hipLaunchKernelGGL((k_fft_z_c2r<R, L, MODE>), g, dim3(NT), 0, c->stream, spec, target, \
-                                     fa, fo, base, c->N, c->NK, addd, scale, twp<R>(c, 2), c->skip)
-    FFT_DISPATCH(c->nz, CALLZI);
+                                     fa, fo, base, nl, c->N, c->NK, addd, scale, twp<R>(c, 2), c->skip)
+    FFT_DISPATCH_REAL(c->nz, CALLZI);
 #undef CALLZI
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }

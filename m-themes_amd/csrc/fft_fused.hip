@@ -363,29 +363,47 @@ constexpr int TILE_FILL = 512;
 // x-line lengths: the Stockham lengths of fft.hip
 #define LINE_DISPATCH(CALL)             \
     switch (c->nx) {                    \
-    case 8: CALL(8); break;             \
-    case 12: CALL(12); break;           \
-    case 16: CALL(16); break;           \
-    case 20: CALL(20); break;           \
-    case 24: CALL(24); break;           \
-    case 32: CALL(32); break;           \
-    case 36: CALL(36); break;           \
-    case 40: CALL(40); break;           \
-    case 48: CALL(48); break;           \
-    case 60: CALL(60); break;           \
-    case 64: CALL(64); break;           \
-    case 72: CALL(72); break;           \
-    case 80: CALL(80); break;           \
-    case 96: CALL(96); break;           \
-    case 100: CALL(100); break;         \
-    case 120: CALL(120); break;         \
-    case 128: CALL(128); break;         \
-    case 144: CALL(144); break;         \
-    case 160: CALL(160); break;         \
-    case 192: CALL(192); break;         \
-    case 200: CALL(200); break;         \
-    case 240: CALL(240); break;         \
-    case 256: CALL(256); break;         \
+    case 8: CALL(8); break; \
+    case 10: CALL(10); break; \
+    case 12: CALL(12); break; \
+    case 15: CALL(15); break; \
+    case 16: CALL(16); break; \
+    case 18: CALL(18); break; \
+    case 20: CALL(20); break; \
+    case 24: CALL(24); break; \
+    case 25: CALL(25); break; \
+    case 27: CALL(27); break; \
+    case 30: CALL(30); break; \
+    case 32: CALL(32); break; \
+    case 36: CALL(36); break; \
+    case 40: CALL(40); break; \
+    case 45: CALL(45); break; \
+    case 48: CALL(48); break; \
+    case 50: CALL(50); break; \
+    case 54: CALL(54); break; \
+    case 60: CALL(60); break; \
+    case 64: CALL(64); break; \
+    case 72: CALL(72); break; \
+    case 75: CALL(75); break; \
+    case 80: CALL(80); break; \
+    case 90: CALL(90); break; \
+    case 96: CALL(96); break; \
+    case 100: CALL(100); break; \
+    case 108: CALL(108); break; \
+    case 120: CALL(120); break; \
+    case 125: CALL(125); break; \
+    case 128: CALL(128); break; \
+    case 144: CALL(144); break; \
+    case 150: CALL(150); break; \
+    case 160: CALL(160); break; \
+    case 180: CALL(180); break; \
+    case 192: CALL(192); break; \
+    case 200: CALL(200); break; \
+    case 216: CALL(216); break; \
+    case 225: CALL(225); break; \
+    case 240: CALL(240); break; \
+    case 250: CALL(250); break; \
+    case 256: CALL(256); break; \
     default: return EVPGPU_ERR_SIZE;    \
     }
 
@@ -443,8 +461,9 @@ int xg(evpgpu_ctx *c)
 // the lengths nx of LINE_DISPATCH
 bool lines_ok(const evpgpu_ctx *c)
 {
-    static const int lines[] = {8,  12, 16, 20, 24,  32,  36,  40,  48,  60,  64, 72,
-                                80, 96, 100, 120, 128, 144, 160, 192, 200, 240, 256};
+    static const int lines[] = {
+        8, 10, 12, 15, 16, 18, 20, 24, 25, 27, 30, 32, 36, 40, 45, 48, 50, 54, 60, 64, 72, 75, 80,
+        90, 96, 100, 108, 120, 125, 128, 144, 150, 160, 180, 192, 200, 216, 225, 240, 250, 256};
     for (int n : lines)
         if (c->nx == n) return true;
     return false;

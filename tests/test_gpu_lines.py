@@ -1,4 +1,7 @@
-"""The x-line Green kernel between the separate y and z passes (grids whose
+"""Transforms of the lengths with a Stockham plan that are not multiples of 4,
+against numpy (the bars of tests/test_gpu_anysize.py: 1e-12 FP64, 2e-6 FP32),
+z lines in groups that do not fill the last workgroup among them; and
+the x-line Green kernel between the separate y and z passes (grids whose
 (y, z) planes do not take the fused kernels) against the seven-pass path: new
 line lengths, tiles of 16, 8, 4 and 2 columns, column counts that leave the last
 tile ragged, odd y and z lengths, FP64 and mixed.  The two paths compute the
@@ -10,6 +13,25 @@ import pytest
 from pyevp import lib
 
 pytestmark = pytest.mark.gpu
+
+
+# every new length along x or y, every new even one along z; nx ny = 1 or 15 mod 16
+@pytest.mark.parametrize("dims", [(15, 25, 10), (27, 45, 18), (75, 3, 30), (125, 5, 50), (225, 3, 54), (5, 15, 90),
+                                  (10, 27, 108), (18, 75, 4), (30, 125, 2), (50, 225, 6), (54, 10, 150), (90, 18, 12),
+                                  (108, 30, 4), (150, 54, 4), (180, 90, 8), (216, 108, 2), (250, 150, 2), (4, 180, 180),
+                                  (3, 216, 216), (3, 250, 250)])
+@pytest.mark.parametrize("prec", [lib.FP64, lib.MIXED])
+def test_mixed_radix_lengths_vs_numpy(dims, prec):
+    rng = np.random.default_rng(sum(dims))
+    x = rng.standard_normal(dims)
+    tol = 1e-12 if prec == lib.FP64 else 2e-6
+    c = lib.Context(*dims, prec)
+    X = c.rfftn(x)
+    ref = np.fft.rfftn(x)
+    assert np.max(np.abs(X - ref)) < tol * np.max(np.abs(ref))
+    y = c.irfftn_unnormalised(ref) / x.size
+    assert np.max(np.abs(y - x)) < tol * np.max(np.abs(x))
+    c.close()
 
 
 def rel(a, b):
