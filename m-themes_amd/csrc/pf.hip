@@ -24,8 +24,8 @@
 //      re-labelled or appended last entry at that turn carries the last
 //      such grain looked up.
 //   4. rho_avg[g-1] at a voxel's turn was written by the last voxel before
-//      it (or itself) whose list held g: sorted (grain, position) keys and a
-//      binary search.  The stored-energy reset to 100 (a new grain passing
+//      it (or itself) whose list held g: the writes sorted by grain, each
+//      grain's in sweep order, and a search.  The stored-energy reset to 100 (a new grain passing
 //      0.5) feeds later voxels' 7x7x7 averages; the triggers are iterated to
 //      their fixed point over the sweep order.
 // Lists are structure of arrays, entry k of cell c at k*NC + c, over the
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(ACT_NT) void k_act_iter(Dims g, const int *emask, i
 // neighbour looked up.  nn: entries; spos: position of that entry or -1;
 // sg: its grain; wn: rho_avg writes (nn on the update branch).
 __global__ __launch_bounds__(NT) void k_slot(Dims g, Lists A, const int *gcnt, const int *gidx, const int *act, int *nn, int *spos,
-                       int *sg, int *wn, int *nupd, int *err)
+                       int *sg, int *wn, int *err)
 {
     // The loads go out in two batches instead of one chain per neighbour:
     // first the voxel's own list (its first OWN entries whatever the count:
@@ -323,7 +323,6 @@ __global__ __launch_bounds__(NT) void k_slot(Dims g, Lists A, const int *gcnt, c
         spos[d] = p;
         sg[d] = s;
         wn[d] = n > 1 ? n : 0;
-        if (n > 1) atomicAdd(nupd, 1);
     }
 }
 
@@ -339,9 +338,21 @@ __device__ inline void entry(const Dims &g, const Lists &A, long long c, int k, 
     }
 }
 
-// rho_avg writes as (grain - 1, sweep position) keys
+// a voxel's part of the writer scan: its writes in the low half, itself (if
+// it has any) in the high half, so that one scan gives the writers' offsets
+// and the number of voxels on the update branch
+constexpr long long SCAN_LOW = 1LL << 32;
+struct WriterScan {
+    __host__ __device__ long long operator()(int n) const { return n > 0 ? SCAN_LOW + n : 0; }
+};
+
+// rho_avg writes in sweep order: keys grain - 1, references voxel * CAP +
+// entry.  A stable sort by the grain alone then leaves each grain's run in
+// sweep order (16 bits of 60 000 grains instead of 37 of grain and position,
+// and the searches read 4-byte references instead of 8-byte keys: the sort
+// took 200 us at 128^3, now 75)
 __global__ __launch_bounds__(NT) void k_emit(Dims g, Lists A, const int *nn, const int *spos, const int *sg, const int *wn,
-                       const long long *woff, unsigned long long *keys, int *refs, int n_rho, int *err)
+                       const long long *woff, unsigned *keys, int *refs, int n_rho, int *err)
 {
     for (long long d = blockIdx.x * (long long)NT + threadIdx.x; d < g.NV; d += (long long)gridDim.x * NT) {
         const int n = wn[d];
@@ -349,7 +360,7 @@ __global__ __launch_bounds__(NT) void k_emit(Dims g, Lists A, const int *nn, con
         int x, y, z;
         vox(g, d, x, y, z);
         const long long c = cix(g, x, y, z);
-        long long o = woff[d];
+        long long o = woff[d] & (SCAN_LOW - 1);
         for (int k = 0; k < n; k++) {
             int gr;
             double v;
@@ -358,7 +369,7 @@ __global__ __launch_bounds__(NT) void k_emit(Dims g, Lists A, const int *nn, con
                 atomicOr(err, PFE_GRAIN);
                 gr = 1;
             }
-            keys[o] = (unsigned long long)(gr - 1) * (unsigned long long)g.NV + (unsigned long long)d;
+            keys[o] = (unsigned)(gr - 1);
             refs[o] = (int)(d * CAP + k);
             o++;
         }
@@ -375,14 +386,40 @@ __global__ __launch_bounds__(NT) void k_emit(Dims g, Lists A, const int *nn, con
 constexpr int TX = 4, TY = 8, TZ = 8, HX = TX + 6, HY = TY + 6, HZ = TZ + 6, HC = HX * HY * HZ;
 static_assert(TX * TY * TZ == NT, "one voxel per thread");
 
+// n words (0 <= n <= 15) for each active lane from an LDS counter: the lane's
+// first word.  One atomic per wave: the lanes' offsets come from ballots of
+// the bits of n (600 atomics on one word took 64 us of a 128^3 pass).
+__device__ inline int wave_take(int *used, int n)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    int off = 0, tot = 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        const unsigned long long m = __ballot((n >> b) & 1);
+        off += __popcll(m & below) << b;
+        tot += __popcll(m) << b;
+    }
+    const unsigned long long act = __ballot(1);
+    const int lead = __ffsll(act) - 1;
+    int base = 0;
+    if (lane == lead) base = atomicAdd(used, tot);
+    return __shfl(base, lead, 64) + off;
+}
+
 // The lists of a 4 x 8 x 8 voxel tile and of its face/edge neighbours (a
-// 6 x 10 x 10 cell box) staged in LDS: counts and the first LE entries;
-// entries beyond LE (rare) are read from memory.  31 KB.
-constexpr int LX = TX + 2, LY = TY + 2, LZ = TZ + 2, LC = LX * LY * LZ, LE = 4;
+// 6 x 10 x 10 cell box) packed in LDS as lookups read them: per cell the run
+// of its entries (a last one below EPSILON left out, since a lookup then never
+// finds it) and what a lookup of any other grain returns.  Cells that do not
+// fit the LE entries (2.5 per cell; the mean is 1.6 to 2.3) are marked and read
+// from memory.  Fixed slots of 4 per cell took 33 KB instead of 26, and sent
+// every list of 5 (one voxel in 100) to memory, a microsecond a trip.
+constexpr int LX = TX + 2, LY = TY + 2, LZ = TZ + 2, LC = LX * LY * LZ, LE = 1536;
 struct ListTile {
-    int cnt[LC];
-    int idx[LE * LC];
-    double val[LE * LC];
+    int meta[LC]; // first entry, entries << 16; -1: read the list from memory
+    int idx[LE + 3];
+    double val[LE], other[LC];
+    int used;
 };
 
 // tile b's first voxel in padded coordinates
@@ -396,21 +433,44 @@ __device__ inline void tile_origin(const Dims &g, int b, int &x0, int &y0, int &
 
 __device__ inline void load_lists(ListTile &T, const Dims &g, const Lists &A, int x0, int y0, int z0)
 {
+    if (threadIdx.x == 0) T.used = 0;
+    __syncthreads();
     for (int q = threadIdx.x; q < LC; q += NT) {
         const int hz = q % LZ, hy = (q / LZ) % LY, hx = q / (LZ * LY);
         const int i = x0 - 1 + hx, j = y0 - 1 + hy, m = z0 - 1 + hz;
-        int n = 0;
-        if (i < g.lx && j < g.ly && m < g.lz) {
-            const long long c = cix(g, i, j, m);
-            n = A.cnt[c];
-#pragma unroll
-            for (int k = 0; k < LE; k++)
-                if (k < n) {
-                    T.idx[k * LC + q] = A.idx[(long long)k * g.NC + c];
-                    T.val[k * LC + q] = A.val[(long long)k * g.NC + c];
-                }
+        const bool in = i < g.lx && j < g.ly && m < g.lz;
+        const long long c = in ? cix(g, i, j, m) : 0;
+        // the first two entries come with the count, whatever it is (the
+        // arrays hold CAP per cell): most lists end there
+        const int n = in ? A.cnt[c] : 0;
+        const int i0 = A.idx[c], i1 = A.idx[g.NC + c];
+        const double v0 = A.val[c], v1 = A.val[g.NC + c];
+        const double back = n == 0 ? 1.0 : n == 1 ? v0 : n == 2 ? v1 : A.val[(long long)(n - 1) * g.NC + c];
+        const bool relabel = back < PF_EPS;
+        const int nf = relabel ? n - 1 : n;
+        int take = nf;
+        if (take == CAP) take = CAP - 1; // (a full list is read from memory)
+        const int o = wave_take(&T.used, take);
+        int meta = -1;
+        double other = 0.0;
+        if (nf < CAP && o + nf <= LE) {
+            meta = o | (nf << 16);
+            if (relabel) other = back;
+            if (nf > 0) {
+                T.idx[o] = i0;
+                T.val[o] = v0;
+            }
+            if (nf > 1) {
+                T.idx[o + 1] = i1;
+                T.val[o + 1] = v1;
+            }
+            for (int k = 2; k < nf; k++) {
+                T.idx[o + k] = A.idx[(long long)k * g.NC + c];
+                T.val[o + k] = A.val[(long long)k * g.NC + c];
+            }
         }
-        T.cnt[q] = n;
+        T.meta[q] = meta;
+        T.other[q] = other;
     }
 }
 
@@ -420,153 +480,184 @@ __device__ inline int tq(int tx, int ty, int tz, int dx, int dy, int dz)
     return ((tx + 1 + dx) * LY + (ty + 1 + dy)) * LZ + (tz + 1 + dz);
 }
 
-__device__ inline int tile_idx(const ListTile &T, const Dims &g, const Lists &A, int q, long long c, int k)
-{
-    return k < LE ? T.idx[k * LC + q] : A.idx[(long long)k * g.NC + c];
-}
-
-__device__ inline double tile_val(const ListTile &T, const Dims &g, const Lists &A, int q, long long c, int k)
-{
-    return k < LE ? T.val[k * LC + q] : A.val[(long long)k * g.NC + c];
-}
-
 // the value a PFdata lookup of grain gr returns from a start-of-sweep list
-// (tile cell q, memory cell c): its value when gr is an entry other than a
-// last entry below EPSILON, else that last entry's value when below, else 0
-__device__ inline double lookup_t(const ListTile &T, const Dims &g, const Lists &A, int q, long long c, int gr)
+// (memory cell c): its value when gr is an entry other than a last entry
+// below EPSILON, else that last entry's value when below, else 0
+__device__ __noinline__ double lookup_list(const Lists &A, long long NC, long long c, int gr)
 {
-    const int n = T.cnt[q];
+    const int n = A.cnt[c];
     if (n == 0) return 0.0;
-    const double back = tile_val(T, g, A, q, c, n - 1);
+    const double back = A.val[(long long)(n - 1) * NC + c];
     const bool relabel = back < PF_EPS;
     const int nf = relabel ? n - 1 : n;
     for (int k = 0; k < nf; k++)
-        if (tile_idx(T, g, A, q, c, k) == gr) return tile_val(T, g, A, q, c, k);
+        if (A.idx[(long long)k * NC + c] == gr) return A.val[(long long)k * NC + c];
     return relabel ? back : 0.0;
 }
 
+// the same from the staged lists (tile cell q): the first matching entry.
+// Three entries are read whatever the count (past the run's end lie other
+// cells' entries, or the array's last words): one trip to LDS.
+__device__ inline double lookup_t(const ListTile &T, const Dims &g, const Lists &A, int q, long long c, int gr)
+{
+    const int meta = T.meta[q];
+    if (meta < 0) return lookup_list(A, g.NC, c, gr);
+    const int o = meta & 0xffff, n = meta >> 16;
+    const int i0 = T.idx[o], i1 = T.idx[o + 1], i2 = T.idx[o + 2];
+    int k = n > 0 && i0 == gr ? 0 : n > 1 && i1 == gr ? 1 : n > 2 && i2 == gr ? 2 : -1;
+    if (k < 0 && n > 3)
+        for (int m = 3; m < n && k < 0; m++) k = T.idx[o + m] == gr ? m : -1;
+    return k < 0 ? T.other[q] : T.val[o + k];
+}
+
 // candidate grains: values above EPSILON in the 3x3x3 neighbourhood, in
-// order of first appearance (src/pf_xrx.c:940-975); lists from the tile
+// order of first appearance (src/pf_xrx.c:940-975).  The tile's box is staged
+// as each cell's candidates, packed as in ListTile.
+constexpr int NO_GRAIN = INT_MIN;
+
 __global__ __launch_bounds__(NT) void k_glist(Dims g, Lists A, int *gcnt, int *gidx, int *err)
 {
-    __shared__ ListTile T;
+    __shared__ int s_meta[LC], s_id[LE + 2], s_used;
+    __shared__ int s_G[CAP * NT]; // the voxel's grains, a column per thread
     int x0, y0, z0;
     tile_origin(g, blockIdx.x, x0, y0, z0);
-    load_lists(T, g, A, x0, y0, z0);
+    if (threadIdx.x == 0) s_used = 0;
+    __syncthreads();
+    for (int q = threadIdx.x; q < LC; q += NT) {
+        const int hz = q % LZ, hy = (q / LZ) % LY, hx = q / (LZ * LY);
+        const int i = x0 - 1 + hx, j = y0 - 1 + hy, m = z0 - 1 + hz;
+        const bool in = i < g.lx && j < g.ly && m < g.lz;
+        const long long c = in ? cix(g, i, j, m) : 0;
+        const int n = in ? A.cnt[c] : 0; // (the first two entries come with it)
+        const int i0 = A.idx[c], i1 = A.idx[g.NC + c];
+        const double v0 = A.val[c], v1 = A.val[g.NC + c];
+        const int o = wave_take(&s_used, n < CAP ? n : CAP - 1);
+        int meta = -1;
+        if (n < CAP && o + n <= LE) {
+            int w = o;
+            if (n > 0 && v0 > PF_EPS) s_id[w++] = i0;
+            if (n > 1 && v1 > PF_EPS) s_id[w++] = i1;
+            for (int k = 2; k < n; k++)
+                if (A.val[(long long)k * g.NC + c] > PF_EPS) s_id[w++] = A.idx[(long long)k * g.NC + c];
+            meta = o | ((w - o) << 16);
+        }
+        s_meta[q] = meta;
+    }
     __syncthreads();
     const int tz = threadIdx.x % TZ, ty = (threadIdx.x / TZ) % TY, tx = threadIdx.x / (TZ * TY);
     const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
     if (!interior(g, x, y, z)) return;
     const long long d = vid(g, x, y, z);
-    int G[CAP];
-    int nG = 0;
+    // The first eight grains also in registers (the free ones hold the first
+    // grain): a grain met is nearly always one of them, and adding one is
+    // eight selects and an LDS write.  (All 16 in a register array made every
+    // addition a chain in which the lanes of a wave took turns; four in
+    // registers left each check an LDS search where five grains meet: 70 us for
+    // the 270 workgroups of a 48 x 40 x 36 grid against 57.)
+    constexpr int NR = 8;
+    int G[NR], nG = 0;
+#pragma unroll
+    for (int k = 0; k < NR; k++) G[k] = 0;
+    int *col = s_G + threadIdx.x;
     bool over = false;
-    for (int i = -1; i <= 1; ++i)
-        for (int j = -1; j <= 1; ++j)
-            for (int m = -1; m <= 1; ++m) {
-                const int q = tq(tx, ty, tz, i, j, m);
+    auto add = [&](int index) {
+        bool seen = false;
+#pragma unroll
+        for (int k = 0; k < NR; k++) seen = seen || index == G[k];
+        if (seen && nG > 0) return;
+        for (int it = NR; it < nG; it++)
+            if (col[it * NT] == index) return;
+        if (nG == CAP) {
+            over = true;
+            return;
+        }
+#pragma unroll
+        for (int k = 0; k < NR; k++) G[k] = nG == 0 || nG == k ? index : G[k];
+        col[nG * NT] = index;
+        nG++;
+    };
+#pragma unroll 1
+    for (int ij = 0; ij < 9; ++ij)
+#pragma unroll
+        for (int m = -1; m <= 1; ++m) {
+            const int i = ij / 3 - 1, j = ij % 3 - 1;
+            const int meta = s_meta[tq(tx, ty, tz, i, j, m)];
+            if (meta < 0) {
                 const long long c = cix(g, x + i, y + j, z + m);
-                const int n = T.cnt[q];
+                const int n = A.cnt[c];
                 for (int k = 0; k < n; ++k)
-                    if (tile_val(T, g, A, q, c, k) > PF_EPS) {
-                        const int index = tile_idx(T, g, A, q, c, k);
-                        bool seen = false;
-#pragma unroll
-                        for (int it = 0; it < CAP; it++) seen = seen || (it < nG && G[it] == index);
-                        if (!seen) {
-                            if (nG == CAP) {
-                                over = true;
-                            } else {
-#pragma unroll
-                                for (int it = 0; it < CAP; it++)
-                                    if (it == nG) G[it] = index;
-                                nG++;
-                            }
-                        }
-                    }
+                    if (A.val[(long long)k * g.NC + c] > PF_EPS) add(A.idx[(long long)k * g.NC + c]);
+                continue;
             }
+            const int o = meta & 0xffff, n = meta >> 16;
+            const int i0 = s_id[o], i1 = s_id[o + 1];
+            if (n > 0) add(i0);
+            if (n > 1) add(i1);
+            for (int k = 2; k < n; k++) add(s_id[o + k]);
+        }
     if (over) atomicOr(err, PFE_CAP);
     gcnt[d] = nG;
-#pragma unroll
-    for (int k = 0; k < CAP; k++)
-        if (k < nG) gidx[(long long)k * g.NV + d] = G[k];
+    for (int k = 0; k < nG; k++) gidx[(long long)k * g.NV + d] = col[k * NT];
 }
 
-
-// the sums of one voxel over its box, for lists of at most M entries (the
-// entries' grains, sums and counts stay in registers)
-template <int M>
-__device__ inline void avg_box(const Dims &g, const Lists &A, long long c, long long d, int n, int p, int s, int tx,
-                               int ty, int tz, int x, int y, int z, const int *s_gid, const double *s_de,
-                               const unsigned char *s_tf, double *avg, int *cdd)
+// exclusive prefix sums of one small count per thread over the workgroup
+// (s_w: NT / 64 ints of LDS); the total in tot
+__device__ inline int block_prefix(int n, int *s_w, int &tot)
 {
-    int gk[M];
-    double a[M];
-    int cn[M];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int x = n;
 #pragma unroll
-    for (int k = 0; k < M; k++) {
-        gk[k] = INT_MIN; // matches no grain, nor the -1 of cells outside the grid
-        if (k < n) {
-            double v;
-            entry(g, A, c, k, p, s, gk[k], v);
-        }
-        a[k] = 0.0;
-        cn[k] = 0;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
     }
-    if constexpr (M > 4) {
-        // long lists (rare): the cell-by-cell loop, which holds fewer registers
-        for (int i = 0; i < 7; ++i)
-            for (int j = 0; j < 7; ++j)
-                for (int m = 0; m < 7; ++m) {
-                    const int q = ((tx + i) * HY + (ty + j)) * HZ + (tz + m);
-                    const int gp = s_gid[q];
-                    bool hit = false;
+    if (lane == 63) s_w[w] = x;
+    __syncthreads();
+    int base = 0;
+    tot = 0;
 #pragma unroll
-                    for (int k = 0; k < M; k++) hit = hit || gp == gk[k];
-                    if (!hit) continue;
-                    double e = s_de[q];
-                    if (s_tf[q] && vid(g, x - 3 + i, y - 3 + j, z - 3 + m) < d) e = 100.0;
+    for (int i = 0; i < NT / 64; i++) {
+        if (i < w) base += s_w[i];
+        tot += s_w[i];
+    }
+    return base + x - n;
+}
+
+// The sums of two entries (grains g0, g1) of one voxel over its box, whose
+// first cell is q0, cell by cell in the reference's order; TRIG: cells an
+// earlier voxel reset (their flag set and their position before d) read 100.
+template <bool TRIG>
+__device__ inline void avg_pair(const Dims &g, const int *s_gid, const double *s_de, const unsigned char *s_tf,
+                                int q0, int x, int y, int z, long long d, int g0, int g1, double &a0, double &a1,
+                                int &c0, int &c1)
+{
+    a0 = a1 = 0.0;
+    c0 = c1 = 0;
+    for (int i = 0; i < 7; ++i)
+        for (int j = 0; j < 7; ++j) {
+            // one z row of the box: its 7 cells' LDS reads go out together,
+            // then the sums in the cells' order.  Adding 0 where a cell is of
+            // another grain leaves the sum as it is: the sums start at +0 and
+            // no sum of doubles turns that into -0.
+            const int q = q0 + (i * HY + j) * HZ;
+            int gp[7];
+            double e[7];
 #pragma unroll
-                    for (int k = 0; k < M; k++)
-                        if (gp == gk[k]) {
-                            a[k] += e;
-                            cn[k] += 1;
-                        }
-                }
-    } else {
-        for (int i = 0; i < 7; ++i)
-            for (int j = 0; j < 7; ++j) {
-                // one z row of the box: its 7 cells' LDS reads go out together,
-                // then the sums in the cells' order (the reads are unconditional,
-                // the sums predicated)
-                const int q0 = ((tx + i) * HY + (ty + j)) * HZ + tz;
-                int gp[7];
-                double ev[7];
-                unsigned char tf[7];
-#pragma unroll
-                for (int m = 0; m < 7; ++m) {
-                    gp[m] = s_gid[q0 + m];
-                    ev[m] = s_de[q0 + m];
-                    tf[m] = s_tf[q0 + m];
-                }
-#pragma unroll
-                for (int m = 0; m < 7; ++m) {
-                    double e = ev[m];
-                    if (tf[m] && vid(g, x - 3 + i, y - 3 + j, z - 3 + m) < d) e = 100.0;
-#pragma unroll
-                    for (int k = 0; k < M; k++)
-                        if (gp[m] == gk[k]) {
-                            a[k] += e;
-                            cn[k] += 1;
-                        }
-                }
+            for (int m = 0; m < 7; ++m) {
+                gp[m] = s_gid[q + m];
+                e[m] = s_de[q + m];
             }
-    }
+            if (TRIG)
 #pragma unroll
-    for (int k = 0; k < M; k++)
-        if (k < n) {
-            avg[(long long)k * g.NV + d] = a[k];
-            cdd[(long long)k * g.NV + d] = cn[k];
+                for (int m = 0; m < 7; ++m)
+                    if (s_tf[q + m] && vid(g, x - 3 + i, y - 3 + j, z - 3 + m) < d) e[m] = 100.0;
+#pragma unroll
+            for (int m = 0; m < 7; ++m) {
+                a0 += gp[m] == g0 ? e[m] : 0.0;
+                c0 += gp[m] == g0;
+                a1 += gp[m] == g1 ? e[m] : 0.0;
+                c1 += gp[m] == g1;
+            }
         }
 }
 
@@ -577,12 +668,14 @@ __global__ __launch_bounds__(NT) void k_avg(Dims g, Lists A, const int *wn, cons
     __shared__ int s_gid[HC];
     __shared__ double s_de[HC];
     __shared__ unsigned char s_tf[HC];
+    __shared__ unsigned short s_item[NT * CAP / 2];
+    __shared__ int s_w[NT / 64];
     const int ntx = (g.Lx + TX - 1) / TX, nty = (g.Ly + TY - 1) / TY;
     const int b = blockIdx.x;
     const int bx = b % ntx, by = (b / ntx) % nty, bz = b / (ntx * nty);
     // padded coordinates of the tile's first voxel and of its box
     const int x0 = 3 + bx * TX, y0 = 3 + by * TY, z0 = 3 + bz * TZ;
-    int changed = tprev ? 0 : 1;
+    int changed = tprev ? 0 : 1, reset = 0;
     for (int q = threadIdx.x; q < HC; q += NT) {
         const int hz = q % HZ, hy = (q / HZ) % HY, hx = q / (HZ * HY);
         const int i = x0 - 3 + hx, j = y0 - 3 + hy, m = z0 - 3 + hz;
@@ -596,6 +689,7 @@ __global__ __launch_bounds__(NT) void k_avg(Dims g, Lists A, const int *wn, cons
                 const long long v = vid(g, i, j, m);
                 tf = trig[v];
                 if (tprev && tprev[v] != tf) changed = 1;
+                if (tf) reset = 1;
             }
         }
         s_gid[q] = gg;
@@ -603,15 +697,43 @@ __global__ __launch_bounds__(NT) void k_avg(Dims g, Lists A, const int *wn, cons
         s_tf[q] = (unsigned char)tf;
     }
     if (!__syncthreads_or(changed)) return;
-    const int tz = threadIdx.x % TZ, ty = (threadIdx.x / TZ) % TY, tx = threadIdx.x / (TZ * TY);
-    const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
-    if (!interior(g, x, y, z)) return;
-    const long long d = vid(g, x, y, z);
-    const int n = wn[d];
-    if (!n) return;
-    const long long c = cix(g, x, y, z);
-    if (n <= 4) avg_box<4>(g, A, c, d, n, spos[d], sg[d], tx, ty, tz, x, y, z, s_gid, s_de, s_tf, avg, cdd);
-    else avg_box<CAP>(g, A, c, d, n, spos[d], sg[d], tx, ty, tz, x, y, z, s_gid, s_de, s_tf, avg, cdd);
+    reset = __syncthreads_or(reset);
+    // Work items: a voxel's list two entries at a time, counted over the tile
+    // and dealt to the threads.  (One thread per voxel with four entries each
+    // paid for four in every wave that had an active voxel, though two in
+    // three voxels are active, with 2.4 entries on average: 700 us per launch
+    // at 128^3 against 242.)
+    int n = 0;
+    {
+        const int tz = threadIdx.x % TZ, ty = (threadIdx.x / TZ) % TY, tx = threadIdx.x / (TZ * TY);
+        if (interior(g, x0 + tx, y0 + ty, z0 + tz)) n = wn[vid(g, x0 + tx, y0 + ty, z0 + tz)];
+    }
+    int total;
+    const int o = block_prefix((n + 1) / 2, s_w, total);
+    for (int k = 0; 2 * k < n; k++) s_item[o + k] = (unsigned short)(threadIdx.x + NT * k);
+    __syncthreads();
+    for (int t = threadIdx.x; t < total; t += NT) {
+        const int it = s_item[t], vx = it % NT, k = 2 * (it / NT);
+        const int tz = vx % TZ, ty = (vx / TZ) % TY, tx = vx / (TZ * TY);
+        const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
+        const long long d = vid(g, x, y, z), c = cix(g, x, y, z);
+        const int p = spos[d], s = sg[d];
+        const bool two = k + 1 < wn[d];
+        int g0, g1 = NO_GRAIN; // (matches no grain, nor the -1 of cells outside the grid)
+        double v, a0, a1;
+        int c0, c1;
+        entry(g, A, c, k, p, s, g0, v);
+        if (two) entry(g, A, c, k + 1, p, s, g1, v);
+        const int q0 = (tx * HY + ty) * HZ + tz;
+        if (reset) avg_pair<true>(g, s_gid, s_de, s_tf, q0, x, y, z, d, g0, g1, a0, a1, c0, c1);
+        else avg_pair<false>(g, s_gid, s_de, s_tf, q0, x, y, z, d, g0, g1, a0, a1, c0, c1);
+        avg[(long long)k * g.NV + d] = a0;
+        cdd[(long long)k * g.NV + d] = c0;
+        if (two) {
+            avg[(long long)(k + 1) * g.NV + d] = a1;
+            cdd[(long long)(k + 1) * g.NV + d] = c1;
+        }
+    }
 }
 
 __device__ inline double writer_value(const Dims &g, const double *avg, const int *cdd, int ref)
@@ -623,34 +745,90 @@ __device__ inline double writer_value(const Dims &g, const double *avg, const in
 }
 
 // rho_avg[gr-1] at voxel d's turn: the last writer of grain gr at or before
-// d, searched in the grain's own run [gfirst, gend) of the sorted keys (a
-// search over all keys takes ~21 dependent loads at 128^3, the grain's run
-// ~13)
-__device__ inline double rho_at(const Dims &g, const unsigned long long *keys, const long long *gfirst,
-                                const long long *gend, const int *refs, const double *avg, const int *cdd,
-                                const double *rho_in, int gr, long long d)
+// d as an index into refs, or -1, searched in the grain's own run [gfirst,
+// gend) of the sorted references
+__device__ inline long long last_writer(const int *refs, const long long *gfirst, const long long *gend, int gr,
+                                        long long d)
 {
-    const unsigned long long key = (unsigned long long)(gr - 1) * (unsigned long long)g.NV + (unsigned long long)d;
+    const int key = (int)(d * CAP) + (CAP - 1); // the references of voxels up to d
     const long long lo0 = gfirst[gr - 1];
-    long long lo = lo0, hi = gend[gr - 1]; // first index of the run with keys[i] > key
-    while (lo < hi) {
-        const long long mid = (lo + hi) >> 1;
-        if (keys[mid] <= key) lo = mid + 1;
-        else hi = mid;
+    long long lo = lo0, hi = gend[gr - 1]; // first index of the run with refs[i] > key
+    // eight parts a step: seven independent probes per trip to memory instead
+    // of one (a run of 12 600 writers takes 5 trips; halving it took 14)
+    while (hi - lo >= 8) {
+        const long long w = (hi - lo) >> 3;
+        int below = 0;
+#pragma unroll
+        for (int i = 1; i < 8; i++) below += refs[lo + i * w - 1] <= key;
+        const long long b = lo + below * w;
+        if (below < 7) hi = b + w;
+        lo = b;
     }
-    if (lo > lo0) return writer_value(g, avg, cdd, refs[lo - 1]);
-    return rho_in[gr - 1];
+    {
+        int below = 0;
+        const long long w = hi - lo;
+#pragma unroll
+        for (int i = 0; i < 7; i++) below += i < w && refs[i < w ? lo + i : lo0] <= key;
+        lo += below;
+    }
+    return lo > lo0 ? lo - 1 : -1;
+}
+
+// The writer each candidate grain of each update-branch voxel reads rho_avg
+// from: its reference (voxel * CAP + entry), -1 for the value before the
+// sweep.  A grain in the voxel's own list reads the voxel's own write (the
+// last such entry), any other the last earlier writer's.  The writers are
+// the same in every pass of the reset fixed point, so this runs once per
+// substep, as a kernel of its own: it is one chain of dependent loads per
+// candidate, which needs all the wavefronts a CU holds, not the three
+// workgroups that k_update's lists leave room for.
+__global__ __launch_bounds__(NT) void k_rho(Dims g, Lists A, const int *gcnt, const int *gidx, const int *nn,
+                                            const int *spos, const int *sg, const long long *gfirst,
+                                            const long long *gend, const int *refs, int n_rho, int *gref)
+{
+    constexpr int OWN = 4;
+    for (long long d = blockIdx.x * (long long)NT + threadIdx.x; d < g.NV; d += (long long)gridDim.x * NT) {
+        const int n = nn[d];
+        if (n <= 1) continue;
+        int x, y, z;
+        vox(g, d, x, y, z);
+        const long long c = cix(g, x, y, z);
+        const int nG = gcnt[d], p = spos[d], s = sg[d];
+        int own[OWN];
+#pragma unroll
+        for (int k = 0; k < OWN; k++) own[k] = A.idx[(long long)k * g.NC + c];
+        for (int it = 0; it < nG; it++) {
+            const int gr = gidx[(long long)it * g.NV + d];
+            int ref = -1;
+            if (gr >= 1 && gr <= n_rho) { // (k_update reports the others)
+                int k0 = -1;
+#pragma unroll
+                for (int k = 0; k < OWN; k++)
+                    if (k < n && k != p && own[k] == gr) k0 = k;
+                for (int k = OWN; k < n; k++)
+                    if (k != p && A.idx[(long long)k * g.NC + c] == gr) k0 = k;
+                if (p >= 0 && s == gr && p > k0) k0 = p;
+                if (k0 >= 0) {
+                    ref = (int)(d * CAP + k0);
+                } else {
+                    const long long w = last_writer(refs, gfirst, gend, gr, d);
+                    if (w >= 0) ref = refs[w];
+                }
+            }
+            gref[(long long)it * g.NV + d] = ref;
+        }
+    }
 }
 
 // each grain's run [gfirst, gend) in the sorted writer keys (both cleared to
 // 0 first: an empty run for grains without writers)
-__global__ __launch_bounds__(NT) void k_grange(const unsigned long long *keys, long long nw, long long NV,
-                                               long long *gfirst, long long *gend)
+__global__ __launch_bounds__(NT) void k_grange(const unsigned *keys, long long nw, long long *gfirst,
+                                               long long *gend)
 {
     for (long long i = blockIdx.x * (long long)NT + threadIdx.x; i < nw; i += (long long)gridDim.x * NT) {
-        const unsigned long long gr = keys[i] / (unsigned long long)NV;
-        if (i == 0 || keys[i - 1] / (unsigned long long)NV != gr) gfirst[gr] = i;
-        if (i + 1 == nw || keys[i + 1] / (unsigned long long)NV != gr) gend[gr] = i + 1;
+        const unsigned gr = keys[i];
+        if (i == 0 || keys[i - 1] != gr) gfirst[gr] = i;
+        if (i + 1 == nw || keys[i + 1] != gr) gend[gr] = i + 1;
     }
 }
 
@@ -666,93 +844,164 @@ struct Coef {
 // not match the arguments: center_up_front, center_down_front,
 // center_up_back, center_down_back, left_down, left_up, left_front,
 // left_back, right_up, right_back, right_down, right_front.
-__constant__ int LAPQ[18][3] = {{1, 0, 0},   {-1, 0, 0},  {0, 1, 0},   {0, -1, 0}, {0, 0, 1},   {0, 0, -1},
-                                {0, -1, 1},  {0, -1, -1}, {0, 1, 1},   {0, 1, -1}, {-1, 0, -1}, {-1, 0, 1},
-                                {-1, -1, 0}, {-1, 1, 0},  {1, 0, 1},   {1, 1, 0},  {1, 0, -1},  {1, -1, 0}};
+constexpr int LAPQ[18][3] = {{1, 0, 0},   {-1, 0, 0},  {0, 1, 0},   {0, -1, 0}, {0, 0, 1},   {0, 0, -1},
+                             {0, -1, 1},  {0, -1, -1}, {0, 1, 1},   {0, 1, -1}, {-1, 0, -1}, {-1, 0, 1},
+                             {-1, -1, 0}, {-1, 1, 0},  {1, 0, 1},   {1, 1, 0},  {1, 0, -1},  {1, -1, 0}};
 
-// the voxel update of src/pf_xrx.c:1034-1246 into the temp lists B
+// The voxel update of src/pf_xrx.c:1034-1246 into the temp lists B.  Work
+// items: the candidate grains of the tile's update-branch voxels, dealt to
+// the threads (a voxel per thread ran every wave to its longest candidate
+// list, 19 list searches each); the results of a run of voxels wait in LDS
+// (UPD_RES at most) until their voxels put them into the new lists in order.
+// Bound by the latency of its loads: 640 us per launch at 128^3 before (with the
+// last-writer searches, now in k_rho, once per substep), 337 now.
+constexpr int UPD_RES = 768, UPD_G = 4; // (three workgroups of 53 KB per CU)
+static_assert(UPD_RES >= CAP, "a voxel's candidates fit one run");
+
 __global__ __launch_bounds__(NT) void k_update(Dims g, Lists A, Lists B, Coef P, const int *gcnt, const int *gidx, const int *nn,
-                         const int *spos, const int *sg, const double *avg, const int *cdd,
-                         const unsigned long long *keys, const long long *gfirst, const long long *gend,
-                         const int *refs, const double *rho_in, int *trig_out, int *err)
+                         const double *avg, const int *cdd, const int *gref, const double *rho_in,
+                         int *trig_out, int *err)
 {
     __shared__ ListTile T;
+    __shared__ double s_res[UPD_RES], s_sum[3][NT];
+    __shared__ unsigned short s_item[UPD_RES];
+    __shared__ int s_g[UPD_G][NT]; // the first candidates
+    __shared__ int s_off[NT + 1], s_w[NT / 64];
+    __shared__ unsigned char s_new[NT], s_trig[NT];
     int x0, y0, z0;
     tile_origin(g, blockIdx.x, x0, y0, z0);
-    load_lists(T, g, A, x0, y0, z0);
-    __syncthreads();
-    const int tz = threadIdx.x % TZ, ty = (threadIdx.x / TZ) % TY, tx = threadIdx.x / (TZ * TY);
+    const int tid = threadIdx.x;
+    const int tz = tid % TZ, ty = (tid / TZ) % TY, tx = tid / (TZ * TY);
     const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
-    if (interior(g, x, y, z)) {
-        const long long d = vid(g, x, y, z);
-        const long long c = cix(g, x, y, z);
-        const int q0 = tq(tx, ty, tz, 0, 0, 0);
-        const int NN = nn[d];
-        const int nG = gcnt[d];
-        Build t(B, g.NC, c);
-        bool ok = true;
-        int trig = 0;
+    const bool in = interior(g, x, y, z);
+    const long long d = in ? vid(g, x, y, z) : 0, c = in ? cix(g, x, y, z) : 0;
+    const int NN = in ? nn[d] : 0, nG = in ? gcnt[d] : 0;
+    load_lists(T, g, A, x0, y0, z0);
+    // the first sums and counts of an update-branch voxel in one trip to
+    // memory, whatever its counts (the arrays hold CAP of each)
+    constexpr int PRE = 3;
+    double pa[PRE];
+    int pc[PRE];
+#pragma unroll
+    for (int k = 0; k < PRE; k++) {
+        pa[k] = 0.0;
+        pc[k] = 0;
         if (NN > 1) {
-            double sum_rex = 0.0, sum1 = 0.0, h_phi_def = 0.0;
-            for (int k = 0; k < NN; k++) {
-                const int cn = cdd[(long long)k * g.NV + d];
-                const double a = avg[(long long)k * g.NV + d];
-                if (cn > 0 && a > 0.0) {
-                    int gr;
-                    double v;
-                    entry(g, A, c, k, spos[d], sg[d], gr, v);
-                    sum_rex += v * v;
-                    sum1 += v * v * v * (10.0 - 15.0 * v + 6.0 * v * v);
-                    h_phi_def += (v * v * v * (10.0 - 15.0 * v + 6.0 * v * v)) * (a / cn);
-                }
+            pa[k] = avg[(long long)k * g.NV + d];
+            pc[k] = cdd[(long long)k * g.NV + d];
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < UPD_G; it++)
+        if (it < nG) s_g[it][tid] = gidx[(long long)it * g.NV + d];
+    __syncthreads();
+    const int qc = tq(tx, ty, tz, 0, 0, 0);
+    if (NN > 1) {
+        double sum_rex = 0.0, sum1 = 0.0, h_phi_def = 0.0;
+        auto term = [&](int cn, double a, double v) {
+            if (cn > 0 && a > 0.0) {
+                sum_rex += v * v;
+                sum1 += v * v * v * (10.0 - 15.0 * v + 6.0 * v * v);
+                h_phi_def += (v * v * v * (10.0 - 15.0 * v + 6.0 * v * v)) * (a / cn);
             }
-            int count = 0;
-            for (int it = 0; it < nG; it++)
-                if (gidx[(long long)it * g.NV + d] > P.init_gid) count++;
-            for (int it = 0; it < nG; it++) {
-                const int index = gidx[(long long)it * g.NV + d];
-                if (index < 1 || index > P.n_rho) {
-                    atomicOr(err, PFE_GRAIN);
-                    break;
-                }
-                const double s = lookup_t(T, g, A, q0, c, index);
-                const double h_phi = s * s * s * (10.0 - 15.0 * s + 6.0 * s * s);
-                const double dh_phi = s * s * (30.0 - 60.0 * s + 30.0 * s * s);
-                const double center_rex = s;
+        };
+        // an entry's value at its turn is its start value, an appended one's 0
+        // (what a lookup of another grain returns: the small last value, or 0)
+        const int meta = T.meta[qc];
+        auto value = [&](int k) {
+            if (meta < 0) return k < A.cnt[c] ? A.val[(long long)k * g.NC + c] : 0.0;
+            return k < (meta >> 16) ? T.val[(meta & 0xffff) + k] : T.other[qc];
+        };
+#pragma unroll
+        for (int k = 0; k < PRE; k++)
+            if (k < NN) term(pc[k], pa[k], value(k));
+        for (int k = PRE; k < NN; k++) term(cdd[(long long)k * g.NV + d], avg[(long long)k * g.NV + d], value(k));
+        int count = 0;
+        for (int it = 0; it < nG; it++)
+            if ((it < UPD_G ? s_g[it][tid] : gidx[(long long)it * g.NV + d]) > P.init_gid) count++;
+        s_sum[0][tid] = sum_rex;
+        s_sum[1][tid] = sum1;
+        s_sum[2][tid] = h_phi_def;
+        s_new[tid] = count > 0;
+    }
+    s_trig[tid] = 0;
+    int total;
+    const int off = block_prefix(NN > 1 ? nG : 0, s_w, total);
+    s_off[tid] = off;
+    if (tid == 0) s_off[NT] = total;
+    __syncthreads();
+    for (int v0 = 0; v0 < NT;) {
+        // the run of voxels v0 .. v1-1 whose results fit (nearly always all)
+        const int o0 = s_off[v0];
+        int v1 = NT;
+        while (s_off[v1] - o0 > UPD_RES) v1--;
+        const bool mine = tid >= v0 && tid < v1;
+        if (mine && NN > 1)
+            for (int it = 0; it < nG; it++) s_item[off - o0 + it] = (unsigned short)(tid + NT * it);
+        __syncthreads();
+        for (int t = tid; t < s_off[v1] - o0; t += NT) {
+            const int vx = s_item[t] % NT, it = s_item[t] / NT;
+            const int uz = vx % TZ, uy = (vx / TZ) % TY, ux = vx / (TZ * TY);
+            const int xx = x0 + ux, yy = y0 + uy, zz = z0 + uz;
+            const long long u = vid(g, xx, yy, zz);
+            const int index = it < UPD_G ? s_g[it][vx] : gidx[(long long)it * g.NV + u];
+            const int ref = gref[(long long)it * g.NV + u];
+            double res = 0.0; // (not above 1e-4: no entry)
+            if (index < 1 || index > P.n_rho) {
+                atomicOr(err, PFE_GRAIN);
+            } else {
+                const int q0 = tq(ux, uy, uz, 0, 0, 0);
                 // laplacian() (src/pf_xrx.c:6-9): faces summed in the call's
                 // order, edges in the order its permuted parameter names sum
                 // them (LAPQ)
+                const double s = lookup_t(T, g, A, q0, cix(g, xx, yy, zz), index);
                 double f = 0.0, e = 0.0;
-#pragma unroll 1
+#pragma unroll
                 for (int q = 0; q < 18; q++) {
                     const int dx = LAPQ[q][0], dy = LAPQ[q][1], dz = LAPQ[q][2];
-                    const double v =
-                        lookup_t(T, g, A, tq(tx, ty, tz, dx, dy, dz), cix(g, x + dx, y + dy, z + dz), index);
+                    const double v = lookup_t(T, g, A, q0 + (dx * LY + dy) * LZ + dz,
+                                              cix(g, xx + dx, yy + dy, zz + dz), index);
                     if (q < 6) f = q == 0 ? v : f + v;
                     else e = q == 6 ? v : e + v;
                 }
-                const double lap_rex = (0.5 * f + 0.125 * e) - 4.5 * center_rex;
-                const double ra = rho_at(g, keys, gfirst, gend, refs, avg, cdd, rho_in, index, d);
+                const double ra = ref >= 0 ? writer_value(g, avg, cdd, ref) : rho_in[index - 1];
+                const double sum_rex = s_sum[0][vx], sum1 = s_sum[1][vx], h_phi_def = s_sum[2][vx];
+                const double h_phi = s * s * s * (10.0 - 15.0 * s + 6.0 * s * s);
+                const double dh_phi = s * s * (30.0 - 60.0 * s + 30.0 * s * s);
+                const double cc = s;
+                const double lap_rex = (0.5 * f + 0.125 * e) - 4.5 * cc;
                 if (ra > 0.0) {
-                    const double cc = center_rex;
-                    const double value_rex =
-                        cc - P.M_coeff * (P.m * (cc * cc * cc - cc + 3.0 * cc * (sum_rex - cc * cc)) -
-                                          P.kappa * lap_rex +
-                                          P.E_disl * dh_phi * ((sum1 - h_phi) * ra - (h_phi_def - h_phi * ra)) /
-                                              (sum1 * sum1));
-                    if (count > 0 && index > P.init_gid && cc < 0.5 && value_rex > 0.5) trig = 1;
-                    if (value_rex > 1E-04) ok = ok && t.put(index, value_rex);
+                    res = cc - P.M_coeff * (P.m * (cc * cc * cc - cc + 3.0 * cc * (sum_rex - cc * cc)) -
+                                            P.kappa * lap_rex +
+                                            P.E_disl * dh_phi * ((sum1 - h_phi) * ra - (h_phi_def - h_phi * ra)) /
+                                                (sum1 * sum1));
+                    if (s_new[vx] && index > P.init_gid && cc < 0.5 && res > 0.5) s_trig[vx] = 1;
                 }
             }
-        } else if (NN == 1) {
-            for (int it = 0; it < nG; it++) {
-                const int index = gidx[(long long)it * g.NV + d];
-                ok = ok && t.put(index, lookup_t(T, g, A, q0, c, index));
-            }
+            s_res[t] = res;
         }
-        if (!ok) atomicOr(err, PFE_CAP);
-        t.finish();
-        trig_out[d] = trig;
+        __syncthreads();
+        if (mine && in) {
+            Build t(B, g.NC, c);
+            bool ok = true;
+            if (NN > 1) {
+                for (int it = 0; it < nG; it++) {
+                    const double v = s_res[off - o0 + it];
+                    if (v > 1E-04)
+                        ok = ok && t.put(it < UPD_G ? s_g[it][tid] : gidx[(long long)it * g.NV + d], v);
+                }
+            } else if (NN == 1) {
+                for (int it = 0; it < nG; it++) {
+                    const int index = it < UPD_G ? s_g[it][tid] : gidx[(long long)it * g.NV + d];
+                    ok = ok && t.put(index, lookup_t(T, g, A, qc, c, index));
+                }
+            }
+            if (!ok) atomicOr(err, PFE_CAP);
+            t.finish();
+            trig_out[d] = s_trig[tid];
+        }
+        __syncthreads();
+        v0 = v1;
     }
 }
 
@@ -764,7 +1013,7 @@ __global__ __launch_bounds__(NT) void k_diff(long long n, const int *a, const in
 
 // after the sweep: the resets to 100 and rho_avg of each written grain (its
 // last writer)
-__global__ __launch_bounds__(NT) void k_finish(Dims g, const int *trig, double *defeng, const unsigned long long *keys, const int *refs,
+__global__ __launch_bounds__(NT) void k_finish(Dims g, const int *trig, double *defeng, const unsigned *keys, const int *refs,
                          long long nw, const double *avg, const int *cdd, double *rho)
 {
     for (long long d = blockIdx.x * (long long)NT + threadIdx.x; d < g.NV; d += (long long)gridDim.x * NT) {
@@ -775,8 +1024,8 @@ __global__ __launch_bounds__(NT) void k_finish(Dims g, const int *trig, double *
         }
     }
     for (long long i = blockIdx.x * (long long)NT + threadIdx.x; i < nw; i += (long long)gridDim.x * NT) {
-        const unsigned long long gr = keys[i] / (unsigned long long)g.NV;
-        if (i + 1 == nw || keys[i + 1] / (unsigned long long)g.NV != gr) rho[gr] = writer_value(g, avg, cdd, refs[i]);
+        const unsigned gr = keys[i];
+        if (i + 1 == nw || keys[i + 1] != gr) rho[gr] = writer_value(g, avg, cdd, refs[i]);
     }
 }
 
@@ -919,15 +1168,15 @@ struct evpgpu_pf {
     int *gcnt, *gidx, *act, *emask, *nn, *spos, *sg, *wn, *trig0, *trig1, *gid_new;
     long long *woff;
     double *avg;
-    int *cdd;
+    int *cdd, *gref;
     double *rho_in, *rho_out;
     long long *gfirst, *gend; // each grain's run in the sorted writer keys
-    unsigned long long *keys[2];
+    unsigned *keys[2];
     int *refs[2];
     long long wcap;
     void *tmp;
     size_t tmp_bytes;
-    int *flags; // [0] error bits, [1] changed, [2] voxels on the update branch
+    int *flags; // [0] error bits, [1] changed
     int *h_flags;
     long long *h_total;
     int *h_last;
@@ -1012,23 +1261,26 @@ int substep(evpgpu_pf *p, const Coef &P)
         if (p->h_flags[0]) return pf_err(p->h_flags[0]);
         if (!p->h_flags[1]) break;
     }
-    if ((st = clear_flag(p, 2))) return st;
     hipLaunchKernelGGL(k_slot, dim3(gv), dim3(NT), 0, s, g, p->A, p->gcnt, p->gidx, p->act, p->nn, p->spos, p->sg,
-                       p->wn, p->flags + 2, p->flags);
-    // writer offsets
+                       p->wn, p->flags);
+    // writer offsets and the number of voxels on the update branch (an atomic
+    // counter in k_slot took most of its time)
     size_t need = 0;
-    EVP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, need, p->wn, p->woff, g.NV, s));
+    hipcub::TransformInputIterator<long long, WriterScan, const int *> win(p->wn, WriterScan());
+    EVP_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, need, win, p->woff, g.NV, s));
     if ((st = ensure_tmp(p, need))) return st;
-    EVP_CHECK(hipcub::DeviceScan::ExclusiveSum(p->tmp, need, p->wn, p->woff, g.NV, s));
+    EVP_CHECK(hipcub::DeviceScan::ExclusiveSum(p->tmp, need, win, p->woff, g.NV, s));
     EVP_CHECK(hipMemcpyAsync(p->h_total, p->woff + g.NV - 1, sizeof(long long), hipMemcpyDeviceToHost, s));
     EVP_CHECK(hipMemcpyAsync(p->h_last, p->wn + g.NV - 1, sizeof(int), hipMemcpyDeviceToHost, s));
     EVP_CHECK(hipStreamSynchronize(s));
-    const long long nw = p->h_total[0] + p->h_last[0];
+    const long long tot = p->h_total[0] + WriterScan()(p->h_last[0]);
+    const long long nw = tot & (SCAN_LOW - 1);
+    p->st.updated += tot >> 32;
     if ((st = ensure_writers(p, nw))) return st;
     hipLaunchKernelGGL(k_emit, dim3(gv), dim3(NT), 0, s, g, p->A, p->nn, p->spos, p->sg, p->wn, p->woff,
                        p->keys[0], p->refs[0], p->n_rho, p->flags);
     int end_bit = 1;
-    while (end_bit < 64 && ((unsigned long long)p->n_rho * (unsigned long long)g.NV) >> end_bit) end_bit++;
+    while (end_bit < 32 && (unsigned)(p->n_rho - 1) >> end_bit) end_bit++;
     if (nw > 0) {
         need = 0;
         EVP_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, need, p->keys[0], p->keys[1], p->refs[0], p->refs[1],
@@ -1041,8 +1293,11 @@ int substep(evpgpu_pf *p, const Coef &P)
     hipLaunchKernelGGL(k_clear, dim3(grid_for(2LL * p->n_rho)), dim3(NT), 0, s, 2LL * p->n_rho, (int *)p->gfirst);
     hipLaunchKernelGGL(k_clear, dim3(grid_for(2LL * p->n_rho)), dim3(NT), 0, s, 2LL * p->n_rho, (int *)p->gend);
     if (nw > 0)
-        hipLaunchKernelGGL(k_grange, dim3(grid_for(nw)), dim3(NT), 0, s, (const unsigned long long *)p->keys[1], nw,
-                           g.NV, p->gfirst, p->gend);
+        hipLaunchKernelGGL(k_grange, dim3(grid_for(nw)), dim3(NT), 0, s, (const unsigned *)p->keys[1], nw,
+                           p->gfirst, p->gend);
+    if (nw > 0)
+        hipLaunchKernelGGL(k_rho, dim3(gv), dim3(NT), 0, s, g, p->A, p->gcnt, p->gidx, p->nn, p->spos, p->sg,
+                           p->gfirst, p->gend, p->refs[1], p->n_rho, p->gref);
     // trigger fixed point; tout holds the resets the previous pass used
     int *tin = p->trig0, *tout = p->trig1;
     hipLaunchKernelGGL(k_clear, dim3(gv), dim3(NT), 0, s, g.NV, tin);
@@ -1052,9 +1307,8 @@ int substep(evpgpu_pf *p, const Coef &P)
         hipLaunchKernelGGL(k_avg, dim3(tiles), dim3(NT), 0, s, g, p->A, p->wn, p->spos, p->sg, p->gid, p->defeng,
                            tin, pass ? tout : (const int *)nullptr, p->avg, p->cdd);
         EVP_CHECK(hipEventRecord(p->eu[1], s));
-        hipLaunchKernelGGL(k_update, dim3(tiles), dim3(NT), 0, s, g, p->A, p->B, P, p->gcnt, p->gidx, p->nn, p->spos,
-                           p->sg, p->avg, p->cdd, p->keys[1], p->gfirst, p->gend, p->refs[1], p->rho_in, tout,
-                           p->flags);
+        hipLaunchKernelGGL(k_update, dim3(tiles), dim3(NT), 0, s, g, p->A, p->B, P, p->gcnt, p->gidx, p->nn, p->avg,
+                           p->cdd, p->gref, p->rho_in, tout, p->flags);
         EVP_CHECK(hipEventRecord(p->eu[2], s));
         if ((st = clear_flag(p, 1))) return st;
         hipLaunchKernelGGL(k_diff, dim3(gv), dim3(NT), 0, s, g.NV, tin, tout, p->flags + 1);
@@ -1085,7 +1339,6 @@ int substep(evpgpu_pf *p, const Coef &P)
     hipLaunchKernelGGL(k_mesh, dim3(gc), dim3(NT), 0, s, g, p->defeng, p->gid);
     if ((st = read_flags(p))) return st;
     if (p->h_flags[0]) return pf_err(p->h_flags[0]);
-    p->st.updated += p->h_flags[2];
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
@@ -1142,7 +1395,7 @@ extern "C" int evpgpu_pf_create(evpgpu_pf **out, int Lx, int Ly, int Lz, int n_r
     bad |= dalloc(&p->emask, g.NV);
     bad |= dalloc(&p->spos, g.NV) | dalloc(&p->sg, g.NV) | dalloc(&p->wn, g.NV) | dalloc(&p->woff, g.NV);
     bad |= dalloc(&p->trig0, g.NV) | dalloc(&p->trig1, g.NV) | dalloc(&p->gid_new, g.NV);
-    bad |= dalloc(&p->avg, g.NV * CAP) | dalloc(&p->cdd, g.NV * CAP);
+    bad |= dalloc(&p->avg, g.NV * CAP) | dalloc(&p->cdd, g.NV * CAP) | dalloc(&p->gref, g.NV * CAP);
     bad |= dalloc(&p->rho_in, n_rho_avg) | dalloc(&p->flags, 3);
     bad |= dalloc(&p->gfirst, n_rho_avg) | dalloc(&p->gend, n_rho_avg);
     bad |= hipHostMalloc((void **)&p->h_flags, 3 * sizeof(int), 0) != hipSuccess;
@@ -1179,7 +1432,7 @@ extern "C" int evpgpu_pf_destroy(evpgpu_pf *p)
     }
     void *dev[] = {p->defeng, p->gid, p->gcnt, p->gidx, p->act, p->emask, p->nn,    p->spos,    p->sg,      p->wn,
                    p->woff,   p->trig0, p->trig1, p->gid_new, p->avg, p->cdd, p->rho_in, p->flags, p->keys[0],
-                   p->keys[1], p->refs[0], p->refs[1], p->tmp, p->gfirst, p->gend};
+                   p->keys[1], p->refs[0], p->refs[1], p->tmp, p->gfirst, p->gend, p->gref};
     for (void *q : dev) (void)hipFree(q);
     if (p->h_flags) (void)hipHostFree(p->h_flags);
     if (p->h_total) (void)hipHostFree(p->h_total);
