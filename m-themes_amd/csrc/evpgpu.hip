@@ -747,21 +747,17 @@ int evpgpu_download_state(evpgpu_ctx *c, double *sig6, double *dg9, double *eps6
     D2H(gamdot12, c->gamdot, 12 * N);
 #undef D2H
     if (dg9) {
-        double *E = (double *)malloc(sizeof(double) * 9 * N), *W = E + 6 * N;
-        if (hipMemcpy(E, c->E, sizeof(double) * 6 * N, hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy(W, c->W, sizeof(double) * 3 * N, hipMemcpyDeviceToHost) != hipSuccess) {
-            free(E);
-            return EVPGPU_ERR_HIP;
-        }
-        for (long long v = 0; v < N; v++) {
-            double e[6], w[3];
-            for (int k = 0; k < 6; k++) e[k] = E[k * N + v];
-            for (int k = 0; k < 3; k++) w[k] = W[k * N + v];
-            double g[9] = {e[0], e[5] + w[2], e[4] + w[1], e[5] - w[2], e[1],
-                           e[3] + w[0], e[4] - w[1], e[3] - w[0], e[2]};
-            for (int k = 0; k < 9; k++) dg9[k * N + v] = g[k];
-        }
-        free(E);
+        // the full tensor from its symmetric and antisymmetric parts: the
+        // diagonal is E's, the six others are formed on the device in the
+        // spectrum's buffer (free between increments)
+        double *off = (double *)c->spec;
+        int st = disgrad_offdiag_launch(c, off);
+        if (st) return st;
+        EVP_CHECK(hipStreamSynchronize(c->stream));
+        for (int k = 0; k < 3; k++)
+            EVP_CHECK(hipMemcpy(dg9 + 4 * k * N, c->E + k * N, sizeof(double) * N, hipMemcpyDeviceToHost));
+        EVP_CHECK(hipMemcpy(dg9 + 1 * N, off, sizeof(double) * 3 * N, hipMemcpyDeviceToHost));
+        EVP_CHECK(hipMemcpy(dg9 + 5 * N, off + 3 * N, sizeof(double) * 3 * N, hipMemcpyDeviceToHost));
     }
     return EVPGPU_OK;
 }

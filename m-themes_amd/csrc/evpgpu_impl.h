@@ -290,6 +290,8 @@ int ctl_iter_launch(evpgpu_ctx *c, int nblk);
 // fields.hip
 int prologue_launch(evpgpu_ctx *c, const double *dE6, int creep, const double *macro_sym6);
 int antisym_add_launch(evpgpu_ctx *c, const double *dW3);
+// DisGrad's components 01 02 10 12 20 21 (6N)
+int disgrad_offdiag_launch(evpgpu_ctx *c, double *out6);
 int epilogue_launch(evpgpu_ctx *c, const EpilogueParams &P, double *partials, int *nblk);
 int fill_zero(evpgpu_ctx *c, double *p, long long n);
 int fill_zero_int(evpgpu_ctx *c, int *p, long long n);

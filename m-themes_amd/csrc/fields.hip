@@ -71,6 +71,23 @@ __global__ void k_prologue(double *E, double *W, long long N, double d0, double 
     for (int c = 0; c < 3; c++) W[c * N + v] = creep ? w[c] : W[c * N + v] + w[c];
 }
 
+// the off-diagonal components of DisGrad = E + W, row-major 01 02 10 | 12 20 21
+// (formed on the host from copies of E and W they took 2.2 ms more at 64^3)
+__global__ void k_disgrad_offdiag(const double *__restrict__ E, const double *__restrict__ W,
+                                  double *__restrict__ out, long long N)
+{
+    const long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= N) return;
+    const double e3 = E[3 * N + v], e4 = E[4 * N + v], e5 = E[5 * N + v];
+    const double w0 = W[v], w1 = W[N + v], w2 = W[2 * N + v];
+    out[v] = e5 + w2;
+    out[N + v] = e4 + w1;
+    out[2 * N + v] = e5 - w2;
+    out[3 * N + v] = e3 + w0;
+    out[4 * N + v] = e4 - w1;
+    out[5 * N + v] = e3 - w0;
+}
+
 // dW (3 comps, fluctuation part from the inverse FFT, in rw) + uniform part m
 // -> W += dW ; rw keeps dW for the epilogue
 __global__ void k_antisym_add(double *W, double *rw, long long N, double m0, double m1, double m2)
@@ -291,6 +308,13 @@ int antisym_add_launch(evpgpu_ctx *c, const double *m3)
 {
     hipLaunchKernelGGL(k_antisym_add, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0, c->stream, c->W,
                        c->rwork, c->N, m3[0], m3[1], m3[2]);
+    return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
+}
+
+int disgrad_offdiag_launch(evpgpu_ctx *c, double *out6)
+{
+    hipLaunchKernelGGL(k_disgrad_offdiag, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0, c->stream,
+                       (const double *)c->E, (const double *)c->W, out6, c->N);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
