@@ -841,13 +841,17 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
 int reduce_partials(evpgpu_ctx *c, const double *partials, int nblk, int nval, double *out, const int *status)
 {
     if (nval > RED_MAXV) return EVPGPU_ERR_ARG;
-    int g = nblk < REDUCE_G ? nblk : REDUCE_G;
-    int per = (nblk + g - 1) / g;
-    g = (nblk + per - 1) / per;
-    hipLaunchKernelGGL(k_reduce_rows, dim3(g), dim3(256), 0, c->stream, partials, nblk, nval, per, c->red2,
-                       (const int *)nullptr, (const int *)nullptr);
-    hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(256), 0, c->stream, (const double *)c->red2, g, nval, g,
-                       out, status, (const int *)nullptr);
+    // (up to REDUCE_G rows the first stage would only copy them)
+    int g = nblk;
+    if (nblk > REDUCE_G) {
+        const int per = (nblk + REDUCE_G - 1) / REDUCE_G;
+        g = (nblk + per - 1) / per;
+        hipLaunchKernelGGL(k_reduce_rows, dim3(g), dim3(256), 0, c->stream, partials, nblk, nval, per, c->red2,
+                           (const int *)nullptr, (const int *)nullptr);
+        partials = c->red2;
+    }
+    hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(256), 0, c->stream, partials, g, nval, g, out, status,
+                       (const int *)nullptr);
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 
