@@ -305,7 +305,8 @@ int evpgpu_adjoint_record(evpgpu_ctx *ctx, int n_increments, int checkpoint_ever
  * symmetric pair).  grad (2 x EVPGPU_NPARAM) receives dL/d(parameters) of
  * the two phases.  Each increment's adjoint solve is a conjugate-gradient
  * solve to relative residual cg_tol (at most cg_max iterations).  Segments
- * are replayed from the checkpoints; the context is left in the state after
+ * are replayed from the checkpoints (the last one's inputs are still held by
+ * the first reverse pass after a recording); the context is left in the state after
  * the recorded increments. */
 int evpgpu_adjoint_run(evpgpu_ctx *ctx, const double *sig_avg_bar, double cg_tol, int cg_max,
                        double *grad, evpgpu_adjoint_stats *stats);
