@@ -249,11 +249,11 @@ int evpgpu_newton_host(evpgpu_ctx *ctx, int n, const int *phase, const int *orie
 /* The per-voxel stress update of evpgpu_newton_host on caller-owned DEVICE
  * buffers (same layouts, n voxels), allocating nothing: no counterpart in
  * the reference; for callers that cannot allocate device memory (code under
- * HIP graph capture, tight serving loops).  The kernel's scratch (the
- * status word) is a file-scope device array of the library, one per GPU, held
- * until the process ends; n is at most 2^21 (EVPGPU_ERR_SIZE above).  Phase and orientation indices are checked on the
- * device first (EVPGPU_ERR_ARG).  Runs on the context's stream and waits for
- * it.  Calls that overlap on one GPU share the scratch array and race. */
+ * HIP graph capture, tight serving loops).  Its scratch is two words of the
+ * context, so calls on different contexts do not meet; n is at most 2^21
+ * (EVPGPU_ERR_SIZE above).  Phase and orientation indices are checked on the
+ * device first: where one is out of range the update does nothing and the
+ * call returns EVPGPU_ERR_ARG.  Runs on the context's stream and waits for it. */
 #define EVPGPU_NOALLOC_MAX_VOXELS (1 << 21)
 int evpgpu_newton_device_noalloc(evpgpu_ctx *ctx, int n, const int *phase, const int *orient,
                                  const double *sgr, int n_orient, double *sig6,

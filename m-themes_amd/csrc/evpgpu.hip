@@ -479,9 +479,9 @@ int evpgpu_create(evpgpu_ctx **out, int nx, int ny, int nz, int precision)
     if (!st) st = dalloc(&c->partials, 2 * nblk * NRED);
     if (!st) st = dalloc(&c->red, NRED + 1);
     if (!st) st = dalloc(&c->red2, (long long)REDUCE_G * NRED);
-    if (!st) st = dalloc(&c->d_status, 1);
+    if (!st) st = dalloc(&c->d_status, 3); // the loop's word, then the batch update's two
     if (!st && hipHostMalloc((void **)&c->h_red, (NRED + 1) * sizeof(double), 0) != hipSuccess) st = EVPGPU_ERR_NOMEM;
-    if (!st && hipHostMalloc((void **)&c->h_status, sizeof(int), 0) != hipSuccess) st = EVPGPU_ERR_NOMEM;
+    if (!st && hipHostMalloc((void **)&c->h_status, 2 * sizeof(int), 0) != hipSuccess) st = EVPGPU_ERR_NOMEM;
     if (!st && hipMalloc((void **)&c->ctl, sizeof(LoopCtl)) != hipSuccess) st = EVPGPU_ERR_NOMEM;
     if (!st && hipMalloc((void **)&c->ctl_k, sizeof(CtlConst)) != hipSuccess) st = EVPGPU_ERR_NOMEM;
     if (!st && hipHostMalloc((void **)&c->h_ctl, 3 * sizeof(LoopCtl), 0) != hipSuccess) st = EVPGPU_ERR_NOMEM;
