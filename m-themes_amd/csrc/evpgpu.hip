@@ -185,6 +185,39 @@ void update_lam_min(evpgpu_ctx *c)
     c->lam_min = m;
 }
 
+// Places phase p's systems in the order of CUB_U and CUB_V; 0 where they are
+// not the twelve of {111}<110> to rounding.  (A normal or direction that is not
+// of unit length, another family or a system given twice all end here.)
+int cubic_order(NewtonParams &P, int p)
+{
+    if (P.is_gas[p] || P.nsys[p] != EVPGPU_NSYSMX) return 0;
+    const double base[3][2] = {{-1., 1.}, {1., 1.}, {2., 0.}};
+    int seen = 0;
+    for (int s = 0; s < EVPGPU_NSYSMX; s++) {
+        double y[5];
+        for (int j = 0; j < 5; j++) y[j] = P.mx[p][s][j] / cub_scale(j);
+        int place = -1, neg = 0;
+        for (int q = 0; q < 2 * EVPGPU_NSYSMX && place < 0; q++) {
+            const int a = (q / 2) / 4, k = (q / 2) & 3;
+            const double sg = q & 1 ? -1. : 1.;
+            double m[5] = {base[a][0], base[a][1], 0., 0., 0.};
+            m[CUB_U[a]] = k == 0 || k == 2 ? 1. : -1.;
+            m[CUB_V[a]] = k == 0 || k == 3 ? 1. : -1.;
+            int j = 0;
+            while (j < 5 && fabs(y[j] - sg * m[j]) <= 4e-15) j++;
+            if (j == 5) {
+                place = q / 2;
+                neg = q & 1;
+            }
+        }
+        if (place < 0) return 0;
+        seen |= 1 << place;
+        P.cub_sys[p][place] = s;
+        P.cub_neg[p][place] = neg;
+    }
+    return seen == (1 << EVPGPU_NSYSMX) - 1;
+}
+
 NewtonParams newton_params(const evpgpu_ctx *c)
 {
     NewtonParams P;
@@ -227,6 +260,7 @@ NewtonParams newton_params(const evpgpu_ctx *c)
             P.mx[p][s][4] = (n[0] * b[1] + n[1] * b[0]) * RSQ2;
         }
     }
+    for (int p = 0; p < c->nphases; p++) P.cubic[p] = cubic_order(P, p);
     P.c0_lo2 = c->c0_lo2;
     P.c0_hi2 = c->c0_hi2;
     P.crss_sym = c->crss_sym;

@@ -25,6 +25,16 @@ __host__ __device__ constexpr int PK(int i, int j)
     return i <= j ? i * 6 - i * (i - 1) / 2 + (j - i) : j * 6 - j * (j - 1) / 2 + (i - j);
 }
 
+// The twelve Schmid tensors of {111}<110> in the crystal 5-vector basis with
+// component j divided by cub_scale(j): axis 0 has (-1 1 0 u v), axis 1
+// (1 1 v 0 u), axis 2 (2 0 v u 0); place 4 axis + {0, 1, 2, 3} is the system of
+// the signs (u, v) = (+ +), (- -), (+ -), (- +).
+constexpr int CUB_U[3] = {3, 4, 3}, CUB_V[3] = {4, 2, 2}; // components of u and v
+__host__ __device__ constexpr double cub_scale(int j)
+{
+    return j == 1 ? 0.5 : 0.28867513459481288225; // 1/sqrt 12
+}
+
 struct NewtonParams {
     double c0p[21];  // C0 (B-basis), packed upper triangle (PK)
     double dt;
@@ -36,6 +46,9 @@ struct NewtonParams {
     int crss_sym;    // 1: forward and backward CRSS are equal in every voxel
     double bn[2][EVPGPU_NSYSMX][3], bb[2][EVPGPU_NSYSMX][3]; // crystal-axis normals, directions
     double mx[2][EVPGPU_NSYSMX][5]; // Schmid tensors, crystal axes (deviatoric 5-vectors)
+    int cubic[2];    // 1: the phase's systems are the twelve of {111}<110>, below in
+                     // the order of CUB_U and CUB_V
+    int cub_sys[2][EVPGPU_NSYSMX], cub_neg[2][EVPGPU_NSYSMX]; // system of each place, 1: of the other sign
     double s0p[21];  // S0 = C0^-1 (B-basis), packed upper triangle: the Newton step is
                      // solved in S0-scaled form
     double kmin_tolx2; // (0.99 TOLX min over orientations of lambda_min(S0 + S))^2

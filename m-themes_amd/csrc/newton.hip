@@ -16,7 +16,8 @@
 //     upper triangle), and d(edot)/d(sigma) is symmetric, so only upper
 //     triangles are formed;
 //   * rates in the crystal axes, where the Schmid tensors are constants of the
-//     phase (scalar registers), between two 5x5 rotations of the voxel;
+//     phase (0, 1 and 2 of a scaled basis for the cubic family, scalar
+//     registers otherwise), between two 5x5 rotations of the voxel;
 //   * |x|^n by repeated squaring for integral n, 1/CRSS multiplied instead of
 //     divided, fused multiply-adds.
 // A non-positive-definite K returns status 35, the reference's singular-LU
@@ -29,11 +30,13 @@
 // constants arrive by scalar loads.  The 12 Schmid tensors in sample axes, as
 // an LDS slab of 30 KB per wave, held the kernel at one wave per SIMD, with
 // 5 LDS reads per system and evaluation, and every iteration evaluated the
-// accepted trial a second time.  Per launch, before and after: 583 -> 266 us at
-// 128^3 with 2 % pores (iterations 1-200 of an increment, n = 10), 81 -> 40 us
-// at 64^3, 118 -> 74 us at 64^3 under the dislocation-density law, 110 -> 37 us at
-// 24^3 with a non-integral exponent (pow() of each system once per evaluation
-// instead of twice, and one evaluation in three less).
+// accepted trial a second time.  Per launch, that form, this one with the
+// Schmid constants from scalar registers, and this one with the sums of the
+// cubic family: 583, 240 and 219 us at 128^3 with 2 % pores (iterations 1-200
+// of an increment, n = 10), 81, 40 and 33 us at 64^3, 118, 74 and 64 us at 64^3
+// under the dislocation-density law, 110, 37 and 33 us at 24^3 with a
+// non-integral exponent (pow() of each system once per evaluation instead of
+// twice, and one evaluation in three less).
 #include <hip/hip_ext.h>
 
 #include "evpgpu_impl.h"
@@ -190,7 +193,16 @@ constexpr int SYS_GROUP = 2;
 // the lane's LDS column w (tangent() reads it if a Newton step follows).
 // it: LDS columns of 1/CRSS, forward then backward (RM_DISL: the passing
 // stress, then 1/(tau_0 + tau_cut)).  GD: the slip rates are written.
-template <int RM, bool CSYM, bool GD, int NE>
+//
+// CUBIC: the phase's systems are the twelve of {111}<110> (or {110}<111>, whose
+// symmetric Schmid tensors are the same) in any order and sign.  In the basis
+// that cubic_basis() scales Q to, the resolved shears of the four systems of a
+// cube axis are b + u + v, b - u - v, b + u - v and b - u + v, b one of R - P,
+// R + P and 2 P and u, v two of the shears: 21 additions instead of 60 fused
+// multiply-adds, 27 for the rate's five components and 40 instead of 240
+// operations for the tangent, and no constants to load.  The LDS columns hold
+// the systems in that order (P.cub_sys: the phase's own index of each).
+template <int RM, bool CSYM, bool GD, int NE, bool CUBIC>
 __device__ __forceinline__ void rates(const NewtonParams &P, int p, const double *it, double *w,
                                       const double *g0c, long long N, const double Q[25],
                                       const double s[6], double ed[5], double *gd, bool keep)
@@ -198,6 +210,42 @@ __device__ __forceinline__ void rates(const NewtonParams &P, int p, const double
     const int ns = RM == RM_FAST || RM == RM_DISL ? EVPGPU_NSYSMX : P.nsys[p];
     const int intn = P.int_n[p];
     const double g0 = P.gam0[p][0], ndt = P.nrs[p][0] * P.dt;
+    // the rate at the resolved shear r of system k (LDS columns in k's order)
+    auto slip = [&](int k, double r) {
+        const int sy = CUBIC ? P.cub_sys[p][k] : k; // the phase's index of it
+        double g, d; // the rate and dt times its derivative in the resolved shear
+        if (RM == RM_DISL) {
+            // gam = gam_o sinh((|rss| - tau_pass)/(tau_0 + tau_cut)) sign(rss)
+            // above the passing stress, 0 below (FORWARD_PLUS_BACKWARD)
+            const double a = fabs(r), tp = it[k * NB_THREADS];
+            const double itc = it[(EVPGPU_NSYSMX + k) * NB_THREADS];
+            const double g0k = g0c[sy * N];
+            g = d = 0.0;
+            if (a > tp) {
+                const double x = (a - tp) * itc;
+                // sinh and cosh from one expm1: with m = e^x - 1 and
+                // q = e^-x, sinh x = m (1 + q) / 2 (no cancellation at
+                // small x) and cosh x = (1 + m + q) / 2
+                const double em = expm1(x), q = rcp_refined(1.0 + em);
+                g = copysign(g0k * (0.5 * em * (1.0 + q)), r);
+                d = g0k * (0.5 * ((1.0 + em) + q)) * itc * P.dt;
+            }
+        } else {
+            const double itau = CSYM ? it[k * NB_THREADS] : it[((r < 0 ? EVPGPU_NSYSMX : 0) + k) * NB_THREADS];
+            const double x = r * itau, a = fabs(x);
+            const double p1 = (RM == RM_FAST ? g0 : P.gam0[p][sy]) * rate_power<RM, NE>(a, intn, P.nrs[p][sy]);
+            g = p1 * x;
+            // n < 1: |x|^(n-1) has no value at x = 0, |x|^n has
+            if (RM == RM_POW && P.nrs[p][sy] < 1.0)
+                g = copysign(P.gam0[p][sy] * pow(a, P.nrs[p][sy]), x);
+            d = (p1 * itau) * (RM == RM_FAST ? ndt : P.nrs[p][sy] * P.dt);
+        }
+        if (GD && keep) {
+            gd[sy * N] = CUBIC && P.cub_neg[p][k] ? -g : g;
+        }
+        w[k * NB_THREADS] = d;
+        return g;
+    };
     double sc[5], e[5];
 #pragma unroll
     for (int j = 0; j < 5; j++) {
@@ -207,57 +255,54 @@ __device__ __forceinline__ void rates(const NewtonParams &P, int p, const double
         sc[j] = a;
         e[j] = 0.0;
     }
-    cdouble mx = params_at(offsetof(NewtonParams, mx)) + p * (EVPGPU_NSYSMX * 5);
-    Consts<5 * SYS_GROUP> next = load_consts<5 * SYS_GROUP>(fresh(mx, s[0]));
+    if (CUBIC) {
+        // (sums of products: left to the compiler, some would be contracted
+        // and some not, another choice in each variant of the kernel)
+#pragma clang fp contract(off)
+        // (the columns are read here each time: hoisted they would spill)
+        __asm__ volatile("" ::: "memory");
+        const double b[3] = {sc[1] - sc[0], sc[1] + sc[0], 2.0 * sc[0]};
+        double G[3], U[3], V[3]; // per axis: sum of the rates, of the rates times the signs of u and v
 #pragma unroll
-    for (int k0 = 0; k0 < EVPGPU_NSYSMX; k0 += SYS_GROUP) {
-        const Consts<5 * SYS_GROUP> m = next;
-        if (k0 + SYS_GROUP < EVPGPU_NSYSMX)
-            next = load_consts<5 * SYS_GROUP>(fresh_after(mx, e) + 5 * (k0 + SYS_GROUP));
+        for (int a = 0; a < 3; a++) {
+            const double u = sc[CUB_U[a]], v = sc[CUB_V[a]], pl = u + v, mi = u - v;
+            const double g0 = slip(4 * a, b[a] + pl), g1 = slip(4 * a + 1, b[a] - pl);
+            const double g2 = slip(4 * a + 2, b[a] + mi), g3 = slip(4 * a + 3, b[a] - mi);
+            const double x = g0 - g1, y = g2 - g3;
+            G[a] = (g0 + g1) + (g2 + g3);
+            U[a] = x + y;
+            V[a] = x - y;
+        }
+        e[0] = fma(2.0, G[2], G[1] - G[0]);
+        e[1] = G[0] + G[1];
+        e[2] = V[1] + V[2];
+        e[3] = U[0] + U[2];
+        e[4] = V[0] + U[1];
+    } else {
+        cdouble mx = params_at(offsetof(NewtonParams, mx)) + p * (EVPGPU_NSYSMX * 5);
+        Consts<5 * SYS_GROUP> next = load_consts<5 * SYS_GROUP>(fresh(mx, s[0]));
 #pragma unroll
-        for (int k = k0; k < k0 + SYS_GROUP; k++) {
-            if (k >= ns) break;
-            const double *mk = m.c + 5 * (k - k0);
-            const double m0 = mk[0], m1 = mk[1], m2 = mk[2], m3 = mk[3], m4 = mk[4];
-            double r = m0 * sc[0];
-            r = fma(m1, sc[1], r);
-            r = fma(m2, sc[2], r);
-            r = fma(m3, sc[3], r);
-            r = fma(m4, sc[4], r);
-            double g, d; // the rate and dt times its derivative in the resolved shear
-            if (RM == RM_DISL) {
-                // gam = gam_o sinh((|rss| - tau_pass)/(tau_0 + tau_cut)) sign(rss)
-                // above the passing stress, 0 below (FORWARD_PLUS_BACKWARD)
-                const double a = fabs(r), tp = it[k * NB_THREADS];
-                const double itc = it[(EVPGPU_NSYSMX + k) * NB_THREADS], g0k = g0c[k * N];
-                g = d = 0.0;
-                if (a > tp) {
-                    const double x = (a - tp) * itc;
-                    // sinh and cosh from one expm1: with m = e^x - 1 and
-                    // q = e^-x, sinh x = m (1 + q) / 2 (no cancellation at
-                    // small x) and cosh x = (1 + m + q) / 2
-                    const double em = expm1(x), q = rcp_refined(1.0 + em);
-                    g = copysign(g0k * (0.5 * em * (1.0 + q)), r);
-                    d = g0k * (0.5 * ((1.0 + em) + q)) * itc * P.dt;
-                }
-            } else {
-                const double itau = CSYM ? it[k * NB_THREADS]
-                                         : it[((r < 0 ? EVPGPU_NSYSMX : 0) + k) * NB_THREADS];
-                const double x = r * itau, a = fabs(x);
-                const double p1 = (RM == RM_FAST ? g0 : P.gam0[p][k]) * rate_power<RM, NE>(a, intn, P.nrs[p][k]);
-                g = p1 * x;
-                // n < 1: |x|^(n-1) has no value at x = 0, |x|^n has
-                if (RM == RM_POW && P.nrs[p][k] < 1.0)
-                    g = copysign(P.gam0[p][k] * pow(a, P.nrs[p][k]), x);
-                d = (p1 * itau) * (RM == RM_FAST ? ndt : P.nrs[p][k] * P.dt);
+        for (int k0 = 0; k0 < EVPGPU_NSYSMX; k0 += SYS_GROUP) {
+            const Consts<5 * SYS_GROUP> m = next;
+            if (k0 + SYS_GROUP < EVPGPU_NSYSMX)
+                next = load_consts<5 * SYS_GROUP>(fresh_after(mx, e) + 5 * (k0 + SYS_GROUP));
+#pragma unroll
+            for (int k = k0; k < k0 + SYS_GROUP; k++) {
+                if (k >= ns) break;
+                const double *mk = m.c + 5 * (k - k0);
+                const double m0 = mk[0], m1 = mk[1], m2 = mk[2], m3 = mk[3], m4 = mk[4];
+                double r = m0 * sc[0];
+                r = fma(m1, sc[1], r);
+                r = fma(m2, sc[2], r);
+                r = fma(m3, sc[3], r);
+                r = fma(m4, sc[4], r);
+                const double g = slip(k, r);
+                e[0] = fma(m0, g, e[0]);
+                e[1] = fma(m1, g, e[1]);
+                e[2] = fma(m2, g, e[2]);
+                e[3] = fma(m3, g, e[3]);
+                e[4] = fma(m4, g, e[4]);
             }
-            if (GD && keep) gd[k * N] = g;
-            w[k * NB_THREADS] = d;
-            e[0] = fma(m0, g, e[0]);
-            e[1] = fma(m1, g, e[1]);
-            e[2] = fma(m2, g, e[2]);
-            e[3] = fma(m3, g, e[3]);
-            e[4] = fma(m4, g, e[4]);
         }
     }
 #pragma unroll
@@ -271,30 +316,64 @@ __device__ __forceinline__ void rates(const NewtonParams &P, int p, const double
 
 // K = K0 + dt d(edot)/d(sigma) (packed upper triangle) from the weights the
 // last rates() left: D' = sum_k w_k m_k m_k^T in crystal axes, then Q D' Q^T.
+template <bool CUBIC>
 __device__ __forceinline__ void tangent(int ns, int p, const double *w, const double Q[25],
                                         const double K0[21], double K[21])
 {
     double D[15]; // upper triangle, row by row
+    if (CUBIC) {
+        // per axis: the sum of the weights, and of the weights times the signs
+        // of u, of v and of u v
+        __asm__ volatile("" ::: "memory");
+        double W[3], U[3], V[3], C[3];
 #pragma unroll
-    for (int i = 0; i < 15; i++) D[i] = 0.0;
-    cdouble mx = params_at(offsetof(NewtonParams, mx)) + p * (EVPGPU_NSYSMX * 5);
-    Consts<5 * SYS_GROUP> next = load_consts<5 * SYS_GROUP>(fresh(mx, K0[0]));
+        for (int a = 0; a < 3; a++) {
+            const double w0 = w[4 * a * NB_THREADS], w1 = w[(4 * a + 1) * NB_THREADS];
+            const double w2 = w[(4 * a + 2) * NB_THREADS], w3 = w[(4 * a + 3) * NB_THREADS];
+            const double pl = w0 + w1, mi = w2 + w3, x = w0 - w1, y = w2 - w3;
+            W[a] = pl + mi;
+            C[a] = pl - mi;
+            U[a] = x + y;
+            V[a] = x - y;
+        }
+        // the columns P R 12 02 01; axis 0 (-1 1 0 u v), 1 (1 1 v 0 u), 2 (2 0 v u 0)
+        D[0] = fma(4.0, W[2], W[0] + W[1]);
+        D[1] = W[1] - W[0];
+        D[2] = fma(2.0, V[2], V[1]);
+        D[3] = fma(2.0, U[2], -U[0]);
+        D[4] = U[1] - V[0];
+        D[5] = W[0] + W[1];
+        D[6] = V[1];
+        D[7] = U[0];
+        D[8] = V[0] + U[1];
+        D[9] = W[1] + W[2];
+        D[10] = C[2];
+        D[11] = C[1];
+        D[12] = W[0] + W[2];
+        D[13] = C[0];
+        D[14] = W[0] + W[1];
+    } else {
 #pragma unroll
-    for (int k0 = 0; k0 < EVPGPU_NSYSMX; k0 += SYS_GROUP) {
-        const Consts<5 * SYS_GROUP> mc = next;
-        if (k0 + SYS_GROUP < EVPGPU_NSYSMX)
-            next = load_consts<5 * SYS_GROUP>(fresh_after(mx, D) + 5 * (k0 + SYS_GROUP));
+        for (int i = 0; i < 15; i++) D[i] = 0.0;
+        cdouble mx = params_at(offsetof(NewtonParams, mx)) + p * (EVPGPU_NSYSMX * 5);
+        Consts<5 * SYS_GROUP> next = load_consts<5 * SYS_GROUP>(fresh(mx, K0[0]));
 #pragma unroll
-        for (int k = k0; k < k0 + SYS_GROUP; k++) {
-            if (k >= ns) break;
-            const double *m = mc.c - 5 * k0;
-            const double wk = w[k * NB_THREADS];
-            int c = 0;
+        for (int k0 = 0; k0 < EVPGPU_NSYSMX; k0 += SYS_GROUP) {
+            const Consts<5 * SYS_GROUP> mc = next;
+            if (k0 + SYS_GROUP < EVPGPU_NSYSMX)
+                next = load_consts<5 * SYS_GROUP>(fresh_after(mx, D) + 5 * (k0 + SYS_GROUP));
 #pragma unroll
-            for (int i = 0; i < 5; i++) {
-                const double a = wk * m[5 * k + i];
+            for (int k = k0; k < k0 + SYS_GROUP; k++) {
+                if (k >= ns) break;
+                const double *m = mc.c - 5 * k0;
+                const double wk = w[k * NB_THREADS];
+                int c = 0;
 #pragma unroll
-                for (int j = i; j < 5; j++, c++) D[c] = fma(a, m[5 * k + j], D[c]);
+                for (int i = 0; i < 5; i++) {
+                    const double a = wk * m[5 * k + i];
+#pragma unroll
+                    for (int j = i; j < 5; j++, c++) D[c] = fma(a, m[5 * k + j], D[c]);
+                }
             }
         }
     }
@@ -422,6 +501,17 @@ __device__ __forceinline__ void rotation5(const double T[9], double Q[25])
     }
 }
 
+// Q to the basis of rates<CUBIC>: P, R and the three shears of the stress as
+// the resolved shears hold them (1/sqrt 6 of n and b included), so that every
+// Schmid component is 0, +-1 or +-2
+__device__ __forceinline__ void cubic_basis(double Q[25])
+{
+#pragma unroll
+    for (int i = 0; i < 5; i++)
+#pragma unroll
+        for (int j = 0; j < 5; j++) Q[5 * i + j] *= cub_scale(j);
+}
+
 // merit function of NR_MODIFIED: |R|^2 / 2 with R = C0 r
 __device__ __forceinline__ double merit(const double r[6])
 {
@@ -453,7 +543,7 @@ __device__ __forceinline__ double merit(const double r[6])
 // Only gamdot (from the rejected trial point) differs; the loop repeats the
 // last Newton launch of an increment with FAST off before edot or gamdot is
 // used, so FAST launches write neither.
-template <int RM, bool CSYM, bool FAST, int NE>
+template <int RM, bool CSYM, bool FAST, int NE, bool CUBIC>
 __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_newton(
     NewtonParams P, long long N, int p, int lead, const int *__restrict__ phase,
     const int *__restrict__ orient, const double *__restrict__ sgr, const double *sig_in, double *sig,
@@ -494,14 +584,15 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             const long long S12 = (long long)EVPGPU_NSYSMX * N;
 #pragma unroll
             for (int k = 0; k < EVPGPU_NSYSMX; k++) {
+                const int sy = CUBIC ? P.cub_sys[p][k] : k; // column k's system
                 if (RM == RM_DISL) {
                     // crss holds the increment's constants: passing stress,
                     // 1/(tau_0 + tau_cut), gam_o, the first call's passing stress
-                    c1[k] = crss[(P.dd_first ? 3 * S12 : 0) + k * N + v];
-                    c2[k] = crss[S12 + k * N + v];
+                    c1[k] = crss[(P.dd_first ? 3 * S12 : 0) + sy * N + v];
+                    c2[k] = crss[S12 + sy * N + v];
                 } else {
-                    c1[k] = crss[(k * 2) * N + v];
-                    if (!CSYM) c2[k] = crss[(k * 2 + 1) * N + v];
+                    c1[k] = crss[(sy * 2) * N + v];
+                    if (!CSYM) c2[k] = crss[(sy * 2 + 1) * N + v];
                 }
             }
             const double *sv = sgr + 36LL * ori;
@@ -525,6 +616,7 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
             for (int i = 0; i < 6; i++) dl[i * NB_THREADS] = d[i];
             rotation5(T9, Q);
+            if (CUBIC) cubic_basis(Q);
 #pragma unroll
             for (int k = 0; k < EVPGPU_NSYSMX; k++) {
                 if (RM == RM_DISL) {
@@ -546,7 +638,7 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
         int iterl = 0, trials = 0;
         {
             double ed[5];
-            rates<RM, CSYM, GD, NE>(P, p, it, w, g0c, N, Q, s, ed, gd, open);
+            rates<RM, CSYM, GD, NE, CUBIC>(P, p, it, w, g0c, N, Q, s, ed, gd, open);
             scaled_residual(P.dt, K0, dl, s, ed, r);
             if (!FAST)
 #pragma unroll
@@ -556,7 +648,8 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             // the first call used the previous call's mobile density; every
             // later one sees the density that call formed
 #pragma unroll
-            for (int k = 0; k < EVPGPU_NSYSMX; k++) it[k * NB_THREADS] = crss[k * N + v];
+            for (int k = 0; k < EVPGPU_NSYSMX; k++)
+                it[k * NB_THREADS] = crss[(CUBIC ? P.cub_sys[p][k] : k) * N + v];
         }
         double y2 = norm2(r);
         bool moved = false; // the last step, accepted, ended the solve
@@ -571,7 +664,7 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             double step[6];
             {
                 double K[21];
-                tangent(ns, p, w, Q, K0, K);
+                tangent<CUBIC>(ns, p, w, Q, K0, K);
 #pragma unroll
                 for (int i = 0; i < 6; i++) step[i] = -r[i];
                 const bool pd = ldl6_solve(K, step);
@@ -613,7 +706,7 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
                 for (int i = 0; i < 6; i++) sn[i] = fma(alam, step[i], s[i]);
                 // (a lane whose search is over repeats its last trial)
-                rates<RM, CSYM, GD, NE>(P, p, it, w, g0c, N, Q, sn, en, gd, search);
+                rates<RM, CSYM, GD, NE, CUBIC>(P, p, it, w, g0c, N, Q, sn, en, gd, search);
                 scaled_residual(P.dt, K0, dl, sn, en, rn);
                 trials += search;
                 y2n = norm2(rn);
@@ -801,35 +894,42 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
     for (int q = 0; q < nc; q++) {
         const int p = crystal[q], lead = q == 0;
         double *part = partials + (long long)q * nblk * NRED;
-        // compile-time exponents for the common n = 10 and n = 20
+        // compile-time exponents for the common n = 10 and n = 20, the sums of
+        // the cubic family wherever a phase has its twelve systems (219 us
+        // against 240 at 128^3) and the rate law is odd in the resolved shear
+        // (a place may hold a system of the other sign): not for unequal
+        // forward and backward CRSS.  RM_LOOP (n of 33 to 64) has no such
+        // variant: no use of it is known.
         const int ne = rm == RM_FAST && P.crss_sym && (P.int_n[p] == 10 || P.int_n[p] == 20) ? P.int_n[p] : 0;
         // the events (when given) take the kernel's own start and end times: no
         // marker packets between the launches
 #define NEWTON_ARGS dim3(nblk), dim3(NB_THREADS), 0, c->stream, lead ? ev_start : nullptr,                  \
                     q == nc - 1 ? ev_stop : nullptr, 0, P, n, p, lead, phase, orient, sgr, sig_in, sig, E, epsp, \
                     edot, tran, crss, gamdot, part, status
-#define LAUNCH(A, B, F) hipExtLaunchKernelGGL((k_newton<A, B, F, 0>), NEWTON_ARGS)
-#define LAUNCH_NE(E, F) hipExtLaunchKernelGGL((k_newton<RM_FAST, true, F, E>), NEWTON_ARGS)
-#define LAUNCH_RM(B, F)                                                                  \
-    do {                                                                                 \
-        if (ne == 10) LAUNCH_NE(10, F);                                                  \
-        else if (ne == 20) LAUNCH_NE(20, F);                                             \
-        else if (rm == RM_FAST) LAUNCH(RM_FAST, B, F);                                   \
-        else if (rm == RM_LOOP) LAUNCH(RM_LOOP, B, F);                                   \
-        else LAUNCH(RM_POW, B, F);                                                       \
+#define LAUNCH(A, B, F, E, C) hipExtLaunchKernelGGL((k_newton<A, B, F, E, C>), NEWTON_ARGS)
+#define LAUNCH_SYM(F, C)                                                                 \
+    do { /* RM_FAST with equal forward and backward CRSS */                              \
+        if (ne == 10) LAUNCH(RM_FAST, true, F, 10, C);                                   \
+        else if (ne == 20) LAUNCH(RM_FAST, true, F, 20, C);                              \
+        else LAUNCH(RM_FAST, true, F, 0, C);                                             \
     } while (0)
-        if (P.dd) {
-            if (fast) LAUNCH(RM_DISL, false, true);
-            else LAUNCH(RM_DISL, false, false);
-        } else if (fast) {
-            if (P.crss_sym) LAUNCH_RM(true, true);
-            else LAUNCH_RM(false, true);
-        } else {
-            if (P.crss_sym) LAUNCH_RM(true, false);
-            else LAUNCH_RM(false, false);
-        }
+#define LAUNCH_RM(F)                                                                     \
+    do {                                                                                 \
+        if (P.dd && P.cubic[p]) LAUNCH(RM_DISL, false, F, 0, true);                      \
+        else if (P.dd) LAUNCH(RM_DISL, false, F, 0, false);                              \
+        else if (rm == RM_FAST && P.crss_sym && P.cubic[p]) LAUNCH_SYM(F, true);         \
+        else if (rm == RM_FAST && P.crss_sym) LAUNCH_SYM(F, false);                      \
+        else if (rm == RM_FAST) LAUNCH(RM_FAST, false, F, 0, false);                     \
+        else if (rm == RM_LOOP && P.crss_sym) LAUNCH(RM_LOOP, true, F, 0, false);        \
+        else if (rm == RM_LOOP) LAUNCH(RM_LOOP, false, F, 0, false);                     \
+        else if (rm == RM_POW && P.crss_sym && P.cubic[p]) LAUNCH(RM_POW, true, F, 0, true); \
+        else if (P.crss_sym) LAUNCH(RM_POW, true, F, 0, false);                          \
+        else LAUNCH(RM_POW, false, F, 0, false);                                         \
+    } while (0)
+        if (fast) LAUNCH_RM(true);
+        else LAUNCH_RM(false);
 #undef LAUNCH_RM
-#undef LAUNCH_NE
+#undef LAUNCH_SYM
 #undef LAUNCH
 #undef NEWTON_ARGS
     }
