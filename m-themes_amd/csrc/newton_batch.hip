@@ -30,16 +30,12 @@
 // start from its rotation and kept in a wave-private LDS slab laid out
 // [component][lane] (conflict-free); C0 and S0 (packed triangles) are a
 // 42-entry LDS table read by broadcast; all other per-voxel arrays live in
-// registers, except the weights of the tangent (a rate's derivative times dt),
-// which wait in LDS from the evaluation that formed them to the step that
-// needs them.  One wave per SIMD (the solve holds about 420 registers; the
-// slab's 37 KB allow no more either), so a SIMD waits out every dependent
-// FP64 operation: what bounds the kernel is the length of the solve.  An
-// accepted trial's evaluation is the next iteration's start, the tangent is
-// formed only where a step follows and n = 10 and n = 20 are compiled in:
-// 1000003 voxels at n = 20 take 797 us where evaluating every iteration
-// anew took 1001 us; 1000 voxels (one wave's latency) 74.5 us for 99.4 us
-// with the one wait of a call.
+// registers.  One wave per SIMD (the solve holds about 420 registers).
+//
+// Taking an accepted trial's evaluation as the next iteration's start, as the
+// loop's kernel does, was measured at 795 us where this form takes 1000 us
+// (1000003 voxels, n = 20) and left out: the compiled tangent rounds
+// differently, and one voxel in a million then reports another count.
 #include "evpgpu_impl.h"
 #include "linesearch.h"
 
@@ -72,23 +68,10 @@ __device__ __forceinline__ double ipow5(double x, int m)
     return r;
 }
 
-// x^M for a compile-time M: the products of ipow with the bit tests folded
-// (x^9 is three squarings and one product)
-template <int M> __device__ __forceinline__ double ipowc(double x)
-{
-    double r = 1.0, b = x;
-#pragma unroll
-    for (int m = M; m; m >>= 1) {
-        if (m & 1) r *= b;
-        if (m > 1) b *= b;
-    }
-    return r;
-}
-
 // Rate-law evaluation: RM_POW pow() for a non-integral exponent, RM_LOOP
 // repeated squaring for an integral one, RM_FAST the common case of every
 // crystal phase having EVPGPU_NSYSMX systems with one integral n <= 32 and
-// one reference rate (n = 10 and n = 20 with the exponent a template constant).
+// one reference rate.
 enum { RM_POW = 0, RM_LOOP = 1, RM_FAST = 2 };
 
 // chg_basis opt 2 for a symmetric tensor given as (11 22 33 23 13 12)
@@ -120,19 +103,20 @@ constexpr int NB_THREADS = 64; // one wave per block: the LDS slab is wave-priva
 struct RateIn {
     const double *sc;                              // LDS slab, sc[(s*5+j)*64]
     const double *k0;                              // LDS: C0 then S0, packed triangles
-    double *w;                                     // LDS columns: dt times the rates' derivatives
     double itf[EVPGPU_NSYSMX], itb[EVPGPU_NSYSMX]; // 1/CRSS forward, backward
 };
 #define SC(i, j) in.sc[((i)*5 + (j)) * NB_THREADS]
 
 // StrainRate_eval (src/constitutive.c:5-67) as one pass over the slip
 // systems: each system's Schmid vector is read from LDS once and feeds the
-// resolved shear, the rate and edot.  The sums run over the systems in
-// ascending order, as the reference's separate loops do.  dt times the
-// derivative of each rate in its resolved shear goes to the LDS column w.
-template <int RM, int NE>
+// resolved shear, the rate, edot and d(edot)/d(sigma).  The sums run over the
+// systems in ascending order, as the reference's separate loops do.
+// DD: dt d(edot)/d(sigma) is added into the packed Newton matrix kk (which
+// holds S0 + S on entry).
+template <bool DD, int RM>
 __device__ __forceinline__ void srate(const NewtonParams &P, int p, const RateIn &in,
-                                      const double s[6], double ed[5], double gd[EVPGPU_NSYSMX])
+                                      const double s[6], double ed[5], double kk[21],
+                                      double gd[EVPGPU_NSYSMX])
 {
     // (the per-system test stays a branch on the phase's count even where it
     // is always 12: without it the compiler interleaves the systems'
@@ -164,7 +148,7 @@ __device__ __forceinline__ void srate(const NewtonParams &P, int p, const RateIn
             r = r * itau;
             double a = fabs(r), p1, p2;
             if (RM == RM_FAST) {
-                p1 = NE > 0 ? ipowc<(NE > 0 ? NE - 1 : 0)>(a) : ipow5(a, intn - 1);
+                p1 = ipow5(a, intn - 1);
                 p2 = p1 * a;
             } else if (RM == RM_LOOP) {
                 p1 = ipow(a, intn - 1);
@@ -174,35 +158,21 @@ __device__ __forceinline__ void srate(const NewtonParams &P, int p, const RateIn
                 p2 = pow(a, P.nrs[p][k]);
             }
             r2 = (RM == RM_FAST ? g0 : P.gam0[p][k]) * p2 * (double)(2 * (r > 0) - 1);
-            r1 = (RM == RM_FAST ? g0n : P.gam0[p][k] * P.nrs[p][k]) * p1 * itau;
+            if (DD) r1 = (RM == RM_FAST ? g0n : P.gam0[p][k] * P.nrs[p][k]) * p1 * itau;
             gd[k] = r2;
 #pragma unroll
             for (int i = 0; i < 5; i++) ed[i] += sc[i] * r2;
-            in.w[k * NB_THREADS] = r1 * P.dt;
-        }
-    }
-}
-
-// dt d(edot)/d(sigma) at the point of the last srate() added into the packed
-// Newton matrix kk (which holds S0 + S on entry), the systems in ascending
-// order
-__device__ __forceinline__ void tangent(const NewtonParams &P, int p, const RateIn &in, double kk[21])
-{
-    const int ns = P.nsys[p];
+            if (DD) {
+                r1 *= P.dt;
 #pragma unroll
-    for (int k = 0; k < EVPGPU_NSYSMX; k++)
-        if (k < ns) {
-            const double r1 = in.w[k * NB_THREADS];
-            double sc[5];
+                for (int i = 0; i < 5; i++) {
+                    const double w = sc[i] * r1;
 #pragma unroll
-            for (int j = 0; j < 5; j++) sc[j] = SC(k, j);
-#pragma unroll
-            for (int i = 0; i < 5; i++) {
-                const double w = sc[i] * r1;
-#pragma unroll
-                for (int j = i; j < 5; j++) kk[PK(i, j)] += w * sc[j];
+                    for (int j = i; j < 5; j++) kk[PK(i, j)] += w * sc[j];
+                }
             }
         }
+    }
 }
 
 // 1/sqrt(d) for a positive normal d: the hardware estimate refined by two
@@ -294,19 +264,14 @@ __device__ __forceinline__ void residual(const NewtonParams &P, const RateIn &in
     }
 }
 
-// edot, the strain mismatch's norm squared, the residual and the merit
-// function at sig
-template <int RM, int NE>
-__device__ __forceinline__ double evaluate(const NewtonParams &P, int p, const RateIn &in, const Vox &V,
-                                           const double sig[6], double ed[5], double &ce, double res[6],
-                                           double gd[EVPGPU_NSYSMX])
+template <int RM>
+__device__ __forceinline__ double nr_quality(const NewtonParams &P, int p, const RateIn &in,
+                                             const Vox &V, const double sig[6],
+                                             double gd[EVPGPU_NSYSMX])
 {
-    double t[6];
-    srate<RM, NE>(P, p, in, sig, ed, gd);
+    double ed[5], t[6], res[6];
+    srate<false, RM>(P, p, in, sig, ed, nullptr, gd);
     residual(P, in, V, sig, ed, t, res);
-    ce = 0.0;
-#pragma unroll
-    for (int i = 0; i < 6; i++) ce += t[i] * t[i];
     double f = 0.0;
 #pragma unroll
     for (int i = 0; i < 6; i++) f += res[i] * res[i];
@@ -314,35 +279,42 @@ __device__ __forceinline__ double evaluate(const NewtonParams &P, int p, const R
 }
 
 // returns 0, EVPGPU_ERR_SINGULAR or EVPGPU_ERR_LINESEARCH
-// An accepted trial's evaluation is the next iteration's start (the same
-// point, so the same bits), and the tangent is formed only where a step is
-// taken, from the weights that evaluation left in LDS.
-template <int RM, int NE>
+template <int RM>
 __device__ int update_voxel(const NewtonParams &P, int p, RateIn &in, const Vox &V,
                             double sig6[6], double edotp[6], double gd[EVPGPU_NSYSMX],
-                            double &conv_s, double &conv_e, int &iterl)
+                            double &conv_s, double &conv_e, int &iterl, int &trials)
 {
+    trials = 0;
     double ed[5], res[6], old[6], k[21];
-    double ce;
+    double ce = 0.0;
     iterl = 0;
+    double erral = 10 * P.nr_tol;
 #pragma unroll
     for (int i = 0; i < 6; i++) sig6[i] = V.xl[i];
-    double f_old = evaluate<RM, NE>(P, p, in, V, sig6, ed, ce, res, gd);
-    for (;;) {
+    while ((iterl < 500) && (fabs(erral) > fabs(P.nr_tol))) {
         // read C0, S0 and the Schmid vectors from LDS where they are used:
         // hoisted out of the loop they would occupy 204 more registers
         __asm__ volatile("" ::: "memory");
         iterl++;
 #pragma unroll
         for (int i = 0; i < 6; i++) old[i] = sig6[i];
-        // the Newton matrix K = S0 + S + dt D
+        // the Newton matrix K = S0 + S + dt D (below), D added by srate
 #pragma unroll
         for (int i = 0; i < 6; i++)
 #pragma unroll
             for (int j = i; j < 6; j++) k[PK(i, j)] = in.k0[21 + PK(i, j)] + V.S[PK(i, j)];
-        tangent(P, p, in, k);
+        srate<true, RM>(P, p, in, sig6, ed, k, gd);
+#pragma unroll
+        for (int i = 0; i < 6; i++) edotp[i] = i < 5 ? ed[i] : 0.0;
         double gradf[6], step[6];
-        // S0 R: the right-hand side of the step
+        {
+            double t[6];
+            residual(P, in, V, sig6, ed, t, res);
+            ce = 0.0;
+#pragma unroll
+            for (int i = 0; i < 6; i++) ce += t[i] * t[i];
+        }
+        // S0 R: the right-hand side of the step, and its norm bounds the step
 #pragma unroll
         for (int i = 0; i < 6; i++) {
             double b = 0.0;
@@ -374,59 +346,52 @@ __device__ int update_voxel(const NewtonParams &P, int p, RateIn &in, const Vox 
 #pragma unroll
             for (int i = 0; i < 6; i++) step[i] = -step[i];
         }
-        const double stpmax = 10.0, ALF = 1.E-4;
-        double sum = 0.0, slope = 0.0;
+        double f_old = 0.0;
+#pragma unroll
+        for (int i = 0; i < 6; i++) f_old += res[i] * res[i];
+        f_old *= 0.5;
+        const double stpmax = 10.0, ALF = 1.E-4, TOLX = P.tolx;
+        double sum = 0.0, slope = 0.0, test = 0.0;
 #pragma unroll
         for (int i = 0; i < 6; i++) sum += step[i] * step[i];
-        if (sum > stpmax * stpmax) {
-            sum = sqrt(sum);
+        sum = sqrt(sum);
+        if (sum > stpmax) {
 #pragma unroll
             for (int i = 0; i < 6; i++) step[i] *= stpmax / sum;
         }
 #pragma unroll
         for (int i = 0; i < 6; i++) slope += gradf[i] * step[i];
         if (slope >= 0) return EVPGPU_ERR_LINESEARCH;
-        double alam = 1.0, alam2 = 0.0, f2 = 0.0, f_new, cen;
-        double edn[5], resn[6];
-        bool rejected;
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            double d = fabs(old[i]);
+            double t = fabs(step[i]) / (d > 1.0 ? d : 1.0);
+            if (t > test) test = t;
+        }
+        double alamin = TOLX / test, alam = 1.0, alam2 = 0.0, f2 = 0.0;
         while (true) {
             __asm__ volatile("" ::: "memory");
 #pragma unroll
             for (int i = 0; i < 6; i++) sig6[i] = old[i] + alam * step[i];
-            f_new = evaluate<RM, NE>(P, p, in, V, sig6, edn, cen, resn, gd);
-            // the trial is rejected when alam max|step_i|/max(|s_i|,1) < TOLX
-            // (compared by products: no divisions)
-            rejected = true;
+            double f_new = nr_quality<RM>(P, p, in, V, sig6, gd);
+            trials++;
+            if (alam < alamin) {
 #pragma unroll
-            for (int i = 0; i < 6; i++) {
-                const double d = fabs(old[i]);
-                if (alam * fabs(step[i]) >= P.tolx * (d > 1.0 ? d : 1.0)) rejected = false;
+                for (int i = 0; i < 6; i++) sig6[i] = old[i];
+                break;
+            } else if (f_new <= f_old + ALF * alam * slope) {
+                break;
             }
-            if (rejected || f_new <= f_old + ALF * alam * slope) break;
             const double next = ls_backtrack(alam, alam2, f_new, f2, f_old, slope);
             alam2 = alam;
             f2 = f_new; // the backtrack value the cubic step needs (Q18)
             alam = next;
         }
-        if (rejected) {
-#pragma unroll
-            for (int i = 0; i < 6; i++) sig6[i] = old[i];
-            break;
-        }
         double conv_nr = 0.0;
 #pragma unroll
         for (int i = 0; i < 6; i++) conv_nr += (sig6[i] - old[i]) * (sig6[i] - old[i]);
-        // done: edot and the norms stay those of the iteration's start
-        if (iterl >= 500 || !(sqrt(conv_nr) / V.signorm > fabs(P.nr_tol))) break;
-#pragma unroll
-        for (int i = 0; i < 5; i++) ed[i] = edn[i];
-#pragma unroll
-        for (int i = 0; i < 6; i++) res[i] = resn[i];
-        ce = cen;
-        f_old = f_new;
+        erral = sqrt(conv_nr) / V.signorm;
     }
-#pragma unroll
-    for (int i = 0; i < 6; i++) edotp[i] = i < 5 ? ed[i] : 0.0;
     // the norms of the last iteration (the reference overwrites them in
     // every iteration)
     double cs = 0.0;
@@ -440,7 +405,7 @@ __device__ int update_voxel(const NewtonParams &P, int p, RateIn &in, const Vox 
 // One lane per voxel.  Reads lambda from sig_in and writes the new stress to
 // sig (which may be the same buffer), edot, gamdot, the error norms and the
 // Newton count.
-template <int RM, int NE>
+template <int RM>
 __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_newton_batch(
     NewtonParams P, long long N, const int *__restrict__ phase, const int *__restrict__ orient,
     const double *__restrict__ sgr, const double *sig_in, double *sig, const double *__restrict__ E,
@@ -449,8 +414,7 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
     double *__restrict__ err_vox, int *__restrict__ niter_vox)
 {
     if (P.skip && *P.skip) return;
-    // the Schmid tensors, then the tangent's weights
-    __shared__ double slab[EVPGPU_NSYSMX * 6 * NB_THREADS];
+    __shared__ double slab[EVPGPU_NSYSMX * 5 * NB_THREADS];
     // C0 and S0 (packed upper triangles) as broadcast LDS reads: kept in
     // scalar registers they do not fit, and each use of a spilled one costs
     // two lane reads
@@ -539,7 +503,6 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
             for (int q = 0; q < 9; q++) T[q / 3][q % 3] = T9[q];
             in.sc = slab + threadIdx.x;
             in.k0 = k0;
-            in.w = slab + EVPGPU_NSYSMX * 5 * NB_THREADS + threadIdx.x;
             // unrolled (straight-line where the count is the constant 12), so
             // that the loads above stay ahead of this arithmetic
 #pragma unroll
@@ -584,8 +547,8 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                 }
             }
             double s6[6], e6[6], gd[EVPGPU_NSYSMX], cs, ce;
-            int it;
-            int st = update_voxel<RM, NE>(P, p, in, V, s6, e6, gd, cs, ce, it);
+            int it, ntr;
+            int st = update_voxel<RM>(P, p, in, V, s6, e6, gd, cs, ce, it, ntr);
             if (st) {
                 atomicCAS(status, 0, st);
             } else {
@@ -623,24 +586,13 @@ int newton_batch_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_
                         double *err_vox, int *niter_vox)
 {
     const dim3 grid((unsigned)((n + NB_THREADS - 1) / NB_THREADS)), block(NB_THREADS);
-#define LAUNCH(RM, NE)                                                                                          \
-    hipLaunchKernelGGL((k_newton_batch<RM, NE>), grid, block, 0, c->stream, P, n, phase, orient, sgr, sig_in, sig, \
-                       E, epsp, edot, tran, crss, gamdot, status, err_vox, niter_vox)
-    // a compile-time exponent where every crystal phase has it
-    bool all10 = true, all20 = true;
-    for (int q = 0; q < 2; q++)
-        if (!P.is_gas[q]) {
-            all10 = all10 && P.int_n[q] == 10;
-            all20 = all20 && P.int_n[q] == 20;
-        }
+#define LAUNCH(RM)                                                                                               \
+    hipLaunchKernelGGL((k_newton_batch<RM>), grid, block, 0, c->stream, P, n, phase, orient, sgr, sig_in, sig, E, \
+                       epsp, edot, tran, crss, gamdot, status, err_vox, niter_vox)
     switch (newton_rate_mode(P)) {
-    case RM_FAST:
-        if (all10) LAUNCH(RM_FAST, 10);
-        else if (all20) LAUNCH(RM_FAST, 20);
-        else LAUNCH(RM_FAST, 0);
-        break;
-    case RM_LOOP: LAUNCH(RM_LOOP, 0); break;
-    default: LAUNCH(RM_POW, 0);
+    case RM_FAST: LAUNCH(RM_FAST); break;
+    case RM_LOOP: LAUNCH(RM_LOOP); break;
+    default: LAUNCH(RM_POW);
     }
 #undef LAUNCH
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
