@@ -34,7 +34,8 @@
 // Schmid constants from scalar registers, and this one with the sums of the
 // cubic family: 583, 240 and 219 us at 128^3 with 2 % pores (iterations 1-200
 // of an increment, n = 10), 81, 40 and 33 us at 64^3, 118, 74 and 64 us at 64^3
-// under the dislocation-density law, 110, 37 and 33 us at 24^3 with a
+// under the dislocation-density law (a first increment; 111 us in its 16th, 94
+// with the rates left out for the lanes that wait), 110, 37 and 33 us at 24^3 with a
 // non-integral exponent (pow() of each system once per evaluation instead of
 // twice, and one evaluation in three less).
 #include <hip/hip_ext.h>
@@ -221,7 +222,9 @@ __device__ __forceinline__ void rates(const NewtonParams &P, int p, const double
             const double itc = it[(EVPGPU_NSYSMX + k) * NB_THREADS];
             const double g0k = g0c[sy * N];
             g = d = 0.0;
-            if (a > tp) {
+            // (only for the lanes at work: a wave that waits for a few lanes'
+            // line searches then skips the systems below their passing stress)
+            if (keep && a > tp) {
                 const double x = (a - tp) * itc;
                 // sinh and cosh from one expm1: with m = e^x - 1 and
                 // q = e^-x, sinh x = m (1 + q) / 2 (no cancellation at
@@ -243,7 +246,7 @@ __device__ __forceinline__ void rates(const NewtonParams &P, int p, const double
         if (GD && keep) {
             gd[sy * N] = CUBIC && P.cub_neg[p][k] ? -g : g;
         }
-        w[k * NB_THREADS] = d;
+        if (RM != RM_DISL || keep) w[k * NB_THREADS] = d;
         return g;
     };
     double sc[5], e[5];
@@ -700,13 +703,17 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                 open = open && !rej;
                 if (!__any(open)) break;
             }
-            double alam2 = 0.0, f2 = 0.0, sn[6], en[5], rn[6], y2n;
+            double alam2 = 0.0, f2 = 0.0, sn[6], en[5] = {0., 0., 0., 0., 0.}, rn[6], y2n;
             bool search = open;
             for (;;) {
 #pragma unroll
                 for (int i = 0; i < 6; i++) sn[i] = fma(alam, step[i], s[i]);
-                // (a lane whose search is over repeats its last trial)
-                rates<RM, CSYM, GD, NE, CUBIC>(P, p, it, w, g0c, N, Q, sn, en, gd, search);
+                // (a lane whose search is over repeats its last trial, with
+                // RM_DISL from the rates that it kept)
+                double et[5];
+                rates<RM, CSYM, GD, NE, CUBIC>(P, p, it, w, g0c, N, Q, sn, et, gd, search);
+#pragma unroll
+                for (int i = 0; i < 5; i++) en[i] = RM != RM_DISL || search ? et[i] : en[i];
                 scaled_residual(P.dt, K0, dl, sn, en, rn);
                 trials += search;
                 y2n = norm2(rn);
