@@ -37,41 +37,38 @@ from pyevp import lib, synth  # noqa: E402
 METRIC = "voxel-iters/s at 128³, mixed vs FP64 GPU at 1e-6 err; adjoint/forward time"
 
 # FP64 operations of the per-voxel Newton kernel, counted by hand from
-# newton.hip (an FMA counts as 2, a refined reciprocal square root as 10):
-#   per crystal voxel and launch: 12 Schmid tensors from the rotation
-#     (~55 each), three basis changes, |lambda|, 12 reciprocal CRSS, two
-#     back-conversions                                                   ~800
-#   per Newton iteration: rate law with dt d(edot)/d(sigma) added into the
-#     packed Newton matrix (12 x ~67), S0 + S (21), strain mismatch and
-#     residual (168), S0 R, C0 R and the merit gradient K C0 R (3 x 72),
-#     6x6 Cholesky and the two triangular solves (~250), step control (~60)
-#                                                                       ~1520
-#   per line-search trial: rate law without derivative (12 x ~29), strain
-#     mismatch, residual, merit function, trial point                    ~540
-NEWTON_FLOPS_VOXEL = 800
-NEWTON_FLOPS_ITER = 1520
-NEWTON_FLOPS_TRIAL = 540
-# The algorithmic count the roofline figure uses: the reference's own per-voxel
-# work, counted from src/evolution.c:44-310 and src/constitutive.c:5-67 --
-# about 0.5 kflop of set-up per voxel and launch (LU of C_gr, basis changes)
-# and 4.7 kflop per Newton iteration (rate law with its derivative, the
-# Jacobian and its pivoted-LU inverse, the step and one line-search trial),
-# with the pow() calls not counted.  The kernel's own, smaller count above
-# (symmetric Cholesky form, precomputed inverse) is reported beside it.
+# newton.hip's variant for the cubic slip family at n = 10 (an FMA counts as 2,
+# a refined reciprocal as 9):
+#   an evaluation: the stress into the crystal axes and the rate out (2 x 45),
+#     resolved shears and sums (~50), twelve rates (9 each), residual (82),
+#     norm (11)                                                          ~340
+#   per crystal voxel and launch: basis changes, d, K0 = S0 + S, the rotation
+#     of deviators, 12 reciprocal CRSS, the closing norms (~530), and the
+#     first evaluation                                                    ~870
+#   per Newton step: the tangent (40 + 375), L D L^T and its solve (~205), an
+#     evaluation (the next iteration's start)                             ~960
+# The last iteration of a solve ends at its residual, without a step.
+NEWTON_FLOPS_VOXEL = 870
+NEWTON_FLOPS_STEP = 960
+# The reference's own per-voxel work, counted from src/evolution.c:44-310 and
+# src/constitutive.c:5-67 -- about 0.5 kflop of set-up per voxel and launch (LU
+# of C_gr, basis changes) and 4.7 kflop per Newton iteration (rate law with its
+# derivative, the Jacobian and its pivoted-LU inverse, the step and one
+# line-search trial), with the pow() calls not counted -- reported beside it.
 ALG_FLOPS_VOXEL = 500
 ALG_FLOPS_ITER = 4700
 # HBM bytes of the Newton kernel per crystal voxel and launch: reads sigma,
 # strain, plastic strain (3 x 48), the rotation (72), CRSS (96: forward =
-# backward), phase + orientation index (8); writes sigma and edot (2 x 48).
-# (The one launch per increment with the shortcut off also writes gamdot,
-# 96 B.)  Gas voxels: phase (4), sigma/edot writes (96), sigma re-read (48).
-NEWTON_BYTES_CRYSTAL = 3 * 48 + 72 + 96 + 8 + 2 * 48
-NEWTON_BYTES_GAS = 4 + 96 + 48
+# backward), phase + orientation index (8); writes sigma (48).  (The one launch
+# per increment with the shortcut off also writes edot and gamdot, 144 B.)  Gas
+# voxels: phase + orientation index (8), sigma written (48).
+NEWTON_BYTES_CRYSTAL = 3 * 48 + 72 + 96 + 8 + 48
+NEWTON_BYTES_GAS = 8 + 48
 # k_newton's HBM traffic per launch on the 128^3 job (launches with the
 # shortcut on), measured: rocprofv3 FETCH_SIZE x 1024 x 2 + WRITE_SIZE x 1024
 # (FETCH_SIZE reads half and WRITE_SIZE all of a plain copy kernel's bytes);
-# 684.5 MB read + 205.5 MB written against 861 MB algorithmic.
-NEWTON_TRAFFIC_128 = 8.900e8
+# 766 MB read + 105 MB written against 759 MB algorithmic.
+NEWTON_TRAFFIC_128 = 8.710e8
 PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFS = 78.6
 
@@ -389,12 +386,12 @@ def main():
     j.close()
     n_cryst = int(np.sum(p == 1))
     n_gas = N - n_cryst
-    flops = (ALG_FLOPS_VOXEL * n_cryst * launches + ALG_FLOPS_ITER * nit) / launches
-    own = (NEWTON_FLOPS_VOXEL * n_cryst * launches + NEWTON_FLOPS_ITER * nit + NEWTON_FLOPS_TRIAL * ntr) / launches
+    ref = (ALG_FLOPS_VOXEL * n_cryst * launches + ALG_FLOPS_ITER * nit) / launches
+    flops = (NEWTON_FLOPS_VOXEL * n_cryst * launches + NEWTON_FLOPS_STEP * (nit - n_cryst * launches)) / launches
     bytes_ = NEWTON_BYTES_CRYSTAL * n_cryst + NEWTON_BYTES_GAS * n_gas
     t_s = avg_ms * 1e-3
     tf = flops / t_s / 1e12
-    tf_own = own / t_s / 1e12
+    tf_ref = ref / t_s / 1e12
     gbs = bytes_ / t_s / 1e9
     # measured HBM bytes per launch of k_newton on this job (rocprofv3 FETCH_SIZE
     # and WRITE_SIZE scaled by a copy kernel's readings), 128^3 workload only
@@ -403,21 +400,16 @@ def main():
                trials_per_voxel_launch=ntr / max(n_cryst * launches, 1),
                flops_per_launch=flops, bytes_per_launch=bytes_, launches=launches,
                timed_launches=sampled,
-               kernel_count=dict(tflops=tf_own, frac=tf_own / PEAK_FP64_TFS, flops_per_launch=own))
-    if tf / PEAK_FP64_TFS >= gbs / PEAK_HBM_GBS:
-        roof = dict(bound="fp64-valu", achieved=tf, peak=PEAK_FP64_TFS, unit="TFLOP/s",
-                    frac=tf / PEAK_FP64_TFS, traffic=traffic, kernel="k_newton",
-                    avg_launch_ms=avg_ms, hbm_gbs=gbs, **per,
-                    note="bound by the FP64 vector ALU (no MFMA instruction is used); peak is "
-                         "the MI355X FP64 vector figure, 78.6 TFLOP/s; achieved counts the "
-                         "reference's work per voxel (0.5 kflop + 4.7 kflop per Newton iteration), "
-                         "kernel_count the kernel's own smaller count; avg_launch_ms from HIP "
-                         "events on the launches of one Green iteration in "
-                         f"{args.timer_every} over the timed region")
-    else:
-        roof = dict(bound="hbm", achieved=gbs, peak=PEAK_HBM_GBS, unit="GB/s",
-                    frac=gbs / PEAK_HBM_GBS, traffic=traffic, kernel="k_newton",
-                    avg_launch_ms=avg_ms, tflops=tf, **per)
+               reference_count=dict(tflops=tf_ref, frac=tf_ref / PEAK_FP64_TFS, flops_per_launch=ref))
+    roof = dict(bound="fp64-valu", achieved=tf, peak=PEAK_FP64_TFS, unit="TFLOP/s",
+                frac=tf / PEAK_FP64_TFS, traffic=traffic, kernel="k_newton",
+                avg_launch_ms=avg_ms, hbm_gbs=gbs, **per,
+                note="bound by the issue of FP64 vector instructions (no MFMA instruction is used); "
+                     "peak is the MI355X FP64 vector figure, 78.6 TFLOP/s; achieved counts the "
+                     "kernel's own operations of the lanes at work, reference_count the reference's "
+                     "work per voxel (0.5 kflop + 4.7 kflop per Newton iteration); avg_launch_ms "
+                     "from HIP events on the launches of one Green iteration in "
+                     f"{args.timer_every} over the timed region")
     kern = {}
     names = ["newton", "fft_forward", "green", "fft_inverse_update", "increment_pro_epilogue",
              "anchor_refresh"]

@@ -130,9 +130,9 @@ typedef struct {
 
 const char *evpgpu_strerror(int status);
 
-/* Create a context for an nx*ny*nz grid, each length in [2, 512].  Powers of
- * two in [8, 256] take the Stockham transforms; other lengths a direct DFT
- * along that axis (O(L) work per element, correct for any length). */
+/* Create a context for an nx*ny*nz grid, each length in [2, 512].  Products of
+ * 2, 3 and 5 in [8, 256] take the Stockham transforms; other lengths a
+ * two-level DFT along that axis (correct for any length). */
 int evpgpu_create(evpgpu_ctx **ctx, int nx, int ny, int nz, int precision);
 int evpgpu_destroy(evpgpu_ctx *ctx);
 int evpgpu_set_precision(evpgpu_ctx *ctx, int precision);

@@ -103,8 +103,8 @@ double now_s()
     return ts.tv_sec + 1e-9 * ts.tv_nsec;
 }
 
-// grid lengths: any length in [2, 512]; powers of two from 8 take the
-// Stockham kernels, the others the direct-DFT ones (fft.hip)
+// grid lengths: any length in [2, 512]; products of 2, 3 and 5 in [8, 256]
+// take the Stockham kernels, the others the two-level DFT ones (fft.hip)
 bool len_ok(int n) { return n >= 2 && n <= 512; }
 
 template <typename T> int dalloc(T **p, size_t n)
