@@ -67,8 +67,8 @@ NEWTON_BYTES_GAS = 8 + 48
 # k_newton's HBM traffic per launch on the 128^3 job (launches with the
 # shortcut on), measured: rocprofv3 FETCH_SIZE x 1024 x 2 + WRITE_SIZE x 1024
 # (FETCH_SIZE reads half and WRITE_SIZE all of a plain copy kernel's bytes);
-# 766 MB read + 105 MB written against 759 MB algorithmic.
-NEWTON_TRAFFIC_128 = 8.710e8
+# 763 MB read + 105 MB written against 759 MB algorithmic.
+NEWTON_TRAFFIC_128 = 8.680e8
 PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFS = 78.6
 
