@@ -132,6 +132,13 @@ __device__ __forceinline__ double rcp_refined(double d)
     return y;
 }
 
+// 1/c for a CRSS: 0 where it is infinite (the system is off), as the reference's
+// division gives; the estimate's refinement alone is NaN there (inf 0).
+__device__ __forceinline__ double rcp_crss(double c)
+{
+    return __builtin_amdgcn_div_fixup(rcp_refined(c), c, 1.0);
+}
+
 constexpr int NB_THREADS = 64; // one wave per block: the LDS columns are wave-private
 
 // The kernel's NewtonParams (its first argument) in the kernel-argument
@@ -626,8 +633,8 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                     it[k * NB_THREADS] = c1[k];
                     it[(EVPGPU_NSYSMX + k) * NB_THREADS] = c2[k];
                 } else {
-                    it[k * NB_THREADS] = rcp_refined(c1[k]);
-                    if (!CSYM) it[(EVPGPU_NSYSMX + k) * NB_THREADS] = rcp_refined(c2[k]);
+                    it[k * NB_THREADS] = rcp_crss(c1[k]);
+                    if (!CSYM) it[(EVPGPU_NSYSMX + k) * NB_THREADS] = rcp_crss(c2[k]);
                 }
             }
         }
