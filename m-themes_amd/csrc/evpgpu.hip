@@ -154,7 +154,9 @@ double sym6_min_eig(double a[6][6], double *max = nullptr)
     return m;
 }
 
-// the squares of C0's extreme eigenvalues, with a margin for their rounding
+// the squares of C0's extreme eigenvalues, with a margin for their rounding;
+// 0 and infinity where C0 is not positive definite: they decide no comparison of
+// the Newton kernel's line search
 void update_c0_bounds(evpgpu_ctx *c)
 {
     double a[6][6], hi;
@@ -162,7 +164,7 @@ void update_c0_bounds(evpgpu_ctx *c)
         for (int j = i; j < 6; j++) a[i][j] = a[j][i] = c->ld.c066[i * 6 + j];
     const double lo = sym6_min_eig(a, &hi);
     c->c0_lo2 = lo > 0.0 ? 0.9999 * lo * lo : 0.0;
-    c->c0_hi2 = lo > 0.0 ? 1.0001 * hi * hi : 0.0;
+    c->c0_hi2 = lo > 0.0 ? 1.0001 * hi * hi : INFINITY;
 }
 
 // min over orientations of lambda_min(S0 + S), both from their upper

@@ -52,7 +52,7 @@ struct NewtonParams {
     double s0p[21];  // S0 = C0^-1 (B-basis), packed upper triangle: the Newton step is
                      // solved in S0-scaled form
     double kmin_tolx2; // (0.99 TOLX min over orientations of lambda_min(S0 + S))^2
-    double c0_lo2, c0_hi2; // squares of C0's extreme eigenvalues (0: unknown)
+    double c0_lo2, c0_hi2; // squares of C0's extreme eigenvalues (not known: 0 and infinity)
     double nr_tol;   // Newton tolerance on the relative step (reference 1e-10)
     double tolx;     // line-search TOLX (reference 1e-7)
     int dd;          // dislocation-density law: the crss argument holds the
@@ -138,7 +138,7 @@ struct evpgpu_ctx {
     double *sgr;      // n_orient x 36: LU_inv_66(C_gr)
     double *h_sgr;    // host copy
     double lam_min;   // min over orientations of lambda_min(S0 + S), < 0 when stale
-    double c0_lo2, c0_hi2; // squares of C0's extreme eigenvalues, with a margin (0: not known)
+    double c0_lo2, c0_hi2; // squares of C0's extreme eigenvalues, with a margin (not known: 0 and infinity)
     int n_orient;
 
     // spectral buffers
