@@ -20,8 +20,9 @@
 //     registers otherwise), between two 5x5 rotations of the voxel;
 //   * |x|^n by repeated squaring for integral n, 1/CRSS multiplied instead of
 //     divided, fused multiply-adds.
-// A non-positive-definite K returns status 35, the reference's singular-LU
-// exit.
+// A K that is not positive definite returns status 35, the reference's
+// singular-LU exit; one that only its rounded sums made so is factored
+// another way first (rank1_solve).
 //
 // What bounds it: FP64 vector issue, two waves per SIMD (256 registers each).
 // One voxel per lane; K0 = S0 + S, the rotation, the stress and the residual
@@ -444,6 +445,76 @@ __device__ __forceinline__ bool ldl6_solve(double k[21], double b[6])
     return pd;
 }
 
+// (K0 + sum_k w_k m_k m_k^T) x = b (b overwritten) by rank-one updates of K0's
+// L D L^T (Gill, Golub, Murray and Saunders 1974, method C1), the Schmid
+// vectors m_k in sample axes and the weights w those of tangent().  Every update
+// raises the pivots, so the factors are positive definite wherever K0 is.
+// The sums of tangent() round to 1e-16 of the largest weight.  The weights go as
+// |x|^(n-1), and where that leaves fewer than five independent systems within
+// 1e16 of the largest, the small pivots can round to below 0: with n of 45 and
+// more, in a first iteration next to a pore, some voxels of 1e5 (none up to
+// n = 40, at any overstress tried).  Taken there only: 12 updates of dependent
+// operations.  (Registers held for it: 1 % of an iteration at n = 33, 0.4 % at
+// n = 12.5 with unequal CRSS.)
+__device__ __forceinline__ bool rank1_solve(const NewtonParams &P, int p, int ns, const double *w,
+                                            const double Q[25], const double K0[21], double b[6])
+{
+    double k[21]; // D on the diagonal, L (unit) above it, transposed
+    bool pd = true;
+#pragma unroll
+    for (int i = 0; i < 21; i++) k[i] = K0[i];
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+        pd = pd && k[PK(j, j)] > 0.0;
+        const double inv = rcp_refined(k[PK(j, j)]);
+#pragma unroll
+        for (int i = j + 1; i < 6; i++) {
+            const double l = k[PK(j, i)] * inv;
+#pragma unroll
+            for (int q = i; q < 6; q++) k[PK(i, q)] = fma(-l, k[PK(j, q)], k[PK(i, q)]);
+        }
+#pragma unroll
+        for (int i = j + 1; i < 6; i++) k[PK(j, i)] *= inv;
+    }
+#pragma unroll 1
+    for (int s = 0; s < ns; s++) {
+        const double *m = P.mx[p][s];
+        double a = w[s * NB_THREADS], z[6];
+#pragma unroll
+        for (int i = 0; i < 5; i++) {
+            z[i] = Q[5 * i] * m[0];
+#pragma unroll
+            for (int j = 1; j < 5; j++) z[i] = fma(Q[5 * i + j], m[j], z[i]);
+        }
+        z[5] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 6; j++) {
+            const double d = k[PK(j, j)], pj = z[j], dn = fma(a * pj, pj, d), inv = rcp_refined(dn);
+            const double be = a * pj * inv;
+            a *= d * inv;
+            k[PK(j, j)] = dn;
+#pragma unroll
+            for (int r = j + 1; r < 6; r++) {
+                z[r] = fma(-pj, k[PK(j, r)], z[r]);
+                k[PK(j, r)] = fma(be, z[r], k[PK(j, r)]);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+        pd = pd && k[PK(j, j)] > 0.0; // (not where a weight is not a number)
+#pragma unroll
+        for (int i = j + 1; i < 6; i++) b[i] = fma(-k[PK(j, i)], b[j], b[i]);
+    }
+#pragma unroll
+    for (int i = 5; i >= 0; i--) {
+        b[i] *= rcp_refined(k[PK(i, i)]);
+#pragma unroll
+        for (int q = i + 1; q < 6; q++) b[i] = fma(-k[PK(i, q)], b[q], b[i]);
+    }
+    return pd;
+}
+
 // y = A x for a packed symmetric 6x6 A of NewtonParams, added to y
 __device__ __forceinline__ void sym6_mul_add(cdouble A, const double x[6], double y[6])
 {
@@ -677,7 +748,17 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                 tangent<CUBIC>(ns, p, w, Q, K0, K);
 #pragma unroll
                 for (int i = 0; i < 6; i++) step[i] = -r[i];
-                const bool pd = ldl6_solve(K, step);
+                bool pd = ldl6_solve(K, step);
+                // (steep rates are RM_LOOP's, or RM_POW's without CUBIC)
+                if (!CUBIC && (RM == RM_POW || RM == RM_LOOP) && __builtin_expect(__any(open && !pd), 0)) {
+                    double x[6];
+#pragma unroll
+                    for (int i = 0; i < 6; i++) x[i] = -r[i];
+                    const bool ok = rank1_solve(P, p, ns, w, Q, K0, x);
+#pragma unroll
+                    for (int i = 0; i < 6; i++) step[i] = pd ? step[i] : x[i];
+                    pd = pd || ok;
+                }
                 singular = singular || (open && !pd);
                 // the slope of the merit function along the step is
                 // -scale |R|^2: zero only where the residual is
@@ -913,7 +994,11 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
         // against 240 at 128^3) and the rate law is odd in the resolved shear
         // (a place may hold a system of the other sign): not for unequal
         // forward and backward CRSS.  RM_LOOP (n of 33 to 64) has no such
-        // variant: no use of it is known.
+        // variant: no use of it is known.  RM_POW's is for n up to 32: above it
+        // the general one, which has rank1_solve (128 us a 48^3 iteration
+        // against 120 at n = 12.5).
+        bool steep = false;
+        for (int k = 0; k < P.nsys[p]; k++) steep = steep || P.nrs[p][k] > 32.0;
         const int ne = rm == RM_FAST && P.crss_sym && (P.int_n[p] == 10 || P.int_n[p] == 20) ? P.int_n[p] : 0;
         // the events (when given) take the kernel's own start and end times: no
         // marker packets between the launches
@@ -936,7 +1021,7 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
         else if (rm == RM_FAST) LAUNCH(RM_FAST, false, F, 0, false);                     \
         else if (rm == RM_LOOP && P.crss_sym) LAUNCH(RM_LOOP, true, F, 0, false);        \
         else if (rm == RM_LOOP) LAUNCH(RM_LOOP, false, F, 0, false);                     \
-        else if (rm == RM_POW && P.crss_sym && P.cubic[p]) LAUNCH(RM_POW, true, F, 0, true); \
+        else if (rm == RM_POW && P.crss_sym && P.cubic[p] && !steep) LAUNCH(RM_POW, true, F, 0, true); \
         else if (P.crss_sym) LAUNCH(RM_POW, true, F, 0, false);                          \
         else LAUNCH(RM_POW, false, F, 0, false);                                         \
     } while (0)

@@ -2,8 +2,9 @@
 switched off by an infinite CRSS (a file or a caller's state may hold one; the
 rate is then 0, the reference's division by infinity), in some voxels of a wave
 and in one direction only, or in a whole phase, which is then elastic, against
-the oracle at the bars of the whole-loop parity tests; and a C0 that is not
-positive definite, as a caller may set one."""
+the oracle at the bars of the whole-loop parity tests; a C0 that is not
+positive definite, as a caller may set one; and rate laws so steep that the
+tangent's terms span more than the 16 digits of its sums."""
 import numpy as np
 import pytest
 
@@ -106,3 +107,33 @@ def test_descent_test_without_bounds_on_c0(job_factory, shortcut):
     assert out[0][:2] == out[1][:2]
     for k in out[0][2]:
         assert np.array_equal(out[0][2][k], out[1][2][k]), k
+
+
+@pytest.mark.parametrize("nrs", [50.0, 50.5])
+def test_steep_rates_next_to_pores(job_factory, nrs):
+    """The first iteration's overstress next to pores at a steep rate law: its
+    tangent's weights span more than 1e16, and rounded sums of them need not be
+    positive definite.  The same stresses as the batch update's, from the same
+    inputs, to where both end (steps below 1e-7 of the stress: a bar of 1e-6);
+    then more iterations of the loop."""
+    inp = job_factory(f"steep{nrs}", n=16, grains=8, seed=25, increments=1, pore_fraction=0.04, pore_radius=2,
+                      material=synth.Material(nrs=nrs))
+    J, g = O.Job(inp), lib.GpuJob(inp)
+    solid = np.where(J.phase() == 1)[0]
+    m = solid.size
+    a = {k: np.ascontiguousarray(v[:, solid]) for k, v in _download(g).items()}
+    g.run(1, forced=1)
+    b = {k: v[:, solid] for k, v in _download(g).items()}
+    d = b["disgrad"]
+    E = np.stack([d[0], d[4], d[8], (d[5] + d[7]) / 2, (d[2] + d[6]) / 2, (d[1] + d[3]) / 2])
+    ctx = lib.Context.__new__(lib.Context)
+    ctx.h = g.ctx
+    st, sig, *_ = ctx.newton(np.ones(m, np.int32), np.arange(m, dtype=np.int32), np.linalg.inv(J.cgr()[solid]), a["sig"], E,
+                             a["eps"], a["tran"], a["crss"])
+    ctx.h = None
+    assert st == 0
+    assert np.abs(b["sig"] - sig).max() < 1e-6 * np.abs(sig).max()
+    g.reset()
+    g.run(1, forced=30)
+    assert np.isfinite(g.state()["Sig"]).all()
+    g.close()
