@@ -1,6 +1,6 @@
 """Grids whose lengths are not powers of two (the reference's FFTW takes any
-length): the direct-DFT transform kernels against numpy, and the whole loop
-against the oracle."""
+length): the mixed-radix and two-level DFT transform kernels against numpy, and
+the whole loop against the oracle."""
 import numpy as np
 import pytest
 
@@ -9,9 +9,9 @@ from pyevp import lib
 
 pytestmark = pytest.mark.gpu
 
-# lengths of the form 2^m 3^a 5^b divisible by 4 (12, 20, 24, 36, 60, 96, 100,
-# 240, ...) take the mixed-radix Stockham kernels, the others (5, 6, 7, 9, 10,
-# 15, 3) the two-level DFT ones
+# the lengths with a Stockham plan (10, 12, 15, 20, 24, 36, 60, 96, 100, 240,
+# ...; along z the even ones) take the mixed-radix kernels, the others (3, 5, 6,
+# 7, 9, and 15 along z) the two-level DFT ones
 SIZES = [(12, 10, 9), (5, 6, 7), (24, 20, 15), (3, 8, 100), (16, 16, 12), (9, 32, 16),
          (96, 40, 36), (60, 100, 12), (240, 20, 24), (72, 144, 48)]
 
@@ -45,10 +45,11 @@ def test_any_length_fp32_vs_numpy(dims):
     ctx.close()
 
 
-@pytest.mark.parametrize("dims", [(12, 10, 9), (10, 12, 12), (24, 20, 12)])
+@pytest.mark.parametrize("dims", [(12, 10, 9), (10, 12, 12), (24, 20, 12), (11, 10, 9)])
 def test_loop_parity_any_size(job_factory, dims):
     """The whole loop on odd and even non-power-of-two grids, pores included,
-    against the oracle (natural convergence, identical iteration counts)."""
+    against the oracle (natural convergence, identical iteration counts): five
+    passes, and seven where nx has no x-line kernel (11)."""
     inp = job_factory(f"anysize{dims}", n=0, dims=dims, grains=6, seed=47, increments=3,
                       pore_fraction=0.02, pore_radius=1)
     J = O.Job(inp)
