@@ -419,78 +419,26 @@ __global__ __launch_bounds__(NT) void k_dft_z_c2r(const typename CT<R>::T *in, d
     });
 }
 
-// Lengths with a Stockham plan: the 2^m 3^a 5^b of FFT_DISPATCH; the others
-// take the two-level DFT kernels.  Real lines (z) go through a transform of
-// half the length, so theirs are the even ones.  (45 x 50 x 27 in FP32: the y
-// passes 8.6 -> 4.3 us each, and x with the Green step 22 -> 9 us, against the
-// DFT kernels these lengths took before.)
-bool is_stockham_len(int L, bool real = false)
-{
-    static const int even[] = {
-        8, 10, 12, 16, 18, 20, 24, 30, 32, 36, 40, 48, 50, 54, 60, 64, 72, 80, 90, 96, 100, 108,
-        120, 128, 144, 150, 160, 180, 192, 200, 216, 240, 250, 256};
-    static const int odd[] = {15, 25, 27, 45, 75, 125, 225};
-    for (int l : even)
-        if (l == L) return true;
-    for (int l : odd)
-        if (l == L) return !real;
-    return false;
-}
+// Lengths without a Stockham plan take the two-level DFT kernels.  (45 x 50 x 27
+// in FP32: the y passes 8.6 -> 4.3 us each, and x with the Green step 22 -> 9 us,
+// against the DFT kernels.)
 
 template <typename R> const typename CT<R>::T *twp(evpgpu_ctx *c, int axis);
 template <> const double2 *twp<double>(evpgpu_ctx *c, int axis) { return c->tw64[axis]; }
 template <> const float2 *twp<float>(evpgpu_ctx *c, int axis) { return c->tw32[axis]; }
 
 // dispatch on a runtime length
-#define FFT_DISPATCH_EVEN(L_, CALL, ODD_) \
-    switch (L_) {              \
-    case 8: CALL(8); break; \
-    case 10: CALL(10); break; \
-    case 12: CALL(12); break; \
-    case 16: CALL(16); break; \
-    case 18: CALL(18); break; \
-    case 20: CALL(20); break; \
-    case 24: CALL(24); break; \
-    case 30: CALL(30); break; \
-    case 32: CALL(32); break; \
-    case 36: CALL(36); break; \
-    case 40: CALL(40); break; \
-    case 48: CALL(48); break; \
-    case 50: CALL(50); break; \
-    case 54: CALL(54); break; \
-    case 60: CALL(60); break; \
-    case 64: CALL(64); break; \
-    case 72: CALL(72); break; \
-    case 80: CALL(80); break; \
-    case 90: CALL(90); break; \
-    case 96: CALL(96); break; \
-    case 100: CALL(100); break; \
-    case 108: CALL(108); break; \
-    case 120: CALL(120); break; \
-    case 128: CALL(128); break; \
-    case 144: CALL(144); break; \
-    case 150: CALL(150); break; \
-    case 160: CALL(160); break; \
-    case 180: CALL(180); break; \
-    case 192: CALL(192); break; \
-    case 200: CALL(200); break; \
-    case 216: CALL(216); break; \
-    case 240: CALL(240); break; \
-    case 250: CALL(250); break; \
-    case 256: CALL(256); break; \
-    ODD_                       \
-    default: return EVPGPU_ERR_SIZE; \
+#define FFT_DISPATCH(L_, CALL)                 \
+    switch (L_) {                              \
+        STOCKHAM_EVEN(STOCKHAM_CASE, CALL)     \
+        STOCKHAM_ODD(STOCKHAM_CASE, CALL)      \
+    default: return EVPGPU_ERR_SIZE;           \
     }
-#define FFT_ODD(CALL) \
-    case 15: CALL(15); break; \
-    case 25: CALL(25); break; \
-    case 27: CALL(27); break; \
-    case 45: CALL(45); break; \
-    case 75: CALL(75); break; \
-    case 125: CALL(125); break; \
-    case 225: CALL(225); break;
-#define FFT_DISPATCH(L_, CALL) FFT_DISPATCH_EVEN(L_, CALL, FFT_ODD(CALL))
-#define FFT_DISPATCH_REAL(L_, CALL) FFT_DISPATCH_EVEN(L_, CALL, )
+#define FFT_DISPATCH_REAL(L_, CALL)            \
+    switch (L_) {                              \
+        STOCKHAM_EVEN(STOCKHAM_CASE, CALL)     \
+    default: return EVPGPU_ERR_SIZE;           \
+    }
 
 template <typename R, bool INV>
 int pass_y(evpgpu_ctx *c, typename CT<R>::T *d, int ncomp)

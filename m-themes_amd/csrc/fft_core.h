@@ -6,7 +6,29 @@
 
 #include <hip/hip_runtime.h>
 
+// The lengths with a Stockham plan, X(length, A) each: products of 2, 3 and 5 in
+// [8, 256] (all but 9, 81, 135, 162 and 243).  Real lines (z) go through a
+// transform of half the length, so theirs are the even ones; x and y lines take
+// both lists.
+#define STOCKHAM_EVEN(X, A)                                                              \
+    X(8, A) X(10, A) X(12, A) X(16, A) X(18, A) X(20, A) X(24, A) X(30, A) X(32, A)      \
+    X(36, A) X(40, A) X(48, A) X(50, A) X(54, A) X(60, A) X(64, A) X(72, A) X(80, A)     \
+    X(90, A) X(96, A) X(100, A) X(108, A) X(120, A) X(128, A) X(144, A) X(150, A)        \
+    X(160, A) X(180, A) X(192, A) X(200, A) X(216, A) X(240, A) X(250, A) X(256, A)
+#define STOCKHAM_ODD(X, A) X(15, A) X(25, A) X(27, A) X(45, A) X(75, A) X(125, A) X(225, A)
+#define STOCKHAM_CASE(L, CALL) case L: CALL(L); break;
+#define STOCKHAM_TRUE(L, A) case L: return A;
+
 namespace fftc {
+
+inline bool is_stockham_len(int len, bool real = false)
+{
+    switch (len) {
+        STOCKHAM_EVEN(STOCKHAM_TRUE, true)
+        STOCKHAM_ODD(STOCKHAM_TRUE, !real)
+    default: return false;
+    }
+}
 
 template <typename R> struct CT;
 template <> struct CT<double> { typedef double2 T; };

@@ -216,8 +216,9 @@ __global__ __launch_bounds__(NTX) void k_x_green(typename CT<R>::T *__restrict__
     for (int i = threadIdx.x; i < NX; i += NTX) s_tw[i] = twx[i];
     if (threadIdx.x < 36) c0s[threadIdx.x] = (R)G.ga[threadIdx.x];
     // The x lines are the columns q = y*nzh + kz of the [x][y][kz] half
-    // spectrum; a workgroup takes TBX consecutive columns q0.. (runs that
-    // start on 128-byte boundaries, as ny*nzh is a multiple of TBX).
+    // spectrum; a workgroup takes TBX consecutive columns q0.. (on
+    // 128-byte boundaries where ny*nzh is a multiple of 8 in FP64, of 16 in FP32;
+    // anywhere, and the last tile ragged, on other grids).
     // Line (c, j) = component c, column q0 + j; element x at spec[c*NK + x*ncol + q0 + j].
     const int ncol = ny * nzh;
     // Workgroups go to the 8 XCDs round robin (block b to XCD b mod 8), and
@@ -360,51 +361,11 @@ constexpr int TILE_FILL = 512;
     default: return EVPGPU_ERR_SIZE;                           \
     }
 
-// x-line lengths: the Stockham lengths of fft.hip
-#define LINE_DISPATCH(CALL)             \
-    switch (c->nx) {                    \
-    case 8: CALL(8); break; \
-    case 10: CALL(10); break; \
-    case 12: CALL(12); break; \
-    case 15: CALL(15); break; \
-    case 16: CALL(16); break; \
-    case 18: CALL(18); break; \
-    case 20: CALL(20); break; \
-    case 24: CALL(24); break; \
-    case 25: CALL(25); break; \
-    case 27: CALL(27); break; \
-    case 30: CALL(30); break; \
-    case 32: CALL(32); break; \
-    case 36: CALL(36); break; \
-    case 40: CALL(40); break; \
-    case 45: CALL(45); break; \
-    case 48: CALL(48); break; \
-    case 50: CALL(50); break; \
-    case 54: CALL(54); break; \
-    case 60: CALL(60); break; \
-    case 64: CALL(64); break; \
-    case 72: CALL(72); break; \
-    case 75: CALL(75); break; \
-    case 80: CALL(80); break; \
-    case 90: CALL(90); break; \
-    case 96: CALL(96); break; \
-    case 100: CALL(100); break; \
-    case 108: CALL(108); break; \
-    case 120: CALL(120); break; \
-    case 125: CALL(125); break; \
-    case 128: CALL(128); break; \
-    case 144: CALL(144); break; \
-    case 150: CALL(150); break; \
-    case 160: CALL(160); break; \
-    case 180: CALL(180); break; \
-    case 192: CALL(192); break; \
-    case 200: CALL(200); break; \
-    case 216: CALL(216); break; \
-    case 225: CALL(225); break; \
-    case 240: CALL(240); break; \
-    case 250: CALL(250); break; \
-    case 256: CALL(256); break; \
-    default: return EVPGPU_ERR_SIZE;    \
+#define LINE_DISPATCH(CALL)                    \
+    switch (c->nx) {                           \
+        STOCKHAM_EVEN(STOCKHAM_CASE, CALL)     \
+        STOCKHAM_ODD(STOCKHAM_CASE, CALL)      \
+    default: return EVPGPU_ERR_SIZE;           \
     }
 
 template <typename R, int IN>
@@ -458,16 +419,8 @@ int xg(evpgpu_ctx *c)
 
 } // namespace
 
-// the lengths nx of LINE_DISPATCH
-bool lines_ok(const evpgpu_ctx *c)
-{
-    static const int lines[] = {
-        8, 10, 12, 15, 16, 18, 20, 24, 25, 27, 30, 32, 36, 40, 45, 48, 50, 54, 60, 64, 72, 75, 80,
-        90, 96, 100, 108, 120, 125, 128, 144, 150, 160, 180, 192, 200, 216, 225, 240, 250, 256};
-    for (int n : lines)
-        if (c->nx == n) return true;
-    return false;
-}
+// the x-line kernel has every Stockham length
+bool lines_ok(const evpgpu_ctx *c) { return fftc::is_stockham_len(c->nx); }
 
 // the fused path covers the plane lengths ny = nz of PLANE_DISPATCH (<= 128:
 // the plane fits in LDS in FP64) and the line lengths
