@@ -277,9 +277,16 @@ int newton_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, do
                   double *gamdot, const int *phase, const int *orient, const double *sgr,
                   long long n, double *partials, int *nblk_out, int *status, int fast,
                   hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
-// rate-law evaluation: 0 non-integral exponent, 1 integral, 2 integral n <= 32
-// with 12 systems of one n and one gam0 in every crystal phase
-int newton_rate_mode(const NewtonParams &P);
+// Rate-law evaluation: RM_POW pow() for a non-integral exponent, RM_LOOP
+// repeated squaring for an integral one, RM_FAST the common case of every
+// crystal phase having EVPGPU_NSYSMX systems with one integral n <= 32 and
+// one reference rate (constants hoisted out of the system loop, straight-line
+// squaring; in newton.hip the exponents 10 and 20 are template constants).
+// RM_DISL (newton.hip alone): the dislocation-density law StrainRate_Orowan
+// (src/constitutive.c:507-721), with its per-voxel constants formed once
+// per increment.
+enum { RM_POW = 0, RM_LOOP = 1, RM_FAST = 2, RM_DISL = 3 };
+int newton_rate_mode(const NewtonParams &P); // of the power law
 // newton_batch.hip: the power-law update of a caller's batch, with each
 // voxel's error norms and Newton count
 int newton_batch_launch(evpgpu_ctx *c, const NewtonParams &P, const double *sig_in, double *sig, const double *E,

@@ -41,37 +41,10 @@
 // twice, and one evaluation in three less).
 #include <hip/hip_ext.h>
 
-#include "evpgpu_impl.h"
 #include "linesearch.h"
+#include "newton_common.h"
 
 namespace {
-
-__device__ __forceinline__ double ipow(double x, int m)
-{
-    double r = 1.0, b = x;
-    while (m) {
-        if (m & 1) r *= b;
-        b *= b;
-        m >>= 1;
-    }
-    return r;
-}
-
-// x^m for a wave-uniform 0 <= m < 32: the products of ipow in the same
-// order, straight-line (a scalar-masked select per exponent bit instead of a
-// scalar loop: with one wave per SIMD every scalar instruction and branch
-// costs an issue slot)
-__device__ __forceinline__ double ipow5(double x, int m)
-{
-    double r = 1.0, b = x;
-#pragma unroll
-    for (int i = 0; i < 5; i++) {
-        const double t = r * b;
-        r = ((m >> i) & 1) ? t : r;
-        if (i < 4) b *= b;
-    }
-    return r;
-}
 
 // x^M for a compile-time M: the products of ipow with the bit tests folded
 // (x^9 is three squarings and one product)
@@ -84,40 +57,6 @@ template <int M> __device__ __forceinline__ double ipowc(double x)
         if (m > 1) b *= b;
     }
     return r;
-}
-
-// Rate-law evaluation: RM_POW pow() for a non-integral exponent, RM_LOOP
-// repeated squaring for an integral one, RM_FAST the common case of every
-// crystal phase having EVPGPU_NSYSMX systems with one integral n <= 32 and
-// one reference rate (constants hoisted out of the system loop, straight-
-// line squaring; for n = 10 and n = 20 the exponent is a template constant).
-// RM_DISL: the dislocation-density law StrainRate_Orowan
-// (src/constitutive.c:507-721), with its per-voxel constants formed once
-// per increment.
-enum { RM_POW = 0, RM_LOOP = 1, RM_FAST = 2, RM_DISL = 3 };
-
-// chg_basis opt 2 for a symmetric tensor given as (11 22 33 23 13 12)
-__device__ __forceinline__ void sym_to_v6(const double t[6], double v[6])
-{
-    const double r2 = RSQ2, r3 = RSQ3, r6 = RSQ6;
-    v[0] = t[0] * (-1. * r2) + t[1] * r2;
-    v[1] = t[0] * (-1. * r6) + t[1] * (-1. * r6) + t[2] * (2. * r6);
-    v[2] = t[3] * r2 + t[3] * r2;
-    v[3] = t[4] * r2 + t[4] * r2;
-    v[4] = t[5] * r2 + t[5] * r2;
-    v[5] = t[0] * r3 + t[1] * r3 + t[2] * r3;
-}
-
-// chg_basis opt 1 -> symmetric (11 22 33 23 13 12)
-__device__ __forceinline__ void v6_to_sym(const double v[6], double t[6])
-{
-    const double r2 = RSQ2, r3 = RSQ3, r6 = RSQ6;
-    t[0] = v[0] * (-1. * r2) + v[1] * (-1. * r6) + v[5] * r3;
-    t[1] = v[0] * r2 + v[1] * (-1. * r6) + v[5] * r3;
-    t[2] = v[1] * (2. * r6) + v[5] * r3;
-    t[3] = v[2] * r2;
-    t[4] = v[3] * r2;
-    t[5] = v[4] * r2;
 }
 
 // 1/d for a normal d: the hardware estimate refined by two Newton steps

@@ -36,67 +36,10 @@
 // loop's kernel does, was measured at 795 us where this form takes 1000 us
 // (1000003 voxels, n = 20) and left out: the compiled tangent rounds
 // differently, and one voxel in a million then reports another count.
-#include "evpgpu_impl.h"
 #include "linesearch.h"
+#include "newton_common.h"
 
 namespace {
-
-__device__ __forceinline__ double ipow(double x, int m)
-{
-    double r = 1.0, b = x;
-    while (m) {
-        if (m & 1) r *= b;
-        b *= b;
-        m >>= 1;
-    }
-    return r;
-}
-
-// x^m for a wave-uniform 0 <= m < 32: the products of ipow in the same
-// order, straight-line (a scalar-masked select per exponent bit instead of a
-// scalar loop: with one wave per SIMD every scalar instruction and branch
-// costs an issue slot)
-__device__ __forceinline__ double ipow5(double x, int m)
-{
-    double r = 1.0, b = x;
-#pragma unroll
-    for (int i = 0; i < 5; i++) {
-        const double t = r * b;
-        r = ((m >> i) & 1) ? t : r;
-        if (i < 4) b *= b;
-    }
-    return r;
-}
-
-// Rate-law evaluation: RM_POW pow() for a non-integral exponent, RM_LOOP
-// repeated squaring for an integral one, RM_FAST the common case of every
-// crystal phase having EVPGPU_NSYSMX systems with one integral n <= 32 and
-// one reference rate.
-enum { RM_POW = 0, RM_LOOP = 1, RM_FAST = 2 };
-
-// chg_basis opt 2 for a symmetric tensor given as (11 22 33 23 13 12)
-__device__ __forceinline__ void sym_to_v6(const double t[6], double v[6])
-{
-    const double r2 = RSQ2, r3 = RSQ3, r6 = RSQ6;
-    v[0] = t[0] * (-1. * r2) + t[1] * r2;
-    v[1] = t[0] * (-1. * r6) + t[1] * (-1. * r6) + t[2] * (2. * r6);
-    v[2] = t[3] * r2 + t[3] * r2;
-    v[3] = t[4] * r2 + t[4] * r2;
-    v[4] = t[5] * r2 + t[5] * r2;
-    v[5] = t[0] * r3 + t[1] * r3 + t[2] * r3;
-}
-
-// chg_basis opt 1 -> symmetric (11 22 33 23 13 12)
-__device__ __forceinline__ void v6_to_sym(const double v[6], double t[6])
-{
-    const double r2 = RSQ2, r3 = RSQ3, r6 = RSQ6;
-    t[0] = v[0] * (-1. * r2) + v[1] * (-1. * r6) + v[5] * r3;
-    t[1] = v[0] * r2 + v[1] * (-1. * r6) + v[5] * r3;
-    t[2] = v[1] * (2. * r6) + v[5] * r3;
-    t[3] = v[2] * r2;
-    t[4] = v[3] * r2;
-    t[5] = v[4] * r2;
-}
 
 constexpr int NB_THREADS = 64; // one wave per block: the LDS slab is wave-private
 
@@ -282,9 +225,8 @@ __device__ __forceinline__ double nr_quality(const NewtonParams &P, int p, const
 template <int RM>
 __device__ int update_voxel(const NewtonParams &P, int p, RateIn &in, const Vox &V,
                             double sig6[6], double edotp[6], double gd[EVPGPU_NSYSMX],
-                            double &conv_s, double &conv_e, int &iterl, int &trials)
+                            double &conv_s, double &conv_e, int &iterl)
 {
-    trials = 0;
     double ed[5], res[6], old[6], k[21];
     double ce = 0.0;
     iterl = 0;
@@ -374,7 +316,6 @@ __device__ int update_voxel(const NewtonParams &P, int p, RateIn &in, const Vox 
 #pragma unroll
             for (int i = 0; i < 6; i++) sig6[i] = old[i] + alam * step[i];
             double f_new = nr_quality<RM>(P, p, in, V, sig6, gd);
-            trials++;
             if (alam < alamin) {
 #pragma unroll
                 for (int i = 0; i < 6; i++) sig6[i] = old[i];
@@ -547,8 +488,8 @@ __global__ __launch_bounds__(NB_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1
                 }
             }
             double s6[6], e6[6], gd[EVPGPU_NSYSMX], cs, ce;
-            int it, ntr;
-            int st = update_voxel<RM>(P, p, in, V, s6, e6, gd, cs, ce, it, ntr);
+            int it;
+            int st = update_voxel<RM>(P, p, in, V, s6, e6, gd, cs, ce, it);
             if (st) {
                 atomicCAS(status, 0, st);
             } else {
