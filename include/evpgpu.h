@@ -131,8 +131,9 @@ typedef struct {
 const char *evpgpu_strerror(int status);
 
 /* Create a context for an nx*ny*nz grid, each length in [2, 512].  Products of
- * 2, 3 and 5 in [8, 256] take the Stockham transforms; other lengths a
- * two-level DFT along that axis (correct for any length). */
+ * 2, 3 and 5 in [8, 256], but for 9, 81, 135, 162 and 243, take the Stockham
+ * transforms (along z the even ones); other lengths a two-level DFT along that
+ * axis (correct for any length). */
 int evpgpu_create(evpgpu_ctx **ctx, int nx, int ny, int nz, int precision);
 int evpgpu_destroy(evpgpu_ctx *ctx);
 int evpgpu_set_precision(evpgpu_ctx *ctx, int precision);
@@ -248,10 +249,10 @@ int evpgpu_newton_host(evpgpu_ctx *ctx, int n, const int *phase, const int *orie
 
 /* The per-voxel stress update of evpgpu_newton_host on caller-owned DEVICE
  * buffers (same layouts, n voxels), allocating nothing: no counterpart in
- * the reference; for callers that cannot allocate device memory (code under
- * HIP graph capture, tight serving loops).  Its scratch is two words of the
- * context, so calls on different contexts do not meet; n is at most 2^21
- * (EVPGPU_ERR_SIZE above).  Phase and orientation indices are checked on the
+ * the reference; for callers that must not allocate device memory (tight
+ * serving loops; it waits for its stream, so it cannot be under HIP graph
+ * capture).  Its scratch is two words of the context, so calls on different
+ * contexts do not meet; n is at most 2^21 (EVPGPU_ERR_SIZE above).  Phase and orientation indices are checked on the
  * device first: where one is out of range the update does nothing and the
  * call returns EVPGPU_ERR_ARG.  Runs on the context's stream and waits for it. */
 #define EVPGPU_NOALLOC_MAX_VOXELS (1 << 21)

@@ -103,8 +103,8 @@ double now_s()
     return ts.tv_sec + 1e-9 * ts.tv_nsec;
 }
 
-// grid lengths: any length in [2, 512]; products of 2, 3 and 5 in [8, 256]
-// take the Stockham kernels, the others the two-level DFT ones (fft.hip)
+// grid lengths: any length in [2, 512]; those of fft_core.h's lists take the
+// Stockham kernels, the others the two-level DFT ones (fft.hip)
 bool len_ok(int n) { return n >= 2 && n <= 512; }
 
 template <typename T> int dalloc(T **p, size_t n)
@@ -354,9 +354,10 @@ bool phase_ends(const LoopCtl &L, int limit, int conv)
 
 // One phase of the Green loop: iterations of one precision while
 // iter < limit (and, with conv, while the error norms exceed Err); first
-// runs at least one.  With loop_batch > 0 the iterations are queued in batches of loop_batch, two batches in flight: the
-// host reads the older batch's flags while the device runs the newer one,
-// and the iterations queued past the end of the phase return at once.
+// runs at least one.  With loop_batch > 0 the iterations are queued in batches
+// of loop_batch, two batches in flight: the host reads the older batch's flags
+// while the device runs the newer one, and the iterations queued past the end
+// of the phase return at once.
 // Otherwise the host waits for every iteration.  On return the host copy of
 // the control block (h_ctl[0]) is current and c->sig is the last stress.
 int run_phase(evpgpu_ctx *c, int prec, int limit, int conv, int first, const CtlConst &K, int *imix)
@@ -695,8 +696,8 @@ int evpgpu_upload_microstructure(evpgpu_ctx *c, const int *grain, const int *pha
         if (orient[v] >= n_orient || (orient[v] < 0 && phase[v] >= 1 && phase[v] <= c->nphases &&
                                       !c->ph[phase[v] - 1].is_gas))
             return EVPGPU_ERR_ARG;
-    // gas voxels carry orientation -1; the kernel never reads their table row,
-    // but keep the index valid
+    // gas voxels carry orientation -1: the Newton kernel's lanes of gas voxels
+    // read row 0 with the others of their wave and drop what they get
     int *o2 = (int *)malloc(sizeof(int) * c->N);
     for (long long v = 0; v < c->N; v++) o2[v] = orient[v] < 0 ? 0 : orient[v];
     if (c->sgr) (void)hipFree(c->sgr);

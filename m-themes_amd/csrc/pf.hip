@@ -855,7 +855,7 @@ constexpr int LAPQ[18][3] = {{1, 0, 0},   {-1, 0, 0},  {0, 1, 0},   {0, -1, 0}, 
 // (UPD_RES at most) until their voxels put them into the new lists in order.
 // Bound by the latency of its loads: 640 us per launch at 128^3 before (with the
 // last-writer searches, now in k_rho, once per substep), 337 now.
-constexpr int UPD_RES = 768, UPD_G = 4; // (three workgroups of 53 KB per CU)
+constexpr int UPD_RES = 768, UPD_G = 4; // (45 KB of LDS: three workgroups per CU)
 static_assert(UPD_RES >= CAP, "a voxel's candidates fit one run");
 
 __global__ __launch_bounds__(NT) void k_update(Dims g, Lists A, Lists B, Coef P, const int *gcnt, const int *gidx, const int *nn,

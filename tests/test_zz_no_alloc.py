@@ -2,8 +2,8 @@
 device buffers, no device allocation) against evpgpu_newton_host (the same
 update on host buffers, which allocates its device copies) through the C
 ABI: bit-for-bit equal stress, strain rate, slip rates, error norms and
-Newton counts, on two calls in a row (the second on a smaller batch, with
-the scratch array still holding the first call's partial sums); the size
+Newton counts, on two calls in a row on one context (the second on a smaller
+batch, with the context's status words still holding the first call's); the size
 limit and an out-of-range orientation index are refused with their status
 codes.  The test's device buffers come from hipMalloc of the HIP runtime the
 library itself loads (through ctypes).""" 
@@ -131,9 +131,10 @@ def test_noalloc_newton_refuses_bad_input(tmp_path):
     b2 = dict(b)
     b2["orient"] = b["orient"].copy()
     b2["orient"][5] = k  # one past the table of k orientations
-    st = _run_noalloc(f, gj.ctx, b2, k, hip)[0]
-    assert st == -1, st  # EVPGPU_ERR_ARG, before the update kernel runs
-    # larger than the scratch array holds: refused before any device work
+    st, sig, *outs = _run_noalloc(f, gj.ctx, b2, k, hip)
+    assert st == -1, st  # EVPGPU_ERR_ARG, and the update kernel does nothing
+    assert np.array_equal(sig, _cols(b["sig"], k)) and not any(o.any() for o in outs)
+    # larger than a call takes: refused before any device work
     x = hip.put(np.zeros(64))
     i = hip.put(np.zeros(64, np.int32))
     st = f(gj.ctx, (1 << 21) + 1, i, i, x, 1, *([x] * 9))
