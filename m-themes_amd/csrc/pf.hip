@@ -1275,7 +1275,6 @@ int substep(evpgpu_pf *p, const Coef &P)
     EVP_CHECK(hipStreamSynchronize(s));
     const long long tot = p->h_total[0] + WriterScan()(p->h_last[0]);
     const long long nw = tot & (SCAN_LOW - 1);
-    p->st.updated += tot >> 32;
     if ((st = ensure_writers(p, nw))) return st;
     hipLaunchKernelGGL(k_emit, dim3(gv), dim3(NT), 0, s, g, p->A, p->nn, p->spos, p->sg, p->wn, p->woff,
                        p->keys[0], p->refs[0], p->n_rho, p->flags);
@@ -1339,6 +1338,7 @@ int substep(evpgpu_pf *p, const Coef &P)
     hipLaunchKernelGGL(k_mesh, dim3(gc), dim3(NT), 0, s, g, p->defeng, p->gid);
     if ((st = read_flags(p))) return st;
     if (p->h_flags[0]) return pf_err(p->h_flags[0]);
+    p->st.updated += tot >> 32; // (a substep that fails adds none)
     return hipGetLastError() == hipSuccess ? EVPGPU_OK : EVPGPU_ERR_HIP;
 }
 

@@ -112,6 +112,7 @@ def test_pf_errors():
         with pytest.raises(lib.EvpError) as e:
             pf.pf_xrx(g2, rho, 2, pf_cases.params(1), np.zeros(4))
         assert e.value.code == gpf.ERR_PF_GRAIN
+        assert pf.stats()["updated"] == 0  # a substep that fails counts none
         # the context is usable again
         gn, _ = pf.pf_xrx(gid, rho, 2, pf_cases.params(1), np.zeros(4))
         assert (gn >= 1).all()
